@@ -6,7 +6,7 @@
 //
 // The recursion is ATLAS's: split the columns, factor the left part, TRSM +
 // GEMM the right part, factor it.  It stops at panels of at most PW columns
-// ("leaves").  Two things differ from a line-by-line reading of getrfC:
+// ("leaves").  Three things differ from a line-by-line reading of getrfC:
 //
 //  * Row interchanges are applied by each leaf, at once, to every column of
 //    the matrix outside the leaf, instead of by the laswp calls of every
@@ -16,7 +16,10 @@
 //    composes its swaps into one "row i receives row j" list, so a leaf's
 //    interchanges cost one gather/scatter pass over the other columns.
 //
-//  * A leaf panel is factored by one cooperative launch (panel_coop): the
+//  * A leaf panel of at most 8192 rows is factored by workgroups of one XCD
+//    (panel_xcd, lu_panel.hpp).
+//
+//  * A taller one is factored by one cooperative launch (panel_coop): the
 //    panel rows live in the registers of G <= 64 workgroups; per column each
 //    workgroup finds its candidate pivot (wavefront argmax over cross-lane
 //    shuffles, then LDS) and publishes it with the candidate row into the
@@ -95,6 +98,15 @@ constexpr long kSpinLimit = 1L << 20;  // default mailbox polls (each one round 
 #ifndef ATLG_LA_PANEL_CUS
 #define ATLG_LA_PANEL_CUS 64
 #endif
+// Tallest matrix whose panels get twice the units (16 of each XCD), so that
+// every panel runs on one XCD (panel_xcd): the panel is the longer path there
+// (N = 8192 with 16 right-hand sides: 74 -> 51 ms, panels included).
+#ifndef ATLG_LA_WIDE_ROWS
+#define ATLG_LA_WIDE_ROWS 8192
+#endif
+inline int la_panel_cus(long M) {
+  return M <= ATLG_LA_WIDE_ROWS ? 2 * ATLG_LA_PANEL_CUS : ATLG_LA_PANEL_CUS;
+}
 // Without reserved units: grid cap of the look-ahead trailing update
 // (workgroups; 0 = no cap), applied while the update is smaller than
 // ATLG_LA_CAP_AREA elements: then the panel beside it is the longer path and
@@ -143,12 +155,18 @@ constexpr long kLaMin = 2048;
 #ifndef ATLG_LA_PANEL_US
 #define ATLG_LA_PANEL_US 7.0
 #endif
+#ifndef ATLG_LA_PANEL_XCD_US
+#define ATLG_LA_PANEL_XCD_US 4.0
+#endif
 template <class S>
-long la_chunk(long rest, long rows, long kb, long nb1, long nb2) {
+long la_chunk(long rest, long rows, long kb, long nb1, long nb2, int panel_cus) {
   if (!ATLG_LA_BALANCE || !std::is_same<S, double>::value || rows <= 0 || nb1 <= 0) return 0;
-  const double panel_s = ATLG_LA_PANEL_US * 1e-6 * (double)nb1;
+  const double panel_s = (rows <= ATLG_LA_WIDE_ROWS ? ATLG_LA_PANEL_XCD_US : ATLG_LA_PANEL_US) *
+                         1e-6 * (double)nb1;
   const double per_col = 2.0 * (double)rows * (double)kb;  // flops per trailing column
-  const double c = ((double)rest - panel_s * ATLG_LA_UPD_TFLOPS * 1e12 / per_col) / 4.0;
+  const double ratio = (256.0 - panel_cus) / panel_cus;    // rate of the update side to the panel's
+  const double rate = ATLG_LA_UPD_TFLOPS * 1e12 * (256.0 - panel_cus) / 192.0;
+  const double c = ((double)rest - panel_s * rate / per_col) / (1.0 + ratio);
   long ci = c > 0 ? ((long)c / 128) * 128 : 0;
   ci = std::min(ci, rest - nb2);  // never the next block's columns
   return ci >= 256 ? ci : 0;
@@ -1185,6 +1203,8 @@ panel_coop(int M, int w, int off, S* __restrict__ P, long lda, int* __restrict__
   }
 }
 
+#include "lu_panel.hpp"
+
 // Pivot record published by the last workgroup of a column step.
 template <class S>
 struct PivRec {
@@ -1402,6 +1422,9 @@ struct LU {
   bool small_lds = false;     // runs beside a GEMM: keep kernels' LDS small
   int mb_par = 0;             // mailbox the next multi-workgroup panel uses
   int mb_g[2] = {0, 0};       // grid of each mailbox's last user (0: clean)
+  XpBox* box = nullptr;       // exchange areas of the XCD panel
+  int box_par = 0;            // the one its next multi-workgroup launch uses
+  int xcd_units = 32;         // compute units of one XCD the panel may count on
 };
 
 // Trailing update C -= A * B of a recursion node.
@@ -1470,11 +1493,36 @@ void launch_coop(LU<S>& f, int M, int w, int off, int G, int* lst) {
                                       dim3(CP_THREADS), args, 0, f.s));
 }
 
+// Workgroups of an XCD panel of M rows with maxg compute units of one XCD at
+// hand; 0 when they do not hold it.
+inline int xcd_groups(long M, int maxg) {
+  if (M <= kXpRows1) return 1;
+  maxg = std::min(maxg, kXpMaxG);
+  if (M > (long)maxg * kXpRowsWg) return 0;
+  return std::min(maxg, (int)((M + ATLG_XP_ROWS_PER_WG - 1) / ATLG_XP_ROWS_PER_WG));
+}
+
+template <class S>
+void launch_xcd(LU<S>& f, int M, int w, int off, int G, int* lst) {
+  const int per = (M + G - 1) / G, par = f.box_par;
+  if (G > 1) f.box_par ^= 1;
+  hipLaunchKernelGGL(panel_xcd<S>, dim3(8 * (G - 1) + 1), dim3(64 * ((per + 63) / 64)), 0, f.s, M,
+                     w, off, at(f, off, off), f.lda, f.ipiv, f.dinfo, f.box, par, G, lst,
+                     f.status, f.limit);
+  ATLG_LAUNCHED();
+}
+
 // Factors the leaf panel at (off, off): m rows, w columns, and applies its
 // interchanges to every other column.
 template <class S>
 void leaf(LU<S>& f, long off, long m, int w) {
   int* lst = f.leaf_lists ? f.leaf_lists + (off / PW) * kLeafListInts : f.list;
+  const int xg = (long)PW * f.lda * (long)sizeof(S) < (1L << 31) ? xcd_groups(m, f.xcd_units) : 0;
+  if (xg > 0) {
+    launch_xcd(f, (int)m, w, (int)off, xg, lst);
+    apply_outside(f, off, w, lst);
+    return;
+  }
   const long cap = (long)CP_MAXG * CP_THREADS;
   if (m <= 4 * cap) {
     const int rpt = std::max(ATLG_PANEL_RPT_MIN, m <= cap ? 1 : (m <= 2 * cap ? 2 : 4));
@@ -1665,8 +1713,13 @@ void init_lu(LU<S>& f, hipStream_t s, long M, long N, S* A, long lda, int* ipiv,
   const size_t b_list = 256 + sizeof(int) * (1 + 4 * KC);
   const size_t b_rec = 256 + sizeof(PivRec<S>) * PW;
   const size_t b_cand = sizeof(Cand) * maxblk;
-  char* base = static_cast<char*>(scratch(s, kSlotPanel, b_cb + b_list + 256 + b_rec + b_cand));
+  const size_t b_box = (2 * sizeof(XpBox) + 255) & ~size_t(255);
+  char* base =
+      static_cast<char*>(scratch(s, kSlotPanel, b_cb + b_box + b_list + 256 + b_rec + b_cand));
   f.cb = reinterpret_cast<CoopBuf<S>*>(base);
+  base += b_cb;
+  f.box = reinterpret_cast<XpBox*>(base);
+  base += b_box - b_cb;  // the fields below are placed from base + b_cb
   f.list = reinterpret_cast<int*>(base + b_cb);
   f.ticket = reinterpret_cast<unsigned*>(base + b_cb + b_list);
   f.rec = reinterpret_cast<PivRec<S>*>(base + b_cb + b_list + 256);
@@ -1676,6 +1729,9 @@ void init_lu(LU<S>& f, hipStream_t s, long M, long N, S* A, long lda, int* ipiv,
   ATLG_LAUNCHED();
   f.mb_par = 0;
   f.mb_g[0] = f.mb_g[1] = 0;
+  hipLaunchKernelGGL(xp_init, dim3(2), dim3(256), 0, s, f.box);
+  ATLG_LAUNCHED();
+  f.box_par = 0;
   const long nblk = (std::min(M, N) + kTrsmNB - 1) / kTrsmNB;
   f.Winv = static_cast<S*>(
       scratch(s, kSlotFactInv, sizeof(S) * std::max<long>(nblk, 1) * kTrsmNB * kTrsmNB));
@@ -1760,7 +1816,8 @@ void getrf_lookahead(LU<S>& f0) {
   // rest, so the latency-bound panel never shares a SIMD with the GEMM; the
   // caller's stream forks to the pair and joins at the end.
   hipStream_t caller = s0, sp = nullptr, sg = nullptr;
-  const bool split = ATLG_LA_PANEL_CUS > 0 && split_streams(ATLG_LA_PANEL_CUS, &sp, &sg);
+  const int panel_cus = la_panel_cus(f0.M);
+  const bool split = panel_cus > 0 && split_streams(panel_cus, &sp, &sg);
   if (split) {
     ATLG_HIP(hipEventRecord(aux_event(2), caller));
     ATLG_HIP(hipStreamWaitEvent(sg, aux_event(2), 0));
@@ -1777,6 +1834,8 @@ void getrf_lookahead(LU<S>& f0) {
   f1.status = f0.status;  // failures are reported on the caller's stream
   f1.limit = f0.limit;
   f1.coop = ATLG_LA_COOP != 0;
+  // without reserved units a whole-unit workgroup would wait for the GEMM's
+  f1.xcd_units = split ? panel_cus / 8 : 0;
   f1.small_lds = true;
   f0.leaf_lists = lists;
   f1.leaf_lists = lists;
@@ -1814,7 +1873,8 @@ void getrf_lookahead(LU<S>& f0) {
     // the next panel.
     const long r0 = k1 + nb1, rest = N - r0;
     const long nb2n = std::min(kLaNB, std::max(0L, mn - r0));
-    const long chunk = (split && nb1 > 0 && M > k1) ? la_chunk<S>(rest, M - k1, kb, nb1, nb2n) : 0;
+    const long chunk =
+        (split && nb1 > 0 && M > k1) ? la_chunk<S>(rest, M - k1, kb, nb1, nb2n, panel_cus) : 0;
     if (chunk_pending) {  // the previous step's share on the panel stream
       ATLG_HIP(hipStreamWaitEvent(s0, e_chunk, 0));
       chunk_pending = false;
