@@ -10,6 +10,10 @@
 // 128x128 C tiles in registers.  The same kernel, with a triangle mask,
 // serves SYRK (ATL_dsyrk, AtlasBase/Clint/l3micro.base:2358-2720).
 //
+// Products of too few 128x128 tiles for the device, and the in-place
+// diagonal-block applications, run as independent 32x32 waves
+// (gemm_wave.hpp); gw_form chooses.
+//
 // Tile: 128x128 C per 256-thread workgroup (4 waves in 2x2), each wave a
 // 64x64 sub-tile = 4x4 MFMA 16x16 tiles = 64 FP64 accumulators per lane.
 // K is consumed 16 at a time (4 MFMA k-steps).  Global->LDS loads are 128-bit
@@ -17,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "atlg_internal.hpp"
@@ -678,130 +683,86 @@ __global__ void syreflect_kernel(int N, double* C, long ldc) {
   }
 }
 
-// Products with one short side: C = alpha op(A) B + beta C with M, K <= 128
-// (LEFT), or C = alpha A op(B) + beta C with N, K <= 128.  C may be B (LEFT)
-// or A (else): the diagonal-block applications of TRSM and TRMM, in place.
-// The 128x128 tiling would give them one workgroup per 128 columns (rows);
-// here a workgroup owns a 32-wide strip of the whole short side instead (4x
-// the workgroups), reads all of its strip (and op(A) / op(B), shared through
-// L2) before a barrier, and only then writes the strip back.  16x16 output
-// tiles, four per wave: LEFT, row tiles 2w, 2w+1 by both column tiles; else
-// both row tiles by column tiles 2w, 2w+1.  T: the short operand transposed.
-// tri: 0 all of C, 1 only C(i,j) with i >= j, 2 only i <= j (the stored
-// triangle of a symmetric diagonal block).  SL: 16-deep K slabs whose
-// operands are loaded per round trip; SL > 1 (for launches of fewer
-// workgroups than compute units, where each round trip's latency is the
-// cost) also loads the old C before the K loop.
-constexpr int kStrip = 32;
-template <class S, bool LEFT, bool T, int SL>
-__global__ void __launch_bounds__(256)
-gemm_strip(int M, int N, int K, S alpha, const S* __restrict__ A, long lda,
-           const S* __restrict__ B, long ldb, S beta, S* C, long ldc,
-           const int* __restrict__ skip, int tri) {
-  typedef Mfma<S> MF;
-  if (skip && *skip) return;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, fx = lane & 15, fk = lane >> 4;
-  const int r0 = LEFT ? 0 : (int)blockIdx.x * kStrip;  // first row / column of the strip
-  const int c0 = LEFT ? (int)blockIdx.x * kStrip : 0;
-  int rt[2], ct[2];  // this wave's row / column tile origins
-#pragma unroll
-  for (int e = 0; e < 2; e++) {
-    rt[e] = LEFT ? r0 + 16 * (2 * w + e) : r0 + 16 * e;
-    ct[e] = LEFT ? c0 + 16 * e : c0 + 16 * (2 * w + e);
-  }
-  // element (m, k) of op(A) and (k, n) of op(B); zero outside the matrices
-  auto aval = [&](int m, int k) -> S {
-    if (m >= M || k >= K) return S(0);
-    return (LEFT && T) ? A[k + (size_t)m * lda] : A[m + (size_t)k * lda];
+#include "gemm_wave.hpp"
+
+// Which form a product takes: the 128x128 tiles, or gemm_wave with 64x64
+// tiles (one slice of K) or 32x32 tiles (four slices), whichever the model
+// below takes for the shortest.  A form's time is a launch, then rounds of
+// one tile per compute unit, each a fixed part (first loads, epilogue) and a
+// part per k; the constants are fits, in microseconds, to sweeps of square,
+// flat, tall and deep shapes on the whole device (28 shapes, FP64 and FP32,
+// each form forced; model within 15% for most).  Measured both ways, FP64,
+// 128x128 tiles against the form chosen: 100^3 24.2 -> 8.7 us (8.7 is the
+// Python call), 500^3 84.8 -> 10.4, 1000^3 160 -> 45, 1531x777x2003 336 ->
+// 101, 4000x100x4000 499 -> 93, 3000^3 (K not a multiple of 32) 1295 -> 922;
+// where the tiles fill the device they stay: 2048x2048x128 27 against 32,
+// 1920^3 254 against 319, 65536x256x256 141 against 198.
+enum GwForm : int { kGwNone = 0, kGw64 = 1, kGw32x4 = 2, kGwLeft = 3, kGwRight = 4 };
+struct GwCost {
+  double launch, fixed, per_k;
+};
+template <class S>
+GwForm gw_form(long M, long N, long K, int mode, bool at, bool reg_a, int units) {
+  const bool dbl = std::is_same<S, double>::value;
+  // A transposed: k-contiguous loads touch more lines per instruction
+  const double tr = at ? 1.12 : 1.0;
+  const GwCost c128 = {8.3, 3.6, reg_a ? 0.1165 : (dbl ? 0.148 : 0.092)};
+  const GwCost c64 = {3.5, 2.0, (dbl ? 0.040 : 0.020) * tr};
+  const GwCost c32 = {6.0, 0.8, (dbl ? 0.0092 : 0.0046) * tr};
+  auto time = [&](const GwCost& c, long T) {
+    const long tm = (M + T - 1) / T, tn = (N + T - 1) / T;
+    const double tiles = mode == 0 ? (double)tm * tn : (double)tri_tiles(mode, (int)tm, (int)tn);
+    return c.launch + std::ceil(tiles / units) * (c.fixed + c.per_k * (double)K);
   };
-  auto bval = [&](int k, int n) -> S {
-    if (k >= K || n >= N) return S(0);
-    return (!LEFT && T) ? B[n + (size_t)k * ldb] : B[k + (size_t)n * ldb];
-  };
-  typename MF::acc_t acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++) acc[i][j] = typename MF::acc_t{0, 0, 0, 0};
-  // lane l, register r: C[rt + (l & 15)][ct + c_n(l, r)]
-  S old[2][2][4];
-  auto load_old = [&]() {
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int j = 0; j < 2; j++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int gi = rt[i] + fx, gj = ct[j] + MF::c_n(lane, r);
-          old[i][j][r] = (beta != S(0) && gi < M && gj < N) ? C[gi + (size_t)gj * ldc] : S(0);
-        }
-  };
-  if (SL > 1) load_old();
-  for (int k0 = 0; k0 < K; k0 += 16 * SL) {  // 4 SL MFMA steps' operands in flight
-    S av[SL][4][2], bv[SL][4][2];
-#pragma unroll
-    for (int l = 0; l < SL; l++)
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-          av[l][q][e] = aval(rt[e] + fx, k0 + 16 * l + 4 * q + fk);
-          bv[l][q][e] = bval(k0 + 16 * l + 4 * q + fk, ct[e] + fx);
-        }
-#pragma unroll
-    for (int l = 0; l < SL; l++)
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-          for (int j = 0; j < 2; j++) acc[i][j] = MF::op(bv[l][q][j], av[l][q][i], acc[i][j]);
-  }
-  if (SL == 1) load_old();
-  __syncthreads();  // every read of the strip precedes every write
-#pragma unroll
-  for (int i = 0; i < 2; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int gi = rt[i] + fx, gj = ct[j] + MF::c_n(lane, r);
-        if (gi < M && gj < N && !(tri == 1 && gi < gj) && !(tri == 2 && gi > gj))
-          C[gi + (size_t)gj * ldc] =
-              (beta == S(0)) ? alpha * acc[i][j][r] : alpha * acc[i][j][r] + beta * old[i][j][r];
-      }
+  const double t128 = time(c128, BM), t64 = time(c64, 2 * GW_T), t32 = time(c32, GW_T);
+  if (t128 <= t64 && t128 <= t32) return kGwNone;
+  return t64 <= t32 ? kGw64 : kGw32x4;
 }
 
-// Strip launches of fewer workgroups than this (a fraction of the device's
-// 256 compute units, latency-bound) load four K slabs per round trip.
-#ifndef ATLG_STRIP_DEEP_MAX
-#define ATLG_STRIP_DEEP_MAX 256
-#endif
-template <class S>
-void launch_strip(hipStream_t s, bool left, bool t, long M, long N, long K, S alpha, const S* A,
-                  long lda, const S* B, long ldb, S beta, S* C, long ldc, const int* skip,
-                  int tri) {
-  const long nstrips = ((left ? N : M) + kStrip - 1) / kStrip;
-  const dim3 gs((unsigned)nstrips);
-  const bool deep = nstrips < ATLG_STRIP_DEEP_MAX;
-#define ATLG_STRIP(L_, T_)                                                                   \
-  do {                                                                                       \
-    if (deep)                                                                                \
-      hipLaunchKernelGGL((gemm_strip<S, L_, T_, 4>), gs, dim3(256), 0, s, (int)M, (int)N,   \
-                         (int)K, alpha, A, lda, B, ldb, beta, C, ldc, skip, tri);            \
-    else                                                                                     \
-      hipLaunchKernelGGL((gemm_strip<S, L_, T_, 1>), gs, dim3(256), 0, s, (int)M, (int)N,   \
-                         (int)K, alpha, A, lda, B, ldb, beta, C, ldc, skip, tri);            \
+// Launches gemm_wave.  kGwLeft / kGwRight: one workgroup owns all of a short
+// side of at most 128 (four waves) and 32 of the long one and reads all of
+// its inputs before it writes, so C may be B (Left) or A (Right): the
+// diagonal-block applications of TRSM and TRMM.  (They were 32-wide strips
+// loaded element by element: 128x1701x128 17.4 -> 9.9 us, with op(A)
+// transposed 22.3 -> 11.9; two or four slices of K were slower.)
+template <class S, bool AT, bool BT>
+void launch_gw(hipStream_t s, GwForm form, long M, long N, long K, S alpha, const S* A, long lda,
+               const S* B, long ldb, S beta, S* C, long ldc, int mode, const int* skip) {
+#define ATLG_GO(WM_, WN_, WS_)                                                                \
+  do {                                                                                        \
+    const int tm_ = (int)((M + GW_T * WM_ - 1) / (GW_T * WM_));                               \
+    const int tn_ = (int)((N + GW_T * WN_ - 1) / (GW_T * WN_));                               \
+    const int nt_ = mode == 0 || WM_ != WN_ ? tm_ * tn_ : tri_tiles(mode, tm_, tn_);          \
+    hipLaunchKernelGGL((gemm_wave<S, AT, BT, WM_, WN_, WS_>), dim3((unsigned)nt_),            \
+                       dim3(64 * WM_ * WN_ * WS_), 0, s, (int)M, (int)N, (int)K, alpha, A,    \
+                       lda, B, ldb, beta, C, ldc, mode, skip);                                \
   } while (0)
-  if (left) {
-    if (t) ATLG_STRIP(true, true);
-    else ATLG_STRIP(true, false);
-  } else {
-    if (t) ATLG_STRIP(false, true);
-    else ATLG_STRIP(false, false);
+  switch (form) {
+    case kGw64: ATLG_GO(2, 2, 1); break;
+    case kGw32x4: ATLG_GO(1, 1, 4); break;
+    case kGwLeft:
+      if constexpr (!BT) ATLG_GO(4, 1, 1);
+      break;
+    case kGwRight:
+      if constexpr (!AT) ATLG_GO(1, 4, 1);
+      break;
+    default: break;
   }
-#undef ATLG_STRIP
+#undef ATLG_GO
   ATLG_LAUNCHED();
+}
+template <class S>
+void launch_gw(hipStream_t s, GwForm form, bool at, bool bt, long M, long N, long K, S alpha,
+               const S* A, long lda, const S* B, long ldb, S beta, S* C, long ldc, int mode,
+               const int* skip) {
+  if (!at && !bt)
+    launch_gw<S, false, false>(s, form, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, mode, skip);
+  else if (!at)
+    launch_gw<S, false, true>(s, form, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, mode, skip);
+  else if (!bt)
+    launch_gw<S, true, false>(s, form, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, mode, skip);
+  else
+    launch_gw<S, true, true>(s, form, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, mode, skip);
 }
 
 template <class S, bool AT, bool BT>
@@ -854,26 +815,30 @@ void gemm(hipStream_t s, int TA, int TB, long M, long N, long K, S alpha, const 
   if (max_wg > 0 && nwg > max_wg) nwg = std::max(8L, (long)(max_wg / 8) * 8);
   const dim3 g((unsigned)nwg);
   const bool at = is_trans(TA), bt = is_trans(TB);
-  // in-place diagonal-block applications (C is B, or C is A) with a short
-  // side of at most 128: strips of 32 across the long side
-  if (mode == 0 && C == B && C != A && M <= BM && K <= BM && !bt) {
-    launch_strip<S>(s, true, at, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, skip, 0);
-    return;
-  }
-  if (mode == 0 && C == A && C != B && N <= BN && K <= BN && !at) {
-    launch_strip<S>(s, false, bt, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, skip, 0);
-    return;
-  }
   const bool va = aligned16<S>(A, lda), vb = aligned16<S>(B, ldb);
   // FP64 with aligned operands, K a multiple of 32 and C not one of the
   // operands (TRSM's in-place diagonal apply): A straight to registers, B
   // through LDS (per-lane byte offsets inside a tile are 32-bit: 128
   // columns or 16 rows of B, 4 columns plus 128 rows or 128 columns of A).
   // Not for A^T x B^T, whose form needs more than 256 registers.
-  if (std::is_same<S, double>::value && !(at && bt) && va && vb && K % (2 * BK) == 0 &&
-      C != A && C != B &&
-      8L * (at ? BM * lda + BK : 4 * lda + BM) < (1L << 31) &&
-      8L * (bt ? BK * ldb + BN : BN * ldb + BK) < (1L << 31)) {
+  const bool reg_a = std::is_same<S, double>::value && !(at && bt) && va && vb &&
+                     K % (2 * BK) == 0 && C != A && C != B &&
+                     8L * (at ? BM * lda + BK : 4 * lda + BM) < (1L << 31) &&
+                     8L * (bt ? BK * ldb + BN : BN * ldb + BK) < (1L << 31);
+  // waves of 32x32: in place with a short side of at most 128, or where the
+  // 128x128 tiles are too few (per-lane byte offsets inside a tile are 32-bit)
+  if (8L * GW_T * std::max(lda, ldb) < (1L << 31)) {
+    GwForm form = kGwNone;
+    if (mode == 0 && C == B && C != A && M <= BM && K <= BM && !bt) form = kGwLeft;
+    else if (mode == 0 && C == A && C != B && N <= BN && K <= BN && !at) form = kGwRight;
+    else if (C != A && C != B && max_wg <= 0)
+      form = gw_form<S>(M, N, K, mode, at, reg_a, stream_units(s));
+    if (form != kGwNone) {
+      launch_gw<S>(s, form, at, bt, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, mode, skip);
+      return;
+    }
+  }
+  if (reg_a) {
     const int vecc = aligned16<S>(C, ldc) ? 1 : 0;
     hipLaunchKernelGGL(at ? gemm_tn_f64 : (bt ? gemm_nt_f64 : gemm_nn_f64),
                        g, dim3(NT), 0, s, (int)M, (int)N, (int)K, (double)alpha,
@@ -896,21 +861,6 @@ void gemm(hipStream_t s, int TA, int TB, long M, long N, long K, S alpha, const 
     launch_t<S, true, true>(s, g, va, vb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, mode,
                             skip);
   ATLG_LAUNCHED();
-}
-
-template <class S>
-bool gemm_narrow(hipStream_t s, int TA, int TB, long M, long N, long K, S alpha, const S* A,
-                 long lda, const S* B, long ldb, S beta, S* C, long ldc, int tri,
-                 const int* skip) {
-  const bool at = is_trans(TA), bt = is_trans(TB);
-  if (M <= 0 || N <= 0 || K <= 0 || K > BM || M > (1L << 30) || N > (1L << 30)) return false;
-  if (N <= BN && !at)  // strips of 32 rows by all N columns
-    launch_strip<S>(s, false, bt, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, skip, tri);
-  else if (M <= BM && !bt)  // strips of 32 columns by all M rows
-    launch_strip<S>(s, true, at, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, skip, tri);
-  else
-    return false;
-  return true;
 }
 
 bool gemm_batched(hipStream_t s, int TA, int TB, long M, long N, long K, double alpha,
@@ -946,10 +896,5 @@ template void gemm<double>(hipStream_t, int, int, long, long, long, double, cons
                            const double*, long, double, double*, long, int, const int*, int);
 template void gemm<float>(hipStream_t, int, int, long, long, long, float, const float*, long,
                           const float*, long, float, float*, long, int, const int*, int);
-template bool gemm_narrow<double>(hipStream_t, int, int, long, long, long, double, const double*,
-                                  long, const double*, long, double, double*, long, int,
-                                  const int*);
-template bool gemm_narrow<float>(hipStream_t, int, int, long, long, long, float, const float*,
-                                 long, const float*, long, float, float*, long, int, const int*);
 
 }  // namespace atlg

@@ -1506,10 +1506,23 @@ template <class S>
 void launch_xcd(LU<S>& f, int M, int w, int off, int G, int* lst) {
   const int per = (M + G - 1) / G, par = f.box_par;
   if (G > 1) f.box_par ^= 1;
-  hipLaunchKernelGGL(panel_xcd<S>, dim3(8 * (G - 1) + 1), dim3(64 * ((per + 63) / 64)), 0, f.s, M,
-                     w, off, at(f, off, off), f.lda, f.ipiv, f.dinfo, f.box, par, G, lst,
-                     f.status, f.limit);
-  ATLG_LAUNCHED();
+  const dim3 grid(8 * (G - 1) + 1), block(64 * ((per + 63) / 64));
+  S* P = at(f, off, off);
+  if (G == 1 || !f.coop) {
+    hipLaunchKernelGGL(panel_xcd<S>, grid, block, 0, f.s, M, w, off, P, f.lda, f.ipiv, f.dinfo,
+                       f.box, par, G, lst, f.status, f.limit);
+    ATLG_LAUNCHED();
+    return;
+  }
+  // Outside the look-ahead's reserved units, panels of several callers'
+  // streams could hold an XCD's units while each waits for more of its own
+  // workgroups: cooperative launches do not overlap each other.
+  int p = par, g = G;
+  long lda = f.lda;
+  void* args[] = {&M,     &w, &off, &P, &lda,      &f.ipiv, &f.dinfo,
+                  &f.box, &p, &g,   &lst, &f.status, &f.limit};
+  ATLG_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&panel_xcd<S>), grid, block,
+                                      args, 0, f.s));
 }
 
 // Factors the leaf panel at (off, off): m rows, w columns, and applies its

@@ -315,10 +315,9 @@ constexpr long kCholLaMin = 2048;
 #define ATLG_CHOL_STEP 0
 #endif
 // Widest block (columns) whose look-ahead update goes in two parts, the
-// diagonal block's triangle and then the rest of the block column, both by
-// 32-row strips (gemm_narrow): the leaf starts after the first part.  N=8192
-// (128-column steps): 10.9 -> 10.3 ms; for the 256/384-column steps of
-// N=12288/16384 the split, by the 128x128 tiling, was 1 ms slower.
+// diagonal block's triangle and then the rest of the block column: the leaf
+// starts after the first part.  N=8192 (128-column steps): 10.9 -> 10.3 ms;
+// for the 256/384-column steps of N=12288/16384 the split was 1 ms slower.
 #ifndef ATLG_CHOL_SPLIT_MAX
 #define ATLG_CHOL_SPLIT_MAX 128
 #endif
@@ -411,29 +410,18 @@ void potrf_lookahead(hipStream_t s0, bool lower, long N, double* A, long lda, in
     }
   };
   // the off-diagonal part of block column c0 (nc wide, r rows/columns past
-  // it) minus the product of block k's panel rows: narrow blocks by strips
+  // it) minus the product of block k's panel rows
   auto update_col = [&](hipStream_t s, long k, long kb, long c0, long nc, long r) {
     if (r <= 0) return;
-    if (lower) {
-      if (!gemm_narrow(s, kNoTrans, kTrans, r, nc, kb, -1.0, at(c0 + nc, k), lda, at(c0, k), lda,
-                       1.0, at(c0 + nc, c0), lda, 0, dinfo))
-        gemm(s, kNoTrans, kTrans, r, nc, kb, -1.0, at(c0 + nc, k), lda, at(c0, k), lda, 1.0,
-             at(c0 + nc, c0), lda, 0, dinfo);
-    } else {
-      if (!gemm_narrow(s, kTrans, kNoTrans, nc, r, kb, -1.0, at(k, c0), lda, at(k, c0 + nc), lda,
-                       1.0, at(c0, c0 + nc), lda, 0, dinfo))
-        gemm(s, kTrans, kNoTrans, nc, r, kb, -1.0, at(k, c0), lda, at(k, c0 + nc), lda, 1.0,
-             at(c0, c0 + nc), lda, 0, dinfo);
-    }
+    if (lower)
+      gemm(s, kNoTrans, kTrans, r, nc, kb, -1.0, at(c0 + nc, k), lda, at(c0, k), lda, 1.0,
+           at(c0 + nc, c0), lda, 0, dinfo);
+    else
+      gemm(s, kTrans, kNoTrans, nc, r, kb, -1.0, at(k, c0), lda, at(k, c0 + nc), lda, 1.0,
+           at(c0, c0 + nc), lda, 0, dinfo);
   };
   // the stored triangle of diagonal block c0 (nc wide) likewise
   auto update_diag = [&](hipStream_t s, long k, long kb, long c0, long nc) {
-    const double* P = lower ? at(c0, k) : at(k, c0);
-    if (lower ? gemm_narrow(s, kNoTrans, kTrans, nc, nc, kb, -1.0, P, lda, P, lda, 1.0,
-                            at(c0, c0), lda, 1, dinfo)
-              : gemm_narrow(s, kTrans, kNoTrans, nc, nc, kb, -1.0, P, lda, P, lda, 1.0,
-                            at(c0, c0), lda, 2, dinfo))
-      return;
     update(s, k, kb, c0, nc, nc, 0);
   };
   hipEvent_t e_col = aux_event(4);

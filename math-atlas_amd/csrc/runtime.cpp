@@ -74,6 +74,7 @@ struct Aux {
   std::map<int, std::pair<hipStream_t, hipStream_t>> split;
 };
 std::map<int, Aux> g_aux;
+std::map<hipStream_t, int> g_units;  // CU-masked stream -> its compute units
 Aux& aux_for_device() {
   int dev = 0;
   ATLG_HIP(hipGetDevice(&dev));
@@ -115,12 +116,34 @@ bool split_streams(int cus, hipStream_t* small, hipStream_t* large) {
         p[0] = p[1] = nullptr;
       }
     }
+    if (p[0]) {
+      g_units[p[0]] = cus;
+      g_units[p[1]] = total - cus;
+    }
     it = a.split.emplace(cus, std::make_pair(p[0], p[1])).first;
   }
   if (!it->second.first) return false;
   *small = it->second.first;
   *large = it->second.second;
   return true;
+}
+
+int stream_units(hipStream_t s) {
+  constexpr int kDevices = 64;
+  static std::atomic<int> total[kDevices];  // by device, 0: not asked yet
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    auto it = g_units.find(s);
+    if (it != g_units.end()) return it->second;
+  }
+  int dev = 0, n = 0;
+  ATLG_HIP(hipGetDevice(&dev));
+  if (dev >= 0 && dev < kDevices) n = total[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    ATLG_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
+    if (dev >= 0 && dev < kDevices) total[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
 }
 
 void* scratch(hipStream_t s, Slot slot, size_t bytes) {
