@@ -23,9 +23,6 @@ namespace atlg {
 namespace {
 
 constexpr int DB = kTrsmNB;    // diagonal block order
-constexpr int LDS_LD = kTriLD;
-constexpr int P_THREADS = kTriThreads;
-static_assert(DB == kTriN, "leaf order must match the block inverter");
 
 // Broadcast of lane `src`'s value (uniform src) through the scalar unit.
 __device__ __forceinline__ double lane_value(double v, int src) {
@@ -36,20 +33,6 @@ __device__ __forceinline__ double lane_value(double v, int src) {
                               static_cast<unsigned int>(lo));
 }
 
-// 1/sqrt(d) for d > 0: the hardware estimate and two Newton steps
-// (quadratic convergence from its ~2^-23 relative error to below an ulp);
-// values below 2^-1000, where the estimate loses range, take sqrt and a
-// division.
-__device__ __forceinline__ double rsqrt_pos(double d) {
-  if (d < 0x1p-1000) return 1.0 / sqrt(d);
-  double y = __builtin_amdgcn_rsq(d);
-  const double h = 0.5 * d;
-  y = y * (1.5 - h * y * y);
-  y = y * (1.5 - h * y * y);
-  return y;
-}
-
-constexpr int SB = 32;  // sub-block order of the in-workgroup factorization
 #ifndef ATLG_POTRF_RB
 #define ATLG_POTRF_RB 384
 #endif
@@ -59,194 +42,291 @@ constexpr long RB = ATLG_POTRF_RB;  // block width of the right-looking outer st
 // block to Dinv (DB x DB, column-major, zeros above the diagonal).
 // lower: A = L L^T from the lower triangle; else A = U^T U from the upper
 // triangle, handled as L = U^T, so one algorithm serves both.  The other
-// triangle of A is never read or written.
+// triangle of A is never read or written; order beyond n is padded with the
+// identity.
 //
-// Factorization (right-looking, 32-wide panels, the block held in LDS;
-// order beyond n is padded with the identity), per panel:
-//   1. wave 0 holds the panel's 32 x 32 diagonal block and the 32 rows
-//      below it in registers, lane i one row, and factors them column by
-//      column: the pivot from lane j by v_readlane, multipliers scaled by
-//      the reciprocal square root (ATLAS's potrfL closed forms multiply by
-//      the reciprocal too), the column's diagonal-block part broadcast to
-//      the other lanes through LDS; no barrier inside the panel;
-//   2. the remaining rows solve X L11^T = A21 right-looking (one row per
-//      thread, the 31 - k updates of step k independent of each other);
-//   3. the trailing lower triangle A22 -= X X^T on the matrix cores.
-// The factor is then inverted in LDS (lower_inverse_inplace).
-__global__ void __launch_bounds__(P_THREADS)
+// What bounds it: the chain of 128 pivots on one compute unit.  Everything is
+// kept in the layout of the matrix core's accumulator: lane (n, k) =
+// (l & 15, l >> 4) holds, of a 16x16 tile, row n and the columns 4 b + k in
+// register b.  A register is then at once the 16x4 and the 4x16 operand of a
+// 16x16x4 MFMA, so a block of four columns needs no data movement: its rows
+// below are X' = X inv(L11)^T (one MFMA per tile, with the 4x4 inverse), and
+// its share of the tile's other columns is one MFMA of X' with X'.
+// Left-looking by 16-column steps d over the tiles in LDS; wave 0 runs the
+// chain, eight waves have one tile each:
+//   1. wave 0 factors tile (d, d) four columns at a time: the 4x4 block
+//      through v_readlane, its factor by every lane alike, X' and
+//      the tile's own update by MFMA, an identity tile carried along to the
+//      tile's inverse.  Beside it the other waves subtract the earlier
+//      columns' products from their tile of column d, and the one whose tile
+//      is that inverse from the next diagonal tile;
+//   2. they multiply their tile by the diagonal tile's inverse.
+// The identity rides along below the block: its rows become L^-T, so the
+// inverse costs MFMAs beside the factorization instead of a chain of its own,
+// and column d always has eight tiles: block rows d + 1 .. 7 and identity
+// rows 0 .. d.  A step is 5400 cycles of factor and 1500 of solve and next
+// diagonal; the block with its inverse takes 28 us (80 us as 32-wide panels
+// factored column by column through LDS, the inverse by doubling after it).
+constexpr int PT = 16;              // tile order
+constexpr int PTN = DB / PT;        // tiles per side
+// Waves are dealt to the four SIMDs in turn: 0 is the chain's, waves 4 and 8
+// only keep its SIMD free, and the tiles go to the others.
+constexpr int PW_WAVES = 11, PW_THREADS = 64 * PW_WAVES;
+// LDS pitches: lane (n, k) reads row n, column k of four: 4 n + k covers the
+// bank pairs evenly
+constexpr int PLD = DB + 4, YLD = PT + 4;
+
+// 1/sqrt(d), d > 0: the hardware estimate (about 2^-23) and one third-order
+// step; the products stay in range for subnormal d.
+__device__ __forceinline__ double rsqrt3(double d) {
+  const double y = __builtin_amdgcn_rsq(d);
+  const double e = __builtin_fma(-(d * y), y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+}
+
+__global__ void __launch_bounds__(PW_THREADS)
 potf2_inv_kernel(int n, double* __restrict__ A, long lda, int lower, int* __restrict__ dinfo,
                  int info_off, double* __restrict__ Dinv) {
-  if (*dinfo != 0) return;
-  __shared__ double S[DB * LDS_LD];
-  __shared__ double LT[SB * SB];   // the panel's diagonal block, transposed
-  __shared__ double rinv_sh[SB];   // its reciprocal pivots
-  __shared__ double cbuf[64];      // wave 0's column broadcast
+  typedef TriMfma<double> TM;
+  typedef TM::acc_t acc_t;
+  const int failed = *dinfo;  // an earlier block's failure: looked at once the loads are issued
+  __shared__ double S[DB * PLD];        // A, then L below and on the diagonal, L^-T above it
+  __shared__ double Y[PTN][PT * YLD];   // diagonal tiles of L^-T
+  // the next diagonal tile, products of the columns before d taken off
+  // (alternating: wave 0 reads one while the next is written)
+  __shared__ double N[2][4][64];
   __shared__ int fail_sh;
-  const int t = threadIdx.x;
-  // fill in batches of 16 elements per thread, all loads of a batch in
-  // flight before the LDS stores
-  constexpr int PER = DB * DB / P_THREADS, BATCH = 16;
-  static_assert(PER % BATCH == 0, "fill batches");
-  for (int b0 = 0; b0 < PER; b0 += BATCH) {
-    double v[BATCH];
+  const int t = threadIdx.x, lane = t & 63, hw = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int w = hw % 4 == 0 ? (hw == 0 ? 0 : -1) : hw - hw / 4;  // 0: the chain, 1..8: tiles
+  const int ln = lane & 15, lk = lane >> 4;
+  const acc_t zero = {0, 0, 0, 0};
+  // element (i, c), i >= c, of the block
+  auto store = [&](int i, int c, double x) {
+    if (i < n && c <= i) {
+      if (lower) A[i + (size_t)c * lda] = x;
+      else A[c + (size_t)i * lda] = x;
+    }
+  };
+  // fill: the tiles on and below the diagonal, 36 of them, four per working
+  // wave, all loads in flight
+  if (w >= 0) {
+    double v[4][4];
+    int ti[4], tc[4];
 #pragma unroll
-    for (int u = 0; u < BATCH; u++) {
-      const int idx = t + (b0 + u) * P_THREADS;
-      const int i = idx % DB, k = idx / DB;
-      double x = 0.0;
-      if (i >= k) {
-        if (i < n && k < n) x = lower ? A[i + (size_t)k * lda] : A[k + (size_t)i * lda];
-        else if (i == k) x = 1.0;
+    for (int q = 0; q < 4; q++) {
+      int u = w + (1 + PTN) * q, i = 0;
+      while (u > i) u -= ++i;
+      ti[q] = i;
+      tc[q] = u;
+      const int gi = PT * i + ln;
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        const int c = PT * u + 4 * b + lk;
+        v[q][b] = gi == c ? 1.0 : 0.0;
+        if (gi < n && c <= gi) v[q][b] = lower ? A[gi + (size_t)c * lda] : A[c + (size_t)gi * lda];
       }
-      v[u] = x;
+    }
+    // the inverse's tiles above the diagonal
+    if (failed == 0)
+    for (int u = w; u < PTN * (PTN - 1) / 2; u += 1 + PTN) {
+      int c = 1, i = u;
+      while (i >= c) i -= c++;
+      double* z = Dinv + PT * i + ln + (size_t)(PT * c + lk) * DB;
+#pragma unroll
+      for (int b = 0; b < 4; b++) z[4 * b * DB] = 0.0;
     }
 #pragma unroll
-    for (int u = 0; u < BATCH; u++) {
-      const int idx = t + (b0 + u) * P_THREADS;
-      S[(idx % DB) * LDS_LD + idx / DB] = v[u];
-    }
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int b = 0; b < 4; b++)
+        S[(PT * ti[q] + ln) * PLD + PT * tc[q] + 4 * b + lk] = v[q][b];
   }
+  if (failed != 0) return;
   if (t == 0) fail_sh = -1;
   __syncthreads();
 
-  int fail = -1;
-  for (int kb = 0; kb < DB; kb += SB) {
-    // 1. wave 0: lane i holds panel row kb + i (the 32 x 32 diagonal block
-    //    for i < 32, the next 32 rows below it for i >= 32) and factors the
-    //    panel right-looking: per column j the pivot comes from lane j
-    //    (v_readlane), the multipliers L(i, j) are scaled by the reciprocal
-    //    square root, and column j's part inside the diagonal block reaches
-    //    the other lanes through a wave-private LDS line (ordered within the
-    //    wave: no barrier)
-    if (t < 64) {
-      const int i = t, r = kb + i;
-      const bool have = r < DB;
-      double x[SB];
+  acc_t T = zero;  // wave 0: the diagonal tile, the others: their tile
+  double keep[4] = {0, 0, 0, 0};  // a finished tile on its way to memory
+  if (w == 0) {
 #pragma unroll
-      for (int c = 0; c < SB; c++)
-        x[c] = (have && (i >= SB || c <= i)) ? S[r * LDS_LD + kb + c] : 0.0;
-      // The chain from one pivot to the next is kept short: the next
-      // column's update (one FMA with the multiplier of row j+1, taken by
-      // v_readlane) and the next pivot's reciprocal square root come first;
-      // the other columns' updates read the column from LDS off that path.
-      int f = -1;  // first non-positive pivot (uniform)
-      double d = lane_value(x[0], 0);
-      int bad = __builtin_amdgcn_readfirstlane((int)!(d > 0.0));
-      double y = bad ? 0.0 : rsqrt_pos(d);
-      double yi = 0.0;  // lane i < 32: its own reciprocal pivot
-#pragma unroll
-      for (int j = 0; j < SB; j++) {
-        if (bad) {
-          f = j;
-          break;
-        }
-        const double L = (i == j) ? d * y : x[j] * y;
-        if (i >= j) x[j] = L;
-        if (i == j) yi = y;
-        const double Lm = (i > j) ? L : 0.0;  // lanes <= j: no update
-        // column j to LDS and back (all reads in flight together), the
-        // next pivot computed while they travel
-        cbuf[i] = L;
-        double cv[SB];
-#pragma unroll
-        for (int c = j + 2; c < SB; c++) cv[c] = cbuf[c];
-        __builtin_amdgcn_sched_barrier(0);
-        if (j + 1 < SB) {
-          x[j + 1] -= Lm * lane_value(L, j + 1);
-          d = lane_value(x[j + 1], j + 1);
-          bad = __builtin_amdgcn_readfirstlane((int)!(d > 0.0));
-          y = bad ? 0.0 : rsqrt_pos(d);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int c = j + 2; c < SB; c++) x[c] -= Lm * cv[c];
-      }
-      if (have) {
-#pragma unroll
-        for (int c = 0; c < SB; c++)
-          if (i >= SB || c <= i) S[r * LDS_LD + kb + c] = x[c];
-      }
-      if (i < SB) {  // the diagonal block transposed: LT[k][c] = L(kb+c, kb+k)
-        rinv_sh[i] = yi;
-#pragma unroll
-        for (int k = 0; k < SB; k++) LT[k * SB + i] = x[k];
-      }
-      if (t == 0) fail_sh = f >= 0 ? kb + f : -1;
-    }
-    __syncthreads();
-    fail = fail_sh;
-    if (fail >= 0) break;
-    const int r0 = kb + SB, nrow = DB - r0;
-    if (nrow <= 0) break;
-    // 2. the rows beyond wave 0's (kb + 64 ..): X L11^T = A21 right-looking,
-    //    the column updates of one step independent of each other
-    if (t >= 64 && kb + t < DB) {
-      const int r = kb + t;
-      double x[SB];
-#pragma unroll
-      for (int c = 0; c < SB; c++) x[c] = S[r * LDS_LD + kb + c];
-#pragma unroll
-      for (int k = 0; k < SB; k++) {
-        double cv[SB];  // row k of LT, all reads in flight together
-        const double rk = rinv_sh[k];
-#pragma unroll
-        for (int c = k + 1; c < SB; c++) cv[c] = LT[k * SB + c];
-        __builtin_amdgcn_sched_barrier(0);
-        x[k] *= rk;
-#pragma unroll
-        for (int c = k + 1; c < SB; c++) x[c] -= x[k] * cv[c];
-      }
-#pragma unroll
-      for (int c = 0; c < SB; c++) S[r * LDS_LD + kb + c] = x[c];
-    }
-    __syncthreads();
-    // 3. trailing lower triangle A22 -= X X^T on the matrix cores: 16 x 16
-    //    tiles (ti >= tj) of the nrow x nrow block, K = 32 in eight steps
-    {
-      typedef TriMfma<double> TM;
-      const int lane = t & 63, wv = t >> 6, lx = lane & 15, lk = lane >> 4;
-      const int T = nrow / 16, ntile = T * (T + 1) / 2;
-      for (int u = wv; u < ntile; u += P_THREADS / 64) {
-        int ti = (int)((sqrtf(8.0f * u + 1.0f) - 1.0f) * 0.5f);
-        while (ti * (ti + 1) / 2 > u) ti--;
-        while ((ti + 1) * (ti + 2) / 2 <= u) ti++;
-        const int tj = u - ti * (ti + 1) / 2;
-        const int ra = r0 + 16 * ti + lx, rb = r0 + 16 * tj + lx;
-        double av[SB / 4], bv[SB / 4];
-#pragma unroll
-        for (int q = 0; q < SB / 4; q++) {
-          av[q] = S[ra * LDS_LD + kb + 4 * q + lk];
-          bv[q] = S[rb * LDS_LD + kb + 4 * q + lk];
-        }
-        TM::acc_t acc = {0, 0, 0, 0};
-#pragma unroll
-        for (int q = 0; q < SB / 4; q++) acc = TM::op(av[q], bv[q], acc);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const int gi = r0 + 16 * ti + TM::row(lane, e), gk = r0 + 16 * tj + lx;
-          if (gi >= gk) S[gi * LDS_LD + gk] -= acc[e];
-        }
-      }
-    }
-    __syncthreads();
+    for (int b = 0; b < 4; b++) T[b] = S[ln * PLD + 4 * b + lk];
   }
-  if (fail >= 0 && t == 0) *dinfo = info_off + fail + 1;
-  // write back (on failure: the partially factored block, as ATLAS leaves it)
-  for (int idx = t; idx < DB * DB; idx += P_THREADS) {
-    const int i = idx % DB, k = idx / DB;
-    if (i >= k && i < n && k < n) {
-      if (lower) A[i + (size_t)k * lda] = S[i * LDS_LD + k];
-      else A[k + (size_t)i * lda] = S[i * LDS_LD + k];
+  for (int d = 0; d < PTN; d++) {
+    const int c0 = PT * d;
+    const double* row_d = S + (c0 + ln) * PLD + lk;  // tile row d, this lane's entries
+    // this wave's tile: block row `rt` (L) or identity row `rt` (L^-T)
+    const bool inv = w >= PTN - d;  // w = 1 .. 7 - d: block rows, then identity rows 0 .. d
+    const int rt = inv ? w - (PTN - d) : d + w;
+    if (w == 0) {
+      int bad = -1;  // first non-positive pivot of the tile
+      acc_t Z;       // the identity on its way to the transposed inverse
+#pragma unroll
+      for (int b = 0; b < 4; b++) Z[b] = ln == 4 * b + lk ? 1.0 : 0.0;
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        double a[4][4], r[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+          for (int i = j; i < 4; i++) a[i][j] = lane_value(T[b], 16 * j + 4 * b + i);
+        bool pos = true;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          if (!(a[j][j] > 0.0) && pos) {
+            pos = false;
+            bad = 4 * b + j;
+          }
+          r[j] = rsqrt3(a[j][j]);
+          a[j][j] *= r[j];
+#pragma unroll
+          for (int i = j + 1; i < 4; i++) a[i][j] *= r[j];
+#pragma unroll
+          for (int c = j + 1; c < 4; c++)
+#pragma unroll
+            for (int i = c; i < 4; i++) a[i][c] -= a[i][j] * a[c][j];
+        }
+        bad = __builtin_amdgcn_readfirstlane(bad);
+        if (bad >= 0) break;
+        // inv(L11): every lane solves for the column lk, and keeps row ln of it
+        double wc[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          double sum = lk == i ? 1.0 : 0.0;
+#pragma unroll
+          for (int c = 0; c < i; c++) sum -= a[i][c] * wc[c];
+          wc[i] = sum * r[i];
+        }
+        double wo = ln < 4 ? wc[0] : 0.0;
+#pragma unroll
+        for (int i = 1; i < 4; i++) wo = ln == i ? wc[i] : wo;
+        const acc_t x = TM::op(wo, T[b], zero);
+        const acc_t z = TM::op(wo, Z[b], zero);
+        __builtin_amdgcn_sched_barrier(0);  // stores in the shadow of the MFMAs
+        if (lane == 0) {
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int c = 0; c <= i; c++) S[(c0 + 4 * b + i) * PLD + c0 + 4 * b + c] = a[i][c];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const double xm = ln >= 4 * b + 4 ? x[0] : 0.0;
+        if (b < 3) {
+          T = TM::op(-xm, xm, T);
+          Z = TM::op(-xm, z[0], Z);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (ln >= 4 * b + 4) S[(c0 + ln) * PLD + c0 + 4 * b + lk] = xm;
+        Y[d][ln * YLD + 4 * b + lk] = z[0];
+      }
+      if (lane == 0 && bad >= 0) fail_sh = c0 + bad;
+    } else if (w > 0) {
+      // T = A(rt, d) - sum over e < d of X(rt, e) X(d, e)^T; identity rows
+      // start at their own column
+      const double* row = S + (PT * rt + ln) * PLD + lk;
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        const double x = row[c0 + 4 * b];
+        T[b] = inv ? (rt == d && ln == 4 * b + lk ? 1.0 : 0.0) : x;
+      }
+      acc_t T2 = zero;
+      for (int e = inv ? rt : 0; e < d; e++) {
+        const double* x2 = inv && e == rt ? &Y[rt][ln * YLD + lk] : row + PT * e;
+        double p[4], q[4];
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+          p[b] = -row_d[PT * e + 4 * b];
+          q[b] = x2[4 * b];
+        }
+        T = TM::op(p[0], q[0], T);
+        T2 = TM::op(p[1], q[1], T2);
+        T = TM::op(p[2], q[2], T);
+        T2 = TM::op(p[3], q[3], T2);
+      }
+#pragma unroll
+      for (int b = 0; b < 4; b++) T[b] += T2[b];
+      if (w == PTN && d + 1 < PTN) {
+        // identity row d has no products yet: this wave does the next
+        // diagonal tile's
+        const double* row_n = row_d + PT * PLD;
+        acc_t U = zero, U2 = zero;
+#pragma unroll
+        for (int b = 0; b < 4; b++) U[b] = row_n[c0 + PT + 4 * b];
+        for (int e = 0; e < d; e++) {
+          double p[4];
+#pragma unroll
+          for (int b = 0; b < 4; b++) p[b] = row_n[PT * e + 4 * b];
+          U = TM::op(-p[0], p[0], U);
+          U2 = TM::op(-p[1], p[1], U2);
+          U = TM::op(-p[2], p[2], U);
+          U2 = TM::op(-p[3], p[3], U2);
+        }
+#pragma unroll
+        for (int b = 0; b < 4; b++) N[d & 1][b][lane] = U[b] + U2[b];
+      }
     }
-  }
-  if (fail >= 0 || Dinv == nullptr) return;
-
-  // ---- inverse of the factor (upper part of S is zero) ----
-  __syncthreads();
-  lower_inverse_inplace(S, n);
-  for (int idx = t; idx < DB * DB; idx += P_THREADS) {
-    const int i = idx % DB, k = idx / DB;
-    Dinv[idx] = (i >= k) ? S[i * LDS_LD + k] : 0.0;
+    lds_barrier();
+    const int fail = fail_sh;
+    if (fail >= 0) {
+      // as ATLAS leaves a failing block: columns left of the failing one
+      // done (as far as they got), the rest as it was
+      if (w == 0) {
+        const int bf = 4 * ((fail - c0) >> 2);
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+          if (4 * b < bf) store(c0 + ln, c0 + 4 * b + lk, row_d[c0 + 4 * b]);
+        if (t == 0) *dinfo = info_off + fail + 1;
+      }
+      return;
+    }
+    if (w > 0 && w < PTN) {  // (the last wave's tile is the inverse itself)
+      const double* y = &Y[d][lk * YLD + ln];
+      double p[4];
+#pragma unroll
+      for (int b = 0; b < 4; b++) p[b] = y[4 * b * YLD];
+      acc_t X = TM::op(p[0], T[0], zero), X2 = TM::op(p[1], T[1], zero);
+      X = TM::op(p[2], T[2], X);
+      X2 = TM::op(p[3], T[3], X2);
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        keep[b] = X[b] + X2[b];
+        S[(PT * rt + ln) * PLD + c0 + 4 * b + lk] = keep[b];
+      }
+    }
+    lds_barrier();
+    // results to memory, off the chain
+    if (w == PTN) {
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        store(c0 + ln, c0 + 4 * b + lk, row_d[c0 + 4 * b]);
+        keep[b] = Y[d][ln * YLD + 4 * b + lk];
+      }
+    }
+    if (w > 0) {
+      if (!inv) {
+#pragma unroll
+        for (int b = 0; b < 4; b++) store(PT * rt + ln, c0 + 4 * b + lk, keep[b]);
+      } else {  // inv(L)(i, c) = L^-T(c, i)
+        double* z = Dinv + c0 + lk + (size_t)(PT * rt + ln) * DB;
+#pragma unroll
+        for (int b = 0; b < 4; b++) z[4 * b] = keep[b];
+      }
+    }
+    if (w == 0 && d + 1 < PTN) {  // column d's product from the next diagonal tile
+      const double* row_n = row_d + PT * PLD + c0;
+      double p[4];
+      acc_t T2 = zero;
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        p[b] = row_n[4 * b];
+        T[b] = N[d & 1][b][lane];
+      }
+      T = TM::op(-p[0], p[0], T);
+      T2 = TM::op(-p[1], p[1], T2);
+      T = TM::op(-p[2], p[2], T);
+      T2 = TM::op(-p[3], p[3], T2);
+#pragma unroll
+      for (int b = 0; b < 4; b++) T[b] += T2[b];
+    }
   }
 }
 
@@ -254,7 +334,7 @@ void potrf_rec(hipStream_t s, bool lower, long N, double* A, long lda, int* dinf
                double* W) {
   if (N <= 0) return;
   if (N <= DB) {
-    hipLaunchKernelGGL(potf2_inv_kernel, dim3(1), dim3(P_THREADS), 0, s, (int)N, A, lda,
+    hipLaunchKernelGGL(potf2_inv_kernel, dim3(1), dim3(PW_THREADS), 0, s, (int)N, A, lda,
                        lower ? 1 : 0, dinfo, off, W + (size_t)(off / DB) * DB * DB);
     ATLG_LAUNCHED();
     return;

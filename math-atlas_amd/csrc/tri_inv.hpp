@@ -10,6 +10,15 @@ constexpr int kTriN = 128;          // largest block order
 constexpr int kTriLD = kTriN + 1;   // LDS pitch (elements) of a kTriN block
 constexpr int kTriThreads = 256;
 
+// A workgroup barrier that orders LDS accesses only: global stores (results
+// nobody in the launch reads back) stay in flight across it, where
+// __syncthreads would wait for each of them.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // One 16x16x4 matrix-core step per scalar type.  Lane l supplies A(l&15,
 // l>>4) and B(l>>4, l&15); register r of lane l receives D(row(l, r), l&15).
 template <class R>
