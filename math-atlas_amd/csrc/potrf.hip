@@ -24,15 +24,6 @@ namespace {
 
 constexpr int DB = kTrsmNB;    // diagonal block order
 
-// Broadcast of lane `src`'s value (uniform src) through the scalar unit.
-__device__ __forceinline__ double lane_value(double v, int src) {
-  const long long u = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane(static_cast<int>(u), src);
-  const int hi = __builtin_amdgcn_readlane(static_cast<int>(u >> 32), src);
-  return __longlong_as_double((static_cast<long long>(hi) << 32) |
-                              static_cast<unsigned int>(lo));
-}
-
 #ifndef ATLG_POTRF_RB
 #define ATLG_POTRF_RB 384
 #endif
@@ -168,7 +159,7 @@ potf2_inv_kernel(int n, double* __restrict__ A, long lda, int lower, int* __rest
 #pragma unroll
         for (int j = 0; j < 4; j++)
 #pragma unroll
-          for (int i = j; i < 4; i++) a[i][j] = lane_value(T[b], 16 * j + 4 * b + i);
+          for (int i = j; i < 4; i++) a[i][j] = tri_lane(T[b], 16 * j + 4 * b + i);
         bool pos = true;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -383,64 +374,51 @@ void potrf_rec(hipStream_t s, bool lower, long N, double* A, long lda, int* dinf
 #endif
 constexpr long kCholLaMin = 2048;
 
-// Look-ahead step width (ATLG_CHOL_STEP when set, a multiple of 128): the
-// chain of diagonal blocks (three 128-block leaves and a panel solve per 384
-// columns) is the longer path at small orders, the trailing SYRK at large
-// ones.  Measured on MI355X (ms, panels on 32 compute units, panel solves
-// moved to the update units where chol_solve_wide says): N=8192 128: 10.9,
-// 256: 11.3, 512: 12.5; N=12288 128: 24.2, 256: 21.3, 512: 22.6; N=16384
-// 128: 47.7, 256: 39.4, 384: 37.3, 512: 38.1 (before the move, 384: 39.8);
-// 48 or 64 panel units were slower at every order.
+// Look-ahead step width where `rem` columns are left (ATLG_CHOL_STEP when
+// set; multiples of 128): the chain of diagonal blocks is the longer path at
+// the end, the trailing SYRK, more efficient the deeper it is, before.
+// Measured on MI355X with one width throughout (ms, 28 us leaves): N=2048
+// 128: 1.07, 256: 1.06, 384: 1.11; N=4096 128: 2.38, 256: 2.18, 384: 2.21,
+// 512: 2.48; N=8192 128: 8.03, 256: 6.82, 384: 6.50, 512: 6.57; N=16384
+// 256: 33.6, 384: 30.8, 512: 30.4; 16 panel units instead of 32 the same, 64
+// 4-12% slower.
 #ifndef ATLG_CHOL_STEP
 #define ATLG_CHOL_STEP 0
 #endif
 // Widest block (columns) whose look-ahead update goes in two parts, the
 // diagonal block's triangle and then the rest of the block column: the leaf
-// starts after the first part.  N=8192 (128-column steps): 10.9 -> 10.3 ms;
-// for the 256/384-column steps of N=12288/16384 the split was 1 ms slower.
+// starts after the first part (N=4096 2.26 -> 2.18 ms, 8192 the same).
 #ifndef ATLG_CHOL_SPLIT_MAX
-#define ATLG_CHOL_SPLIT_MAX 128
+#define ATLG_CHOL_SPLIT_MAX 512
 #endif
-inline long chol_step(long N) {
+inline long chol_step(long rem) {
   if (ATLG_CHOL_STEP > 0) return ATLG_CHOL_STEP;
-  return N < 10240 ? 128 : (N < 14336 ? 256 : 384);
+  return rem < 4608 ? 256 : (rem < 12288 ? 384 : 512);
 }
 
 // Whether step k's panel solve (rest x nb1, after the diagonal block of nb1
 // columns) goes to the update side.  Per step, the update side runs the
-// block column's update and the trailing SYRK (U), the panel side the leaves
-// (P) and, when narrow, the solve on its ATLG_CHOL_PANEL_CUS units (Sn); a
-// wide solve (Sw) runs after U on the update side instead.  The step takes
-// max(U, P + Sn) narrow and max(U, P) + Sw wide, so the solve goes wide when
-// U < P + Sn - Sw: the test for blocks of at most ATLG_CHOL_MODEL2_MAX
-// columns, with 32 TFLOP/s for their 128-deep updates (measured at
-// N = 8192; 26 and 40 were slower).  Wider blocks keep the simpler test
-// T < P + Sn (T the trailing SYRK alone) with the 50 TFLOP/s found by a
-// sweep at N = 16384 (the full test measured the same there).
-#ifndef ATLG_CHOL_WIDE_SOLVE
-#define ATLG_CHOL_WIDE_SOLVE 1
-#endif
+// trailing SYRK (U, at ATLG_CHOL_UPD_TFLOPS), the panel side the leaves
+// (ATLG_CHOL_LEAF_US per 128 columns, with the small solves and updates
+// between them) and, when narrow, the solve on its ATLG_CHOL_PANEL_CUS units;
+// wide, it runs after U on the update side, whose units would else wait.
+// (N = 2048 .. 16384 within 2% for 30 to 100 us and 40 to 60 TFLOP/s.)
 #ifndef ATLG_CHOL_UPD_TFLOPS
 #define ATLG_CHOL_UPD_TFLOPS 50.0
 #endif
-#ifndef ATLG_CHOL_UPD128_TFLOPS
-#define ATLG_CHOL_UPD128_TFLOPS 32.0
-#endif
-#ifndef ATLG_CHOL_MODEL2_MAX
-#define ATLG_CHOL_MODEL2_MAX 128
+#ifndef ATLG_CHOL_LEAF_US
+#define ATLG_CHOL_LEAF_US 35.0
 #endif
 inline bool chol_solve_wide(long rest, long nb1) {
-  if (!ATLG_CHOL_WIDE_SOLVE || rest <= 0) return false;
-  const double upd_rate = (nb1 <= 128 ? ATLG_CHOL_UPD128_TFLOPS : ATLG_CHOL_UPD_TFLOPS) * 1e12,
+  if (rest <= 0) return false;
+  const double upd_rate = ATLG_CHOL_UPD_TFLOPS * 1e12,
                panel_rate = upd_rate * ATLG_CHOL_PANEL_CUS / (256.0 - ATLG_CHOL_PANEL_CUS);
   const double r = (double)rest, b = (double)nb1;
-  const double t_solve_n = 2.0 * r * b * b / panel_rate, t_solve_w = 2.0 * r * b * b / upd_rate;
-  if (nb1 > ATLG_CHOL_MODEL2_MAX) return r * r * b / upd_rate < b / 128.0 * 95e-6 + t_solve_n;
-  const double t_upd = r * r * b / upd_rate + 2.0 * r * b * b / upd_rate;
-  return t_upd < b / 128.0 * 95e-6 + t_solve_n - t_solve_w;
+  return r * r * b / upd_rate <
+         b / 128.0 * ATLG_CHOL_LEAF_US * 1e-6 + 2.0 * r * b * b / panel_rate;
 }
 
-// Right-looking Cholesky by chol_step(N)-column blocks with one step of
+// Right-looking Cholesky by chol_step()-column blocks with one step of
 // look-ahead:
 // while the caller's stream applies step k's SYRK to the columns right of
 // block k+1, the auxiliary stream factors block k+1 (updated first) and
@@ -505,12 +483,12 @@ void potrf_lookahead(hipStream_t s0, bool lower, long N, double* A, long lda, in
     update(s, k, kb, c0, nc, nc, 0);
   };
   hipEvent_t e_col = aux_event(4);
-  const long rb = chol_step(N);
-  const long kb0 = std::min(rb, N);
+  auto width = [&](long k) { return std::min(chol_step(N - k), N - k); };
+  const long kb0 = width(0);
   potrf_rec(s0, lower, kb0, A, lda, dinfo, 0, W);
   solve_panel(s0, 0, kb0, N - kb0);
-  for (long k0 = 0; k0 + kb0 < N; k0 += rb) {
-    const long kb = std::min(rb, N - k0), k1 = k0 + kb, nb1 = std::min(rb, N - k1);
+  for (long k0 = 0; k0 + width(k0) < N; k0 += width(k0)) {
+    const long kb = width(k0), k1 = k0 + kb, nb1 = width(k1);
     const long rest = N - k1 - nb1;
     // block k+1 first, then the rest of step k's update, beside which the
     // auxiliary stream factors block k+1 and solves its panel; for narrow

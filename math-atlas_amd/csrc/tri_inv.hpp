@@ -19,6 +19,15 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Broadcast of lane `src`'s value (uniform src) through the scalar unit.
+__device__ __forceinline__ double tri_lane(double v, int src) {
+  const long long u = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane(static_cast<int>(u), src);
+  const int hi = __builtin_amdgcn_readlane(static_cast<int>(u >> 32), src);
+  return __longlong_as_double((static_cast<long long>(hi) << 32) |
+                              static_cast<unsigned int>(lo));
+}
+
 // One 16x16x4 matrix-core step per scalar type.  Lane l supplies A(l&15,
 // l>>4) and B(l>>4, l&15); register r of lane l receives D(row(l, r), l&15).
 template <class R>

@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "atlg_internal.hpp"
 #include "tri_inv.hpp"
@@ -26,8 +27,6 @@ namespace atlg {
 namespace {
 
 constexpr int NB = kTrsmNB;    // diagonal block order (<= GEMM tile edge)
-constexpr int TRI_THREADS = kTriThreads;
-static_assert(NB == kTriN, "TRSM blocks are inverted by the 128-block inverter");
 
 // Element (i, j) of op(A).
 template <class S>
@@ -37,63 +36,146 @@ __device__ inline S opa(const S* A, long lda, bool trans, long i, long j) {
 
 // Inverts the diagonal blocks of op(A) (order na).  Block b covers rows and
 // columns [b*NB, b*NB + nbb).  An upper-triangular op(A) block U is handled
-// as the lower-triangular J U J (J = order reversal), so one in-place lower
-// inversion serves all cases.  Output: Dinv + b*NB*NB, column-major, ld NB,
-// zeros outside the triangle; Unit diagonals are never read.  NT is the
-// order held in LDS: NB for the general case; 32 or 64 when na <= NT (one
-// block), which then writes only the leading NT x NT part of the block (the
-// solves read the leading na x na part) and needs a fraction of the LDS, so
-// the launch fits beside GEMM workgroups on a busy device.
+// as the lower-triangular J U J (J = order reversal), so one lower inversion
+// serves all cases.  Output: Dinv + b*NB*NB, column-major, ld NB, zeros
+// outside the triangle; Unit diagonals are never read.  NT is the order held
+// in LDS: NB for the general case; 32 or 64 when na <= NT (one block), which
+// then writes only the leading NT x NT part of the block (the solves read the
+// leading na x na part) and needs a fraction of the LDS, so the launch fits
+// beside GEMM workgroups on a busy device.
+//
+// Latency-bound: one workgroup per block, a wave per row of 16x16 tiles.
+// Tiles are kept in the accumulator's layout (lane (n, k) = (l & 15, l >> 4)
+// holds row n, columns 4 b + k in register b), in which a register is also an
+// operand of the 16x16x4 MFMA.  The waves first invert the diagonal tiles,
+// four columns at a time, each its own, by carrying the identity to L^-T;
+// then each computes its row of L^-T tile by tile from its own results, the
+// tiles of L in LDS and the diagonal inverses, with no barrier between the
+// waves.  128-block 31 -> 11 us (8x8 register inverses and five doubling
+// levels with four barriers each before).
 template <class R, int NT>
-__global__ void __launch_bounds__(TRI_THREADS)
+__global__ void __launch_bounds__(4 * NT)
 trtri_diag_kernel(int na, const R* __restrict__ A, long lda, int trans, int lower, int unit,
                   R* __restrict__ Dinv, const int* __restrict__ skip) {
-  if (skip && *skip) return;
-  constexpr int LD = NT + 1;
-  __shared__ R S[NT * LD];
-  const int b = blockIdx.x, t = threadIdx.x;
-  const long o = (long)b * NB;
+  typedef TriMfma<R> M;
+  typedef typename M::acc_t acc_t;
+  constexpr int TS = 16, TN = NT / TS, LD = NT + 4, YLD = TS + 4;
+  constexpr int TILES = TN * (TN + 1) / 2, PER = (TILES + TN - 1) / TN;
+  __shared__ R S[NT * LD];        // L below and on the diagonal, L^-T above it
+  __shared__ R Y[TN][TS * YLD];   // diagonal tiles of L^-T
+  const int bk = blockIdx.x, t = threadIdx.x;
+  const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int ln = lane & 15, lk = lane >> 4;
+  // as an operand's row (a result's column), lane ln stands for column pm
+  const int pm = std::is_same<R, double>::value ? ln : 4 * (ln & 3) + (ln >> 2);
+  const acc_t zero = {0, 0, 0, 0};
+  const long o = (long)bk * NB;
   const int n = (int)min((long)NT, na - o);
   const bool tr = trans != 0;
-  // the fill goes in batches of 16 elements per thread whose loads are all
-  // issued before any of them is stored to LDS (one memory latency per
-  // batch instead of one per element)
-  constexpr int PER = NT * NT / TRI_THREADS, BATCH = PER < 16 ? PER : 16;
-  for (int b0 = 0; b0 < PER; b0 += BATCH) {
-    R v[BATCH];
+  const bool skipped = skip && *skip;
+  {
+    R v[PER][4];
 #pragma unroll
-    for (int u = 0; u < BATCH; u++) {
-      const int idx = t + (b0 + u) * TRI_THREADS;
-      const int i = idx % NT, j = idx / NT;
-      R x = R(0);
-      if (i >= j) {
-        if (i < n && j < n) {
-          if (i == j && unit) x = R(1);
-          else x = lower ? opa(A, lda, tr, o + i, o + j)
-                         : opa(A, lda, tr, o + n - 1 - i, o + n - 1 - j);
-        } else if (i == j) {
-          x = R(1);
-        }
+    for (int q = 0; q < PER; q++) {
+      int u = w + TN * q, ti = 0;
+      while (u > ti) u -= ++ti;
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        const int i = TS * ti + ln, j = TS * u + 4 * b + lk;
+        R x = i == j ? R(1) : R(0);
+        if (i >= j && i < n && !(i == j && unit))
+          x = lower ? opa(A, lda, tr, o + i, o + j) : opa(A, lda, tr, o + n - 1 - i, o + n - 1 - j);
+        v[q][b] = x;
       }
-      v[u] = x;
     }
+    if (skipped) return;
 #pragma unroll
-    for (int u = 0; u < BATCH; u++) {
-      const int idx = t + (b0 + u) * TRI_THREADS;
-      S[(idx % NT) * LD + idx / NT] = v[u];
+    for (int q = 0; q < PER; q++) {
+      int u = w + TN * q, ti = 0;
+      const bool in = u < TILES;
+      while (u > ti) u -= ++ti;
+      if (in) {
+#pragma unroll
+        for (int b = 0; b < 4; b++) S[(TS * ti + ln) * LD + TS * u + 4 * b + lk] = v[q][b];
+      }
     }
   }
-  __syncthreads();
-  lower_inverse_inplace<R, NT>(S, n);
-  R* D = Dinv + (size_t)b * NB * NB;
-  for (int idx = t; idx < NT * NT; idx += TRI_THREADS) {
+  R* D = Dinv + (size_t)bk * NB * NB;
+  for (int idx = t; idx < NT * NT; idx += 4 * NT) {
     const int i = idx % NT, j = idx / NT;
-    R v = R(0);
-    if (i < n && j < n) {
-      if (lower) v = (i >= j) ? S[i * LD + j] : R(0);
-      else v = (i <= j) ? S[(n - 1 - i) * LD + (n - 1 - j)] : R(0);
+    if (!(lower ? (i >= j && i < n) : (i <= j && j < n))) D[i + (size_t)j * NB] = R(0);
+  }
+  // inv(L)(i, j) to its place
+  auto put = [&](int i, int j, R x) {
+    if (i >= j && i < n) D[lower ? i + (size_t)j * NB : n - 1 - i + (size_t)(n - 1 - j) * NB] = x;
+  };
+  lds_barrier();
+  {  // the diagonal tile of this wave's row
+    const R* row = S + (TS * w + ln) * LD + TS * w + lk;
+    const R* rop = S + (TS * w + pm) * LD + TS * w + lk;
+    acc_t Z;
+#pragma unroll
+    for (int b = 0; b < 4; b++) Z[b] = ln == 4 * b + lk ? R(1) : R(0);
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+      const double x = (double)row[4 * b];
+      R a[4][4], wc[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int i = j; i < 4; i++) a[i][j] = (R)tri_lane(x, 16 * j + 4 * b + i);
+      // the 4x4 block's inverse: every lane solves for column lk and keeps
+      // the row its operand lane stands for
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        R sum = lk == i ? R(1) : R(0);
+#pragma unroll
+        for (int c = 0; c < i; c++) sum -= a[i][c] * wc[c];
+        wc[i] = sum * (R(1) / a[i][i]);
+      }
+      R wo = pm == 0 ? wc[0] : R(0);
+#pragma unroll
+      for (int i = 1; i < 4; i++) wo = pm == i ? wc[i] : wo;
+      const R z = M::op(wo, Z[b], zero)[0];
+      if (b < 3) Z = M::op(pm >= 4 * b + 4 ? -rop[4 * b] : R(0), z, Z);
+      Z[b] = z;
+      Y[w][ln * YLD + 4 * b + lk] = z;
+      put(TS * w + 4 * b + lk, TS * w + ln, z);
     }
-    D[i + (size_t)j * NB] = v;
+  }
+  lds_barrier();
+  // row w of L^-T: tile d = -(sum over e < d of its tile e times L(d, e)^T)
+  // times the inverse of diagonal tile d
+  R* mine = S + (TS * w + ln) * LD + lk;
+  for (int d = w + 1; d < TN; d++) {
+    const R* ld = S + (TS * d + pm) * LD + lk;
+    acc_t T = zero, T2 = zero;
+    for (int e = w; e < d; e++) {
+      const R* x2 = e == w ? &Y[w][ln * YLD + lk] : mine + TS * e;
+      R p[4], q[4];
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        p[b] = -ld[TS * e + 4 * b];
+        q[b] = x2[4 * b];
+      }
+      T = M::op(p[0], q[0], T);
+      T2 = M::op(p[1], q[1], T2);
+      T = M::op(p[2], q[2], T);
+      T2 = M::op(p[3], q[3], T2);
+    }
+    const R* y = &Y[d][lk * YLD + pm];
+    acc_t X = zero, X2 = zero;
+#pragma unroll
+    for (int b = 0; b < 4; b += 2) {
+      X = M::op(y[4 * b * YLD], T[b] + T2[b], X);
+      X2 = M::op(y[4 * (b + 1) * YLD], T[b + 1] + T2[b + 1], X2);
+    }
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+      const R x = X[b] + X2[b];
+      mine[TS * d + 4 * b] = x;
+      put(TS * d + 4 * b + lk, TS * w + ln, x);
+    }
   }
 }
 
@@ -400,13 +482,13 @@ void tri_inverse_blocks(hipStream_t s, long na, const S* A, long lda, int ta, in
   const long nblk = (na + NB - 1) / NB;
   const int trn = tr ? 1 : 0, low = (uplo == kLower) != tr ? 1 : 0, un = diag == kUnit ? 1 : 0;
   if (na <= 32)
-    hipLaunchKernelGGL((trtri_diag_kernel<S, 32>), dim3(1), dim3(TRI_THREADS), 0, s, (int)na, A,
+    hipLaunchKernelGGL((trtri_diag_kernel<S, 32>), dim3(1), dim3(4 * 32), 0, s, (int)na, A,
                        lda, trn, low, un, Dinv, skip);
   else if (na <= 64)
-    hipLaunchKernelGGL((trtri_diag_kernel<S, 64>), dim3(1), dim3(TRI_THREADS), 0, s, (int)na, A,
+    hipLaunchKernelGGL((trtri_diag_kernel<S, 64>), dim3(1), dim3(4 * 64), 0, s, (int)na, A,
                        lda, trn, low, un, Dinv, skip);
   else
-    hipLaunchKernelGGL((trtri_diag_kernel<S, NB>), dim3((unsigned)nblk), dim3(TRI_THREADS), 0, s,
+    hipLaunchKernelGGL((trtri_diag_kernel<S, NB>), dim3((unsigned)nblk), dim3(4 * NB), 0, s,
                        (int)na, A, lda, trn, low, un, Dinv, skip);
   ATLG_LAUNCHED();
 }
