@@ -64,13 +64,21 @@ hipStream_t aux_stream();
 constexpr int kAuxEvents = 8;
 hipEvent_t aux_event(int i);  // i = 0 .. kAuxEvents-1
 // A pair of streams restricted to disjoint compute units: *small gets the
-// first `cus` units, *large the rest (hipExtStreamCreateWithCUMask).  Made
-// once per device and unit count; false when cus <= 0 or the masked streams
-// are unavailable.
-bool split_streams(int cus, hipStream_t* small, hipStream_t* large);
+// first `cus` units, *large the rest (hipExtStreamCreateWithCUMask); false
+// when cus <= 0 or the masked streams are unavailable.  `caller` is the
+// stream that will wait for them: its first call makes pairs and times which
+// one its wait does not slow down (some 10 ms, synchronizing these streams;
+// under capture nothing is timed).  Called with aux_lock() held.
+bool split_streams(int cus, hipStream_t caller, hipStream_t* small, hipStream_t* large);
 // Compute units that work queued on the stream runs on: a split_streams()
 // stream's share, else the device's.
 int stream_units(hipStream_t s);
+// Whether ordinary launches on this stream may hold workgroups that wait for
+// each other on one XCD (at most 16 compute units of its 32).  Two such
+// launches at once always fit, more might each hold units the others need:
+// one stream per device gets the right, the first to ask, beside the
+// look-ahead's reserved units; others launch cooperatively or go without.
+bool gang_stream(hipStream_t s);
 // Held by a look-ahead driver while it queues work on the shared auxiliary
 // streams and events above, so that calls from several host threads do not
 // interleave their event records and waits (the device work of successive
@@ -105,7 +113,8 @@ enum Slot : int {
   kSlotTriFull = 21,    // dense zero-padded copy of a triangle (TRTRI, LAUUM, POTRI)
   kSlotTriTemp = 22,    // products of the doubling inverse
   kSlotAdjP = 23,       // the potrf adjoint's product matrix
-  kNumSlots = 24
+  kSlotGang = 24,       // exchange area of the one-XCD triangular solve
+  kNumSlots = 25
 };
 void* scratch(hipStream_t s, Slot slot, size_t bytes);
 

@@ -1424,6 +1424,7 @@ struct LU {
   int mb_g[2] = {0, 0};       // grid of each mailbox's last user (0: clean)
   XpBox* box = nullptr;       // exchange areas of the XCD panel
   int box_par = 0;            // the one its next multi-workgroup launch uses
+  bool gang = false;          // the stream may launch XCD panels without a cooperative launch
   int xcd_units = 32;         // compute units of one XCD the panel may count on
 };
 
@@ -1508,7 +1509,7 @@ void launch_xcd(LU<S>& f, int M, int w, int off, int G, int* lst) {
   if (G > 1) f.box_par ^= 1;
   const dim3 grid(8 * (G - 1) + 1), block(64 * ((per + 63) / 64));
   S* P = at(f, off, off);
-  if (G == 1 || !f.coop) {
+  if (G == 1 || !f.coop || f.gang) {
     hipLaunchKernelGGL(panel_xcd<S>, grid, block, 0, f.s, M, w, off, P, f.lda, f.ipiv, f.dinfo,
                        f.box, par, G, lst, f.status, f.limit);
     ATLG_LAUNCHED();
@@ -1516,7 +1517,9 @@ void launch_xcd(LU<S>& f, int M, int w, int off, int G, int* lst) {
   }
   // Outside the look-ahead's reserved units, panels of several callers'
   // streams could hold an XCD's units while each waits for more of its own
-  // workgroups: cooperative launches do not overlap each other.
+  // workgroups: cooperative launches do not overlap each other (they cost
+  // about 40 us each, N=1500: 7.2 against 5.0 ms, so the device's gang
+  // stream goes without).
   int p = par, g = G;
   long lda = f.lda;
   void* args[] = {&M,     &w, &off, &P, &lda,      &f.ipiv, &f.dinfo,
@@ -1830,8 +1833,12 @@ void getrf_lookahead(LU<S>& f0) {
   // caller's stream forks to the pair and joins at the end.
   hipStream_t caller = s0, sp = nullptr, sg = nullptr;
   const int panel_cus = la_panel_cus(f0.M);
-  const bool split = panel_cus > 0 && split_streams(panel_cus, &sp, &sg);
+  const bool split = panel_cus > 0 && split_streams(panel_cus, caller, &sp, &sg);
   if (split) {
+    // after the last look-ahead too, which may have run on another split:
+    // its panels and these would share compute units
+    ATLG_HIP(hipStreamWaitEvent(sg, aux_event(3), 0));
+    ATLG_HIP(hipStreamWaitEvent(sp, aux_event(3), 0));
     ATLG_HIP(hipEventRecord(aux_event(2), caller));
     ATLG_HIP(hipStreamWaitEvent(sg, aux_event(2), 0));
     ATLG_HIP(hipStreamWaitEvent(sp, aux_event(2), 0));
@@ -1965,6 +1972,7 @@ void getrf(hipStream_t s, long M, long N, S* A, long lda, int* ipiv, int* dinfo,
   if (M == 0 || N == 0) return;
   LU<S> f;
   init_lu(f, s, M, N, A, lda, ipiv, dinfo, gemm_prec);
+  f.gang = gang_stream(s);
   f.status = status_word(s);
   f.limit = wait_limit(kSpinLimit);
   if (ATLG_LU_LOOKAHEAD && std::min(M, N) >= kLaMin)

@@ -432,7 +432,8 @@ void potrf_lookahead(hipStream_t s0, bool lower, long N, double* A, long lda, in
   // with a CU-masked pair the 128-block leaves (132 KB of LDS) never wait
   // for a compute unit free of SYRK workgroups
   hipStream_t caller = s0, sp = nullptr, sg = nullptr;
-  const bool split = ATLG_CHOL_PANEL_CUS > 0 && split_streams(ATLG_CHOL_PANEL_CUS, &sp, &sg);
+  const bool split =
+      ATLG_CHOL_PANEL_CUS > 0 && split_streams(ATLG_CHOL_PANEL_CUS, caller, &sp, &sg);
   if (split) {
     ATLG_HIP(hipEventRecord(aux_event(2), caller));
     ATLG_HIP(hipStreamWaitEvent(sg, aux_event(2), 0));

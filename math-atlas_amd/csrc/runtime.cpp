@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <chrono>
 #include <climits>
 #include <cstdio>
 #include <cstdlib>
@@ -70,11 +71,16 @@ struct Aux {
   hipStream_t stream = nullptr;
   hipEvent_t ev[kAuxEvents] = {};
   // CU-masked pairs by the small side's unit count, created on first use
-  // ({nullptr, nullptr}: unavailable)
-  std::map<int, std::pair<hipStream_t, hipStream_t>> split;
+  // (none: unavailable), and the one chosen for each caller's stream
+  struct Split {
+    std::vector<std::pair<hipStream_t, hipStream_t>> pairs;
+    std::map<hipStream_t, int> choice;
+  };
+  std::map<int, Split> split;
 };
 std::map<int, Aux> g_aux;
 std::map<hipStream_t, int> g_units;  // CU-masked stream -> its compute units
+std::map<int, hipStream_t> g_gang;   // device -> the stream of gang_stream()
 Aux& aux_for_device() {
   int dev = 0;
   ATLG_HIP(hipGetDevice(&dev));
@@ -95,36 +101,121 @@ std::unique_lock<std::mutex> aux_lock() { return std::unique_lock<std::mutex>(g_
 hipStream_t aux_stream() { return aux_for_device().stream; }
 hipEvent_t aux_event(int i) { return aux_for_device().ev[(unsigned)i % kAuxEvents]; }
 
-bool split_streams(int cus, hipStream_t* small, hipStream_t* large) {
-  Aux& a = aux_for_device();
-  std::lock_guard<std::mutex> lk(g_mu);
-  auto it = a.split.find(cus);
-  if (it == a.split.end()) {
-    int dev = 0, total = 0;
-    ATLG_HIP(hipGetDevice(&dev));
-    ATLG_HIP(hipDeviceGetAttribute(&total, hipDeviceAttributeMultiprocessorCount, dev));
-    hipStream_t p[2] = {nullptr, nullptr};
-    if (cus > 0 && cus < total) {
-      const int words = (total + 31) / 32;
-      std::vector<uint32_t> m0(words, 0u), m1(words, 0u);
-      for (int c = 0; c < total; c++) (c < cus ? m0 : m1)[c / 32] |= 1u << (c % 32);
-      if (hipExtStreamCreateWithCUMask(&p[0], words, m0.data()) != hipSuccess ||
-          hipExtStreamCreateWithCUMask(&p[1], words, m1.data()) != hipSuccess) {
-        (void)hipGetLastError();
-        for (auto& st : p)
-          if (st) (void)hipStreamDestroy(st);
-        p[0] = p[1] = nullptr;
-      }
-    }
-    if (p[0]) {
-      g_units[p[0]] = cus;
-      g_units[p[1]] = total - cus;
-    }
-    it = a.split.emplace(cus, std::make_pair(p[0], p[1])).first;
+// ---- choice of a CU-masked pair -----------------------------------------
+//
+// Hardware queues share dispatch pipes.  While a look-ahead driver's streams
+// work, the caller's stream holds a waiting barrier, and a queue on the same
+// pipe then starts each kernel some 20 us later: DGETRF N=8192 takes 32 or 51
+// ms, N=16384 111 or 152, DPOTRF 8192 6.5 or 8.3, by nothing but the order in
+// which a process created its streams.  Which pipe a queue is on cannot be
+// asked, so it is timed, once per caller's stream: a chain of empty kernels
+// across the pair with the caller's stream waiting for it, against the same
+// chain without; a pair that slows down is passed over for a new one.
+namespace {
+constexpr int kProbeChain = 24;      // kernels on each stream of the pair
+constexpr int kMaxPairs = 4;         // pairs made per unit count
+constexpr double kProbeSlow = 1.35;  // waiting caller / free caller (seen: 1.07-1.14 or 1.60-1.68)
+
+__global__ void probe_empty() {}
+// Holds the stream for some 0.5 ms (a fixed count), so that the whole chain
+// and the caller's wait are queued before it starts.
+__global__ void probe_hold() {
+  for (int i = 0; i < 9000; i++) __builtin_amdgcn_s_sleep(2);
+}
+
+// Seconds from the first launch until the caller's stream is idle again.
+double probe(hipStream_t small, hipStream_t large, hipStream_t caller, const Aux& a, bool waiting) {
+  ATLG_HIP(hipStreamSynchronize(caller));
+  ATLG_HIP(hipStreamSynchronize(small));
+  ATLG_HIP(hipStreamSynchronize(large));
+  const auto t0 = std::chrono::steady_clock::now();
+  hipLaunchKernelGGL(probe_hold, dim3(1), dim3(64), 0, small);
+  for (int i = 0; i < kProbeChain; i++)
+    hipLaunchKernelGGL(probe_empty, dim3(1), dim3(64), 0, small);
+  ATLG_HIP(hipEventRecord(a.ev[0], small));
+  ATLG_HIP(hipStreamWaitEvent(large, a.ev[0], 0));
+  for (int i = 0; i < kProbeChain; i++)
+    hipLaunchKernelGGL(probe_empty, dim3(1), dim3(64), 0, large);
+  ATLG_LAUNCHED();
+  ATLG_HIP(hipEventRecord(a.ev[1], large));
+  if (waiting) {
+    ATLG_HIP(hipStreamWaitEvent(caller, a.ev[1], 0));
+    ATLG_HIP(hipStreamSynchronize(caller));
+  } else {
+    ATLG_HIP(hipStreamSynchronize(large));
   }
-  if (!it->second.first) return false;
-  *small = it->second.first;
-  *large = it->second.second;
+  return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+}
+
+bool make_pair(int cus, std::pair<hipStream_t, hipStream_t>* out) {
+  int dev = 0, total = 0;
+  ATLG_HIP(hipGetDevice(&dev));
+  ATLG_HIP(hipDeviceGetAttribute(&total, hipDeviceAttributeMultiprocessorCount, dev));
+  if (cus <= 0 || cus >= total) return false;
+  const int words = (total + 31) / 32;
+  std::vector<uint32_t> m0(words, 0u), m1(words, 0u);
+  for (int c = 0; c < total; c++) (c < cus ? m0 : m1)[c / 32] |= 1u << (c % 32);
+  hipStream_t p[2] = {nullptr, nullptr};
+  if (hipExtStreamCreateWithCUMask(&p[0], words, m0.data()) != hipSuccess ||
+      hipExtStreamCreateWithCUMask(&p[1], words, m1.data()) != hipSuccess) {
+    (void)hipGetLastError();
+    for (auto& st : p)
+      if (st) (void)hipStreamDestroy(st);
+    return false;
+  }
+  std::lock_guard<std::mutex> lk(g_mu);
+  g_units[p[0]] = cus;
+  g_units[p[1]] = total - cus;
+  *out = {p[0], p[1]};
+  return true;
+}
+}  // namespace
+
+bool split_streams(int cus, hipStream_t caller, hipStream_t* small, hipStream_t* large) {
+  Aux& a = aux_for_device();
+  Aux::Split& sp = a.split[cus];
+  if (sp.pairs.empty()) {
+    std::pair<hipStream_t, hipStream_t> p;
+    if (!make_pair(cus, &p)) return false;
+    sp.pairs.push_back(p);
+  }
+  int pick = 0;
+  auto it = sp.choice.find(caller);
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (it != sp.choice.end()) {
+    pick = it->second;
+  } else if (hipStreamIsCapturing(caller, &cap) == hipSuccess &&
+             cap == hipStreamCaptureStatusNone) {  // (an error: some other capture is open)
+    double best = 0.0;
+    for (int i = 0; i < kMaxPairs; i++) {
+      if (i == (int)sp.pairs.size()) {
+        std::pair<hipStream_t, hipStream_t> p;
+        if (!make_pair(cus, &p)) break;
+        sp.pairs.push_back(p);
+      }
+      const auto& p = sp.pairs[i];
+      // the first round also warms the streams up; the faster of two counts
+      double wait = 0.0, free = 0.0;
+      for (int r = 0; r < 3; r++) {
+        const double f = probe(p.first, p.second, caller, a, false);
+        const double w = probe(p.first, p.second, caller, a, true);
+        if (r == 1 || (r > 1 && f < free)) free = f;
+        if (r == 1 || (r > 1 && w < wait)) wait = w;
+      }
+      const double slow = wait / free;
+      if (i == 0 || slow < best) {
+        best = slow;
+        pick = i;
+      }
+      if (slow < kProbeSlow) break;
+    }
+    if (sp.choice.size() > 64) sp.choice.clear();  // streams come and go
+    sp.choice[caller] = pick;
+  } else {
+    (void)hipGetLastError();
+  }
+  *small = sp.pairs[pick].first;
+  *large = sp.pairs[pick].second;
   return true;
 }
 
@@ -144,6 +235,13 @@ int stream_units(hipStream_t s) {
     if (dev >= 0 && dev < kDevices) total[dev].store(n, std::memory_order_relaxed);
   }
   return n;
+}
+
+bool gang_stream(hipStream_t s) {
+  int dev = 0;
+  ATLG_HIP(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lk(g_mu);
+  return g_gang.emplace(dev, s).first->second == s;
 }
 
 void* scratch(hipStream_t s, Slot slot, size_t bytes) {
@@ -236,10 +334,11 @@ void teardown() {
   g_status.clear();
   for (auto& kv : g_aux) {
     Aux& a = kv.second;
-    for (auto& sp : a.split) {
-      if (sp.second.first) (void)hipStreamDestroy(sp.second.first);
-      if (sp.second.second) (void)hipStreamDestroy(sp.second.second);
-    }
+    for (auto& sp : a.split)
+      for (auto& p : sp.second.pairs) {
+        (void)hipStreamDestroy(p.first);
+        (void)hipStreamDestroy(p.second);
+      }
     a.split.clear();
     for (auto& e : a.ev)
       if (e) (void)hipEventDestroy(e);
