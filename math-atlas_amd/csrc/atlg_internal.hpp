@@ -104,7 +104,7 @@ enum Slot : int {
   kSlotBatchWork = 12,  // FP32 factors and right-hand sides of the mixed solver
   kSlotMixed = 13,      // FP32 factor, residual partials and norms of dsgesv
   kSlotBf16 = 14,       // BF16 operand copies of the low-precision update
-  kSlotTrsv = 15,       // ready flags of the few-RHS triangular solve
+  kSlotTrsv = 15,       // ready flags or exchange area of the few-RHS triangular solves
   kSlotLaLists = 16,    // per-leaf interchange lists of the look-ahead LU
   kSlotLaPerm = 17,     // row maps of the look-ahead LU's deferred interchanges
   kSlotLaTemp = 18,     // staging of one column block for those interchanges
@@ -113,10 +113,12 @@ enum Slot : int {
   kSlotTriFull = 21,    // dense zero-padded copy of a triangle (TRTRI, LAUUM, POTRI)
   kSlotTriTemp = 22,    // products of the doubling inverse
   kSlotAdjP = 23,       // the potrf adjoint's product matrix
-  kSlotGang = 24,       // exchange area of the one-XCD triangular solve
-  kNumSlots = 25
+  kNumSlots = 24
 };
 void* scratch(hipStream_t s, Slot slot, size_t bytes);
+// The same, or nullptr where that (or the stream's failure word) would have
+// to be allocated while the stream is being captured.
+void* scratch_in_capture(hipStream_t s, Slot slot, size_t bytes);
 
 // The stream's failure word: a device int that kernels whose bounded waits
 // give up OR their ATLG_FAIL_* bit into (zero otherwise).  Allocated and

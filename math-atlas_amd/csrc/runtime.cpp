@@ -273,6 +273,19 @@ void* scratch(hipStream_t s, Slot slot, size_t bytes) {
   return p;
 }
 
+void* scratch_in_capture(hipStream_t s, Slot slot, size_t bytes) {
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    auto it = g_slots.find(std::make_pair(s, static_cast<int>(slot)));
+    auto st = g_status.find(s);
+    if (it != g_slots.end() && it->second.bytes >= bytes && st != g_status.end() && st->second)
+      return it->second.p;
+  }
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+  return cap == hipStreamCaptureStatusNone ? scratch(s, slot, bytes) : nullptr;
+}
+
 int* status_word(hipStream_t s) {
   std::lock_guard<std::mutex> lk(g_mu);
   int*& w = g_status[s];

@@ -179,6 +179,17 @@ trtri_diag_kernel(int na, const R* __restrict__ A, long lda, int trans, int lowe
   }
 }
 
+constexpr long kSvSpin = 1L << 22;         // default polls (round trips) before giving up
+
+__device__ inline int ld_flag(const int* p) {
+  return __hip_atomic_load(const_cast<int*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void st_flag(int* p, int v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+#include "trsv_xcd.hpp"
+
 template <class S>
 struct Ctx {
   hipStream_t s;
@@ -191,6 +202,7 @@ struct Ctx {
   const S* Dinv;
   int dtrans;  // kTrans when Dinv holds the transposes of inv(op(A)_bb)
   const int* skip;
+  bool alloc;  // scratch memory may be used
 };
 
 // op(A)[i0:, j0:] as a GEMM operand: pointer and transpose flag.
@@ -227,6 +239,11 @@ void solve(const Ctx<S>& c, long r0, long n, S alpha) {
     }
     return;
   }
+  if (c.left && c.alloc && n <= kTxMaxN && c.N <= kTxRhs &&
+      trsv_one_launch<S>(c.s, c.lower_eff, c.trans, n, c.N, alpha, c.A + r0 + r0 * c.lda, c.lda,
+                         c.Dinv + (size_t)(r0 / NB) * NB * NB, c.dtrans == kTrans, c.B + r0, c.ldb,
+                         c.skip))
+    return;
   const long n1 = split(n), n2 = n - n1;
   const S* Ap;
   int ta;
@@ -269,9 +286,9 @@ void solve(const Ctx<S>& c, long r0, long n, S alpha) {
   }
 }
 
-// ---- few right-hand sides: one sync-free cooperative launch ----------------
+// ---- one right-hand side, long triangle: one sync-free cooperative launch ---
 //
-// op(A) = A (Left, NoTrans) with at most 4 right-hand sides.  The rows are cut
+// op(A) = A (Left, NoTrans).  The rows are cut
 // into 128-row blocks; workgroup w solves the blocks w, w+G, w+2G, ... in
 // solve order (top down for lower, bottom up for upper).  For its block it
 // accumulates A(block, q) x_q over the earlier blocks q as soon as each x_q
@@ -284,8 +301,12 @@ void solve(const Ctx<S>& c, long r0, long n, S alpha) {
 // agent-scope (coherence point) atomic loads and stores, as in getrf's
 // cooperative panel.
 constexpr int SV_T = 256;                  // threads: 2 per block row
-constexpr long kTrsvMin = 1024;            // shortest triangle that takes this path
-constexpr long kSvSpin = 1L << 22;         // default polls (round trips) before giving up
+// Shortest triangle that takes this path.  Against halving down to
+// trsv_xcd.hpp's launches, one right-hand side, op(A) = A: order 4096 178
+// against 168 us, 6000 238 against 268, 16384 734 against 830; with two
+// right-hand sides or op(A) = A^T the halving is the faster at every order
+// (8192: 378 against 406 and 390 against 648 us).
+constexpr long kTrsvMin = 4097;
 
 template <class S>
 __device__ inline S ld_co(const S* p);
@@ -310,12 +331,6 @@ __device__ inline void st_co(float* p, float x) {
   __hip_atomic_store(reinterpret_cast<unsigned*>(p), __float_as_uint(x), __ATOMIC_RELAXED,
                      __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ inline int ld_flag(const int* p) {
-  return __hip_atomic_load(const_cast<int*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline void st_flag(int* p, int v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 // Publication of a solved block.  Everything that crosses workgroups (the
 // solved x values and the flags) is accessed only with agent-scope atomic
 // loads and stores, which gfx950 performs coherently at the device level
@@ -333,42 +348,31 @@ __global__ void sv_reset(int* flags, int n) {
     flags[e] = 0;
 }
 
-template <class S, int R, bool TR>
+template <class S>
 __global__ void __launch_bounds__(SV_T)
 trsv_sf_kernel(int n, int nb, int upper, S alpha, const S* __restrict__ A, long lda,
-               const S* __restrict__ Dinv, S* __restrict__ B, long ldb, int* __restrict__ flags,
+               const S* __restrict__ Dinv, S* __restrict__ B, int* __restrict__ flags,
                int* __restrict__ err, int* __restrict__ status, long limit) {
-  __shared__ S part[2][NB][R];
-  __shared__ S xs[NB][R];
+  __shared__ S part[2][NB];
+  __shared__ S xs[NB];
   __shared__ int ok;
   const int t = threadIdx.x, r = t & (NB - 1), h = t >> 7;
   for (int li = blockIdx.x; li < nb; li += gridDim.x) {
     const int p = upper ? nb - 1 - li : li;
     const long r0 = (long)p * NB;
     const int rows = (int)min((long)NB, n - r0);
-    S acc[R];
-#pragma unroll
-    for (int k = 0; k < R; k++) acc[k] = S(0);
+    S acc = S(0);
     for (int lj = 0; lj < li; lj++) {
       const int q = upper ? nb - 1 - lj : lj;
       const long c0 = (long)q * NB;
       const int cols = (int)min((long)NB, n - c0);
       // this thread's 64 entries of op(A)(block p, block q): issued before
-      // the wait, they do not depend on x_q (TR: op(A) = A^T, the thread's
-      // entries are contiguous in A)
+      // the wait, they do not depend on x_q
       S va[64];
-      {
-        const int cend = (r < rows) ? min(64, cols - h * 64) : 0;
-        if (TR) {
-          const S* a = A + (c0 + h * 64) + (size_t)(r0 + r) * lda;
+      const int cend = (r < rows) ? min(64, cols - h * 64) : 0;
+      const S* a = A + (r0 + r) + (size_t)(c0 + h * 64) * lda;
 #pragma unroll
-          for (int c = 0; c < 64; c++) va[c] = (c < cend) ? a[c] : S(0);
-        } else {
-          const S* a = A + (r0 + r) + (size_t)(c0 + h * 64) * lda;
-#pragma unroll
-          for (int c = 0; c < 64; c++) va[c] = (c < cend) ? a[(size_t)c * lda] : S(0);
-        }
-      }
+      for (int c = 0; c < 64; c++) va[c] = (c < cend) ? a[(size_t)c * lda] : S(0);
       if (t == 0) {
         // one round trip per poll; the error word only every 256 polls
         bool good = true;
@@ -385,49 +389,30 @@ trsv_sf_kernel(int n, int nb, int upper, S alpha, const S* __restrict__ A, long 
       }
       __syncthreads();  // x_q is read (ld_co) only after the flag was seen
       if (!ok) return;  // same value in every thread
-      if (t < NB) {
-#pragma unroll
-        for (int k = 0; k < R; k++) xs[t][k] = (t < cols) ? ld_co(&B[c0 + t + (size_t)k * ldb]) : S(0);
-      }
+      if (t < NB) xs[t] = (t < cols) ? ld_co(&B[c0 + t]) : S(0);
       __syncthreads();
 #pragma unroll
-      for (int c = 0; c < 64; c++)
-#pragma unroll
-        for (int k = 0; k < R; k++) acc[k] += va[c] * xs[h * 64 + c][k];
+      for (int c = 0; c < 64; c++) acc += va[c] * xs[h * 64 + c];
       __syncthreads();
     }
-#pragma unroll
-    for (int k = 0; k < R; k++) part[h][r][k] = acc[k];
+    part[h][r] = acc;
     __syncthreads();
-    if (t < NB) {
-#pragma unroll
-      for (int k = 0; k < R; k++)
-        xs[t][k] = (t < rows) ? alpha * B[r0 + t + (size_t)k * ldb] - part[0][t][k] - part[1][t][k]
-                              : S(0);
-    }
+    if (t < NB) xs[t] = (t < rows) ? alpha * B[r0 + t] - part[0][t] - part[1][t] : S(0);
     __syncthreads();
     // x = inv(A_pp) (alpha b - acc): thread (r, h) sums 64 of the 128 columns
     const S* D = Dinv + (size_t)p * NB * NB + r + (size_t)h * 64 * NB;
-    S y[R];
-#pragma unroll
-    for (int k = 0; k < R; k++) y[k] = S(0);
+    S y = S(0);
 #pragma unroll
     for (int c0 = 0; c0 < 64; c0 += 16) {
       S d[16];
 #pragma unroll
       for (int c = 0; c < 16; c++) d[c] = D[(size_t)(c0 + c) * NB];
 #pragma unroll
-      for (int c = 0; c < 16; c++)
-#pragma unroll
-        for (int k = 0; k < R; k++) y[k] += d[c] * xs[h * 64 + c0 + c][k];
+      for (int c = 0; c < 16; c++) y += d[c] * xs[h * 64 + c0 + c];
     }
-#pragma unroll
-    for (int k = 0; k < R; k++) part[h][r][k] = y[k];
+    part[h][r] = y;
     __syncthreads();
-    if (t < rows) {
-#pragma unroll
-      for (int k = 0; k < R; k++) st_co(&B[r0 + t + (size_t)k * ldb], part[0][t][k] + part[1][t][k]);
-    }
+    if (t < rows) st_co(&B[r0 + t], part[0][t] + part[1][t]);
     // every thread's x stores are acknowledged before the barrier, and the
     // flag is stored after it
     __builtin_amdgcn_s_waitcnt(0);
@@ -436,13 +421,11 @@ trsv_sf_kernel(int n, int nb, int upper, S alpha, const S* __restrict__ A, long 
   }
 }
 
-// Few-RHS Left solve with op(A) = A (tr false) or A^T (tr true), `lower`
-// saying whether op(A) is lower triangular, and Dinv holding the inverses
-// of op(A)'s diagonal blocks; returns false when the shape is not handled.
+// Left solve with op(A) = A and one right-hand side, `lower` saying whether A
+// is lower triangular, and Dinv holding the inverses of A's diagonal blocks.
 template <class S>
-bool trsv_few(hipStream_t s, bool lower, bool tr, long n, long nrhs, S alpha, const S* A,
-              long lda, const S* Dinv, S* B, long ldb) {
-  if (nrhs < 1 || nrhs > 4) return false;
+void trsv_long(hipStream_t s, bool lower, long n, S alpha, const S* A, long lda, const S* Dinv,
+               S* B) {
   const int nb = (int)((n + NB - 1) / NB);
   int* flags = static_cast<int*>(scratch(s, kSlotTrsv, sizeof(int) * (nb + 64)));
   int* err = flags + nb;
@@ -456,20 +439,9 @@ bool trsv_few(hipStream_t s, bool lower, bool tr, long n, long nrhs, S alpha, co
   int G = std::max(1, std::min(nb, cus));
   int* status = status_word(s);
   long limit = wait_limit(kSvSpin);
-  void* args[] = {&nn, &nbk, &up, &alpha, &A, &lda, &Dinv, &B, &ldb, &flags, &err, &status, &limit};
-  const void* fn = nullptr;
-  switch (nrhs + (tr ? 4 : 0)) {
-    case 1: fn = reinterpret_cast<const void*>(&trsv_sf_kernel<S, 1, false>); break;
-    case 2: fn = reinterpret_cast<const void*>(&trsv_sf_kernel<S, 2, false>); break;
-    case 3: fn = reinterpret_cast<const void*>(&trsv_sf_kernel<S, 3, false>); break;
-    case 4: fn = reinterpret_cast<const void*>(&trsv_sf_kernel<S, 4, false>); break;
-    case 5: fn = reinterpret_cast<const void*>(&trsv_sf_kernel<S, 1, true>); break;
-    case 6: fn = reinterpret_cast<const void*>(&trsv_sf_kernel<S, 2, true>); break;
-    case 7: fn = reinterpret_cast<const void*>(&trsv_sf_kernel<S, 3, true>); break;
-    default: fn = reinterpret_cast<const void*>(&trsv_sf_kernel<S, 4, true>); break;
-  }
-  ATLG_HIP(hipLaunchCooperativeKernel(fn, dim3(G), dim3(SV_T), args, 0, s));
-  return true;
+  void* args[] = {&nn, &nbk, &up, &alpha, &A, &lda, &Dinv, &B, &flags, &err, &status, &limit};
+  ATLG_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&trsv_sf_kernel<S>), dim3(G),
+                                      dim3(SV_T), args, 0, s));
 }
 
 }  // namespace
@@ -513,22 +485,20 @@ void trsm(hipStream_t s, int side, int uplo, int ta, int diag, long M, long N, S
   c.M = M;
   c.N = N;
   c.skip = skip;
+  c.alloc = true;
   const long na = c.left ? M : N;
   c.dtrans = dinv ? (dinv_trans ? kTrans : kNoTrans) : kNoTrans;
   if (dinv) {
     c.Dinv = dinv;
-    if (c.left && !dinv_trans && !skip && na >= kTrsvMin &&
-        trsv_few<S>(s, c.lower_eff, c.trans, na, N, alpha, A, lda, dinv, B, ldb))
-      return;
   } else {
     const long nblk = (na + NB - 1) / NB;
     S* D = static_cast<S*>(scratch(s, kSlotTrsmInv, sizeof(S) * nblk * NB * NB));
     tri_inverse_blocks<S>(s, na, A, lda, ta, uplo, diag, D, skip);
     c.Dinv = D;
-    // a few right-hand sides on a long triangle: one sync-free launch
-    if (c.left && !skip && na >= kTrsvMin &&
-        trsv_few<S>(s, c.lower_eff, c.trans, na, N, alpha, A, lda, D, B, ldb))
-      return;
+  }
+  if (c.left && !c.trans && c.dtrans == kNoTrans && !skip && N == 1 && na >= kTrsvMin) {
+    trsv_long<S>(s, c.lower_eff, na, alpha, A, lda, c.Dinv, B);
+    return;
   }
   solve(c, 0, na, alpha);
 }
@@ -563,6 +533,7 @@ void trsm_noalloc(hipStream_t s, int side, int uplo, int ta, int diag, long M, l
   c.M = M;
   c.N = N;
   c.skip = nullptr;
+  c.alloc = false;
   c.Dinv = D;
   c.dtrans = kNoTrans;
   solve(c, 0, na, alpha);
