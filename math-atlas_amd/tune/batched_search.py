@@ -10,7 +10,7 @@ findNB, and the generated-header emitters such as atlas-mmcpy.base:3369):
   MFLOP being the rate in MFLOP/s, as in ATLAS's *.sum files) to
   tune/res/<rout>.sum; a later run reads the file and times only what is
   missing, so an interrupted search resumes;
-* the search is coarse first, then refined: block-column width per order
+* the search is coarse first, then refined: rows a wave takes at a time per order
   (16 versus 32 on a ladder of orders, then bisection between the last order
   where 16 wins and the first where 32 wins), then workgroups per compute
   unit on a sample of the uneven workload (a coarse ladder, then the
@@ -20,7 +20,7 @@ findNB, and the generated-header emitters such as atlas-mmcpy.base:3369):
   precision the workgroups per compute unit of the fastest uneven-sample
   line, and a decision tree on the system order (ATLAS's generated
   decision code of atlas-tlp.base:5126-5300 decides on problem size the
-  same way) whose leaves are the fastest block-column width on each
+  same way) whose leaves are the fastest row count on each
   interval between measured orders.
 
 Usage (on a machine with the GPU, the library built):
@@ -37,7 +37,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 sys.path.insert(0, PKG)
 
-BIG = 1 << 30  # t16_max that forces 16-wide block columns for every order
+BIG = 1 << 30  # t16_max that forces 16 rows a wave for every order
 ROUT = {"d": "dposv_batched", "s": "sposv_batched"}
 
 
@@ -162,7 +162,7 @@ def search(prec, res, samples, quick):
     nsys = 2 * cus  # one full wave of persistent workgroups, twice
     nrhs = 4
 
-    # -- stage 1: block-column width per order (coarse ladder) -------------
+    # -- stage 1: rows a wave takes at a time per order (coarse ladder) -------------
     ladder = [16, 32, 48, 64, 96, 128, 192, 256, 384, 512]
     if quick:
         ladder = [32, 64, 128, 256, 512]
@@ -244,7 +244,7 @@ def emit(path, res_dir, device=""):
         "// math-atlas_amd/tune/batched_search.py from its summary files",
         "// (math-atlas_amd/tune/res/*.sum)%s." % ((" measured on " + device) if device else ""),
         "// Per precision: persistent workgroups per compute unit, and the",
-        "// block-column width (16 or 32) as a decision tree on the system order.",
+        "// rows per wave (16 or 32) as a decision tree on the system order.",
         "#pragma once",
     ]
     for tag in ("d", "s"):
