@@ -239,10 +239,13 @@ void solve(const Ctx<S>& c, long r0, long n, S alpha) {
     }
     return;
   }
-  if (c.left && c.alloc && n <= kTxMaxN && c.N <= kTxRhs &&
-      trsv_one_launch<S>(c.s, c.lower_eff, c.trans, n, c.N, alpha, c.A + r0 + r0 * c.lda, c.lda,
-                         c.Dinv + (size_t)(r0 / NB) * NB * NB, c.dtrans == kTrans, c.B + r0, c.ldb,
-                         c.skip))
+  // X op(A) = B is op(A)^T X^T = B^T
+  const long rhs = c.left ? c.N : c.M;
+  if (c.alloc && n <= tx_order(rhs) &&
+      trsv_one_launch<S>(c.s, c.lower_eff == c.left, c.trans == c.left, n, rhs, alpha,
+                         c.A + r0 + r0 * c.lda, c.lda, c.Dinv + (size_t)(r0 / NB) * NB * NB,
+                         (c.dtrans == kTrans) == c.left, c.B + (c.left ? r0 : r0 * c.ldb),
+                         c.left ? 1 : c.ldb, c.left ? c.ldb : 1, c.skip))
     return;
   const long n1 = split(n), n2 = n - n1;
   const S* Ap;

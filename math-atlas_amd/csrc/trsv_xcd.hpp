@@ -1,5 +1,5 @@
-// Left triangular solve of order up to kTxMaxN with few right-hand sides in
-// one launch; included by trsm.hip.
+// Triangular solve with few right-hand sides in one launch; included by
+// trsm.hip.
 //
 // What bounds such a solve: a chain over the diagonal blocks.  The blocked
 // recursion pays two launches per 128-row block (order 1000: 16 launches,
@@ -27,11 +27,8 @@
 #pragma once
 
 constexpr int kTxB = 64;                    // rows per workgroup
-constexpr long kTxMaxN = 2048;              // order (longer ones: halved first, so that
-                                            // the whole device reads what lies off the blocks)
 constexpr int kTxCols = 16;                 // right-hand sides per group
-constexpr int kTxGroups = 8;                // groups, an XCD each
-constexpr long kTxRhs = kTxCols * kTxGroups;
+constexpr int kTxGroups = 8;                // groups side by side, an XCD each
 constexpr int kTxWaves = kTxB / 16;           // multiplying waves; as many fetch
 constexpr int kTxThreads = 2 * 64 * kTxWaves;
 constexpr int kTxLd = kTxCols + 1;          // LDS pitch of a block of right-hand sides
@@ -74,13 +71,13 @@ __device__ __forceinline__ int tx_lane_col(int ln) {
 
 template <class S, bool TR>
 __global__ void __launch_bounds__(kTxThreads)
-trsv_xcd(int n, int nb, int nrhs, int upper, S alpha, const S* __restrict__ A, long lda,
-         const S* __restrict__ Dinv, int dtrans, S* __restrict__ B, long ldb,
+trsv_xcd(int n, int nb, int nrhs, int gpad, int upper, S alpha, const S* __restrict__ A, long lda,
+         const S* __restrict__ Dinv, int dtrans, S* __restrict__ B, long bi, long bj,
          tx_word* __restrict__ xb, int* __restrict__ err, int* __restrict__ status, long limit,
          const int* __restrict__ skip) {
   typedef TriMfma<S> M;
   typedef typename M::acc_t acc_t;
-  const int grp = blockIdx.x & (kTxGroups - 1), li = blockIdx.x / kTxGroups;
+  const int grp = blockIdx.x % gpad, li = blockIdx.x / gpad;
   const int c0 = grp * kTxCols;  // the group's first right-hand side
   if (c0 >= nrhs || (skip && *skip)) return;
   const int nc = min(kTxCols, nrhs - c0);
@@ -148,7 +145,7 @@ trsv_xcd(int n, int nb, int nrhs, int upper, S alpha, const S* __restrict__ A, l
 #pragma unroll
   for (int r = 0; r < 4; r++) {
     const int c = M::row(lane, r);
-    rhs[r] = in && c < nc ? alpha * B[r0 + row + (size_t)(c0 + c) * ldb] : S(0);
+    rhs[r] = in && c < nc ? alpha * B[(r0 + row) * bi + (c0 + c) * bj] : S(0);
   }
   if (li > 1) load_a(a0, 0);
   if (li > 2) load_a(a1, 1);
@@ -226,18 +223,29 @@ trsv_xcd(int n, int nb, int nrhs, int upper, S alpha, const S* __restrict__ A, l
     if (c < nc) {
       __hip_atomic_store(out + c * kTxB, static_cast<tx_word>(__double_as_longlong((double)x)),
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (in) B[r0 + row + (size_t)(c0 + c) * ldb] = x;
+      if (in) B[(r0 + row) * bi + (c0 + c) * bj] = x;
     }
   }
 }
 
+// Largest order solved in one launch.  Up to 128 right-hand sides (a group per
+// XCD) 2048: longer triangles are halved first, so that the whole device
+// reads what lies off the diagonal blocks.  More groups take turns on a
+// compute unit and the products outweigh the chain: order 2500 with 200 / 500
+// / 1000 / 1701 right-hand sides takes 180 / 213 / 303 / 460 us with launches
+// up to order 1024, 220 / 251 / 334 / 492 up to 512 and 347 / 375 / 441 / 549
+// without; with 4000 they lose (914 against 836).
+inline long tx_order(long nrhs) {
+  return nrhs <= kTxCols * kTxGroups ? 2048 : nrhs <= 2048 ? 1024 : 0;
+}
+
 // Solves op(A) X = alpha B, op(A) lower (or upper) triangular of order n <=
-// kTxMaxN, nrhs <= kTxRhs; Dinv holds the inverses of op(A)'s NB x NB
-// diagonal blocks, or their transposes (dtrans).  False, with nothing queued,
+// tx_order(nrhs), element (i, j) of X and B at i bi + j bj; Dinv holds the inverses
+// of op(A)'s NB x NB diagonal blocks, or their transposes (dtrans).  False, with nothing queued,
 // where the exchange area cannot be had.
 template <class S>
 bool trsv_one_launch(hipStream_t s, bool lower, bool tr, long n, long nrhs, S alpha, const S* A,
-                     long lda, const S* Dinv, int dtrans, S* B, long ldb, const int* skip) {
+                     long lda, const S* Dinv, int dtrans, S* B, long bi, long bj, const int* skip) {
   const int nb = (int)((n + kTxB - 1) / kTxB);
   const int groups = (int)((nrhs + kTxCols - 1) / kTxCols);
   const long words = (long)groups * nb * kTxBlock;
@@ -249,16 +257,17 @@ bool trsv_one_launch(hipStream_t s, bool lower, bool tr, long n, long nrhs, S al
   hipLaunchKernelGGL(tx_reset, dim3((unsigned)std::min(256L, (words + 511) / 512)), dim3(512), 0,
                      s, xb, words, err);
   ATLG_LAUNCHED();
-  const dim3 grid(kTxGroups * (nb - 1) + groups), block(kTxThreads);
+  const int gpad = (groups + kTxGroups - 1) / kTxGroups * kTxGroups;
+  const dim3 grid(gpad * (nb - 1) + groups), block(kTxThreads);
   const int up = lower ? 0 : 1;
   int* status = status_word(s);
   const long limit = wait_limit(kSvSpin);
   if (tr)
-    hipLaunchKernelGGL((trsv_xcd<S, true>), grid, block, 0, s, (int)n, nb, (int)nrhs, up, alpha, A,
-                       lda, Dinv, dtrans, B, ldb, xb, err, status, limit, skip);
+    hipLaunchKernelGGL((trsv_xcd<S, true>), grid, block, 0, s, (int)n, nb, (int)nrhs, gpad, up, alpha, A,
+                       lda, Dinv, dtrans, B, bi, bj, xb, err, status, limit, skip);
   else
-    hipLaunchKernelGGL((trsv_xcd<S, false>), grid, block, 0, s, (int)n, nb, (int)nrhs, up, alpha, A,
-                       lda, Dinv, dtrans, B, ldb, xb, err, status, limit, skip);
+    hipLaunchKernelGGL((trsv_xcd<S, false>), grid, block, 0, s, (int)n, nb, (int)nrhs, gpad, up, alpha, A,
+                       lda, Dinv, dtrans, B, bi, bj, xb, err, status, limit, skip);
   ATLG_LAUNCHED();
   return true;
 }

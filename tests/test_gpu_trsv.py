@@ -1,7 +1,7 @@
-"""Left triangular solves with few right-hand sides (one launch up to order
-2048, halves above; one right-hand side above 4096 by the sync-free launch):
+"""Triangular solves with few right-hand sides (one launch up to order 2048 or
+1024, halves above; one right-hand side above 4096 by the sync-free launch):
 orders around the 64-row blocks and the 128-row inverses, right-hand sides
-around the 16-column groups, every triangle, transpose and diagonal.
+around the 16-column groups, every side, triangle, transpose and diagonal.
 
 Accepted residual: with op(A)'s diagonal in [1, 2] and the sum of a row's
 other entries at most 1/2 in magnitude, a solve through inverted blocks errs
@@ -47,7 +47,8 @@ def close(n, t, x, b, alpha):
 @pytest.mark.parametrize("uplo", [O.Lower, O.Upper])
 @pytest.mark.parametrize("trans", [O.NoTrans, O.Trans])
 @pytest.mark.parametrize("n,k", [(129, 1), (191, 16), (192, 17), (193, 3), (256, 128), (257, 129),
-                                 (500, 5), (1000, 33), (2047, 2), (2048, 1), (2049, 1), (4097, 1)])
+                                 (500, 5), (1000, 33), (2047, 2), (2048, 1), (2049, 1), (4097, 1),
+                                 (1024, 250), (1025, 300), (300, 2048), (200, 2049)])
 def test_few_rhs(G, uplo, trans, n, k):
     a, b = system(n, k, n + k)
     for diag, alpha in ((O.NonUnit, 1.0), (O.Unit, -0.7)):
@@ -56,6 +57,21 @@ def test_few_rhs(G, uplo, trans, n, k):
         x = G.to_fortran(db)
         assert np.array_equal(x[n:], b[n:])
         assert close(n, op(a, n, uplo, trans, diag), x[:n], b[:n], alpha)
+
+
+@pytest.mark.parametrize("uplo", [O.Lower, O.Upper])
+@pytest.mark.parametrize("trans", [O.NoTrans, O.Trans])
+@pytest.mark.parametrize("n,k", [(129, 1), (192, 17), (500, 5), (1000, 200), (2049, 3)])
+def test_right(G, uplo, trans, n, k):
+    # X op(A) = alpha B is op(A)^T X^T = alpha B^T
+    a, b = system(n, k, n + k)
+    b = np.asfortranarray(b.T)
+    for diag, alpha in ((O.NonUnit, 1.0), (O.Unit, -0.7)):
+        da, db = G.from_fortran(a), G.from_fortran(b)
+        G.dtrsm(G.Right, uplo, trans, diag, k, n, alpha, da, n + 1, db, k, check=True)
+        x = G.to_fortran(db)
+        assert np.array_equal(x[:, n:], b[:, n:])
+        assert close(n, op(a, n, uplo, trans, diag).T, x[:, :n].T, b[:, :n].T, alpha)
 
 
 def test_not_finite(G):
