@@ -190,7 +190,11 @@ put_tri_blocks_kernel(int na, double* __restrict__ A, long lda, int lower, int u
 // up to 32, leading dimension np) as a lower triangle with zeros everywhere
 // else (an upper triangle is transposed in), so that the products below can
 // take whole tiles: TRTRI by doubling, LAUUM as one triangle-masked product.
-constexpr long kTriFullMin = 2 * NB;                  // smallest order that uses them
+// Smallest orders that use them.  TRTRI of one block is that block's inverse
+// (order 128: 44 us against 55, 129: 61 against 63); LAUUM and POTRI take the
+// product from order 48 (POTRI 47 against 39 us; 128: 205 against 58, 255:
+// 480 against 72).
+constexpr long kTriFullMin = NB + 1, kLauumFullMin = 48;
 constexpr size_t kTriFullCap = size_t(4) << 30;       // largest dense copy (bytes)
 constexpr int kCT = 32;                               // copy tile
 
@@ -356,9 +360,9 @@ void trtri_rec(hipStream_t s, bool lower, int diag, long off, long N, double* A0
 
 long tri_full_order(long n) { return (n + kCT - 1) / kCT * kCT; }
 
-static bool tri_full_fits(long n) {
+static bool tri_full_fits(long n, long least) {
   const long np = tri_full_order(n);
-  return n >= kTriFullMin && (size_t)np * np * sizeof(double) <= kTriFullCap;
+  return n >= least && (size_t)np * np * sizeof(double) <= kTriFullCap;
 }
 
 void tri_copy_to(hipStream_t s, bool lower, bool unit, long n, const double* A, long lda,
@@ -375,7 +379,7 @@ void tri_copy_to(hipStream_t s, bool lower, bool unit, long n, const double* A, 
 // 4NB, ... with halves already inverted, X21 <- -X22 (X21 X11).  The full
 // blocks of a level go in one batched launch per product, each product
 // restricted to the K range its triangular operand can reach; a ragged
-// last block takes two ordinary products (its zero padding keeps them exact).
+// last block takes the same two products with its rows padded by zeros.
 void tri_invert_full(hipStream_t s, int diag, long n, double* X, long np, const int* skip) {
   const long nblk = (n + NB - 1) / NB;
   double* D = static_cast<double*>(scratch(s, kSlotTrsmInv, sizeof(double) * nblk * NB * NB));
@@ -400,10 +404,13 @@ void tri_invert_full(hipStream_t s, int diag, long n, double* X, long np, const 
     }
     const long o = nfull * sz, r = n - o - h;
     if (r > 0) {
-      gemm<double>(s, kNoTrans, kNoTrans, r, h, h, 1.0, X + o + h + o * np, np, X + o + o * np, np,
-                   0.0, T, h, 0, skip);
-      gemm<double>(s, kNoTrans, kNoTrans, r, h, r, -1.0, X + (o + h) + (o + h) * np, np, T, h, 0.0,
-                   X + o + h + o * np, np, 0, skip);
+      // the same with the last block's rows, zero padded to np
+      const long rp = np - o - h;
+      if (!gemm_batched(s, kNoTrans, kNoTrans, rp, h, h, 1.0, X + o + h + o * np, np, 0,
+                        X + o + o * np, np, 0, 0.0, T, h, 0, 1, 0, 1, skip) ||
+          !gemm_batched(s, kNoTrans, kNoTrans, r, h, rp, -1.0, X + (o + h) * (np + 1), np, 0, T, h,
+                        0, 0.0, X + o + h + o * np, np, 0, 1, 0, 4, skip))
+        throw HipFailure{"trtri: the last block's product does not apply"};
     }
   }
 }
@@ -481,7 +488,7 @@ void trtri(hipStream_t s, int uplo, int diag, long N, double* A, long lda, int* 
     hipLaunchKernelGGL(diag_zero_kernel, dim3(1), dim3(256), 0, s, (int)N, A, lda, dinfo);
     ATLG_LAUNCHED();
   }
-  if (tri_full_fits(N)) {
+  if (tri_full_fits(N, kTriFullMin)) {
     const long np = tri_full_order(N);
     double* X = tri_copy_in(s, lower, diag == kUnit, N, A, lda, dinfo);
     tri_invert_full(s, diag, N, X, np, dinfo);
@@ -503,7 +510,7 @@ void trtri(hipStream_t s, int uplo, int diag, long N, double* A, long lda, int* 
 void lauum(hipStream_t s, int uplo, long N, double* A, long lda, const int* skip) {
   if (N <= 0) return;
   const bool lower = uplo == kLower;
-  if (tri_full_fits(N)) {
+  if (tri_full_fits(N, kLauumFullMin)) {
     const double* X = tri_copy_in(s, lower, false, N, A, lda, skip);
     lauum_from_full(s, lower, N, X, tri_full_order(N), A, lda, skip);
     return;
@@ -514,7 +521,7 @@ void lauum(hipStream_t s, int uplo, long N, double* A, long lda, const int* skip
 // clapack_dpotri (atlas-clp.base:316-362): trtri, then lauum only when the
 // factor had no zero on its diagonal (the device info word skips it).
 void potri(hipStream_t s, int uplo, long N, double* A, long lda, int* dinfo) {
-  if (N > 0 && tri_full_fits(N)) {
+  if (N > 0 && tri_full_fits(N, kLauumFullMin)) {
     // the inverse stays in the dense copy, from which the product reads
     const bool lower = uplo == kLower;
     set_int(s, dinfo, 0);

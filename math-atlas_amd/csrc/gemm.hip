@@ -147,10 +147,10 @@ struct TileLoader {
 // one XCD (hardware deals ids round-robin over the 8 XCDs) cover a compact
 // block of tiles, sharing A row panels and B column panels in that XCD's L2.
 __device__ inline void tile_of(int bid, int nblk, int tilesM, int tilesN, int& tm,
-                               int& tn, bool compact = true) {
+                               int& tn) {
   const int per = nblk / 8, rem = nblk % 8;
   const int xcd = bid % 8, local = bid / 8;
-  const int id = (!ATLG_GEMM_XCD || !compact) ? bid
+  const int id = !ATLG_GEMM_XCD ? bid
                  : (xcd < rem) ? xcd * (per + 1) + local
                                : rem * (per + 1) + (xcd - rem) * per + local;
   constexpr int GM = ATLG_GEMM_GM;  // tile rows per group
@@ -192,6 +192,22 @@ __device__ inline void tri_tile_of(int id, int mode, int tilesM, int tilesN, int
   } else {
     tn = a;
     tm = b;
+  }
+}
+
+// Tiles of a product whose K range depends on the tile (ktrim, see
+// gemm_rega_f64), longest ranges first.
+__device__ inline void trim_tile_of(int id, int mode, int ktrim, int tilesM, int tilesN, int& tm,
+                                    int& tn) {
+  if (mode != 0) {  // k >= row and column: row by row (mode 2: column by column)
+    tri_tile_of(id, mode, tilesM, tilesN, tm, tn);
+  } else if (ktrim & 1) {  // k >= n0
+    tn = id / tilesM;
+    tm = id - tn * tilesM;
+  } else {  // k >= m0, or k < m0 + BM
+    tm = id / tilesN;
+    tn = id - tm * tilesN;
+    if (ktrim & 4) tm = tilesM - 1 - tm;
   }
 }
 
@@ -388,26 +404,37 @@ __device__ __forceinline__ void gemm_rega_f64(int M, int N, int K, double alpha,
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm0 = (wave >> 1) * WM, wn0 = (wave & 1) * WN;
   const int fx = lane & 15, fk = lane >> 4;
-  if (XT) {  // batch member blockIdx.y: operands at fixed element strides
-    A += (size_t)blockIdx.y * sa;
-    B += (size_t)blockIdx.y * sb;
-    C += (size_t)blockIdx.y * sc;
-  }
   // With K-trimmed tiles the work per tile follows its row or column, and
   // the XCD-compact order (each XCD a contiguous range of tiles) would give
-  // one XCD all the long ones: those keep the dispatch order, which deals
-  // consecutive tiles to the XCDs in turn.
+  // one XCD all the long ones: those go longest first in dispatch order,
+  // which deals consecutive tiles to the XCDs in turn, the members of a batch
+  // interleaved, so that a compute unit's second tile is a short one (POTRI of
+  // order 8192: 6.9 -> 6.2 ms).
   const bool compact = !(XT && ktrim != 0);
-  for (int bid = blockIdx.x; bid < ntiles; bid += gridDim.x) {
+  int bid0 = blockIdx.x;
+  if (XT) {  // a batch member's operands lie at fixed element strides
+    unsigned member = blockIdx.y;
+    if (!compact) {
+      const unsigned id = blockIdx.y * gridDim.x + blockIdx.x;
+      member = id % gridDim.y;
+      bid0 = id / gridDim.y;
+    }
+    A += (size_t)member * sa;
+    B += (size_t)member * sb;
+    C += (size_t)member * sc;
+  }
+  for (int bid = bid0; bid < ntiles; bid += gridDim.x) {
     int tm, tn;
-    if (mode == 0) {
-      tile_of(bid, ntiles, tilesM, tilesN, tm, tn, compact);
+    if (!compact) {
+      trim_tile_of(bid, mode, ktrim, tilesM, tilesN, tm, tn);
+    } else if (mode == 0) {
+      tile_of(bid, ntiles, tilesM, tilesN, tm, tn);
     } else {
       const int per = ntiles / 8, rem = ntiles % 8, xcd = bid % 8, local = bid / 8;
-      const int id = (!ATLG_GEMM_XCD || !compact) ? bid
+      const int id = !ATLG_GEMM_XCD ? bid
                      : (xcd < rem) ? xcd * (per + 1) + local
                                    : rem * (per + 1) + (xcd - rem) * per + local;
-      if (ATLG_GEMM_TRI_GROUPED && compact) tri_tile_grouped(id, mode, tilesM, tilesN, tm, tn);
+      if (ATLG_GEMM_TRI_GROUPED) tri_tile_grouped(id, mode, tilesM, tilesN, tm, tn);
       else tri_tile_of(id, mode, tilesM, tilesN, tm, tn);
     }
     const int m0 = tm * BM, n0 = tn * BN;
@@ -702,7 +729,8 @@ struct GwCost {
   double launch, fixed, per_k;
 };
 template <class S>
-GwForm gw_form(long M, long N, long K, int mode, bool at, bool reg_a, int units) {
+GwForm gw_form(long M, long N, long K, int mode, bool at, bool reg_a, int units, int batch = 1,
+               double mean = 1.0) {
   const bool dbl = std::is_same<S, double>::value;
   // A transposed: k-contiguous loads touch more lines per instruction
   const double tr = at ? 1.12 : 1.0;
@@ -711,13 +739,17 @@ GwForm gw_form(long M, long N, long K, int mode, bool at, bool reg_a, int units)
   const GwCost c32 = {6.0, 0.8, (dbl ? 0.0092 : 0.0046) * tr};
   auto time = [&](const GwCost& c, long T) {
     const long tm = (M + T - 1) / T, tn = (N + T - 1) / T;
-    const double tiles = mode == 0 ? (double)tm * tn : (double)tri_tiles(mode, (int)tm, (int)tn);
-    return c.launch + std::ceil(tiles / units) * (c.fixed + c.per_k * (double)K);
+    const double tiles =
+        batch * (mode == 0 ? (double)tm * tn : (double)tri_tiles(mode, (int)tm, (int)tn));
+    return c.launch + std::max(1.0, mean * std::ceil(tiles / units)) * (c.fixed + c.per_k * (double)K);
   };
   const double t128 = time(c128, BM), t64 = time(c64, 2 * GW_T), t32 = time(c32, GW_T);
   if (t128 <= t64 && t128 <= t32) return kGwNone;
   return t64 <= t32 ? kGw64 : kGw32x4;
 }
+
+// (mean: a tile's average share of K, where triangular operands trim it; the
+// longest tile has all of it.)
 
 // Launches gemm_wave.  kGwLeft / kGwRight: one workgroup owns all of a short
 // side of at most 128 (four waves) and 32 of the long one and reads all of
@@ -735,7 +767,7 @@ void launch_gw(hipStream_t s, GwForm form, long M, long N, long K, S alpha, cons
     const int nt_ = mode == 0 || WM_ != WN_ ? tm_ * tn_ : tri_tiles(mode, tm_, tn_);          \
     hipLaunchKernelGGL((gemm_wave<S, AT, BT, WM_, WN_, WS_>), dim3((unsigned)nt_),            \
                        dim3(64 * WM_ * WN_ * WS_), 0, s, (int)M, (int)N, (int)K, alpha, A,    \
-                       lda, B, ldb, beta, C, ldc, mode, skip);                                \
+                       lda, B, ldb, beta, C, ldc, mode, skip, 0L, 0L, 0L, 0);                 \
   } while (0)
   switch (form) {
     case kGw64: ATLG_GO(2, 2, 1); break;
@@ -880,6 +912,25 @@ bool gemm_batched(hipStream_t s, int TA, int TB, long M, long N, long K, double 
   if (((ktrim & 1) && N > K) || ((ktrim & 2) && M > K) || ((ktrim & 4) && (ktrim & 2)) ||
       ((ktrim & 4) && (ktrim & 1) && mode != 1))
     return false;
+  // as gemm() chooses, for products that leave the device idle (POTRI of
+  // order 1000: 378 -> 153 us, 2048: 870 -> 294, 8192: 6.2 -> 5.9 ms)
+  if (!bt && C != A && C != B && 8L * GW_T * std::max(lda, ldb) < (1L << 31)) {
+    const GwForm f =
+        gw_form<double>(M, N, K, mode, at, true, stream_units(s), batch, ktrim ? 0.55 : 1.0);
+    if (f != kGwNone) {
+      const int T = f == kGw64 ? 2 * GW_T : GW_T;
+      const int tm = (int)((M + T - 1) / T), tn = (int)((N + T - 1) / T);
+      const dim3 g(mode == 0 ? tm * tn : tri_tiles(mode, tm, tn), (unsigned)batch);
+      const auto fn = f == kGw64 ? (at ? gemm_wave<double, true, false, 2, 2, 1, true>
+                                       : gemm_wave<double, false, false, 2, 2, 1, true>)
+                                 : (at ? gemm_wave<double, true, false, 1, 1, 4, true>
+                                       : gemm_wave<double, false, false, 1, 1, 4, true>);
+      hipLaunchKernelGGL(fn, g, dim3(256), 0, s, (int)M, (int)N, (int)K, alpha, A, lda, B, ldb,
+                         beta, C, ldc, mode, skip, sa, sb, sc, ktrim);
+      ATLG_LAUNCHED();
+      return true;
+    }
+  }
   const long tilesM = (M + BM - 1) / BM, tilesN = (N + BN - 1) / BN;
   const long nwg = mode == 0 ? tilesM * tilesN : tri_tiles(mode, (int)tilesM, (int)tilesN);
   const int vecc = aligned16<double>(C, ldc) ? 1 : 0;

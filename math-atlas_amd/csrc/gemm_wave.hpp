@@ -87,17 +87,26 @@ struct GwOperand {
   }
 };
 
-template <class S, bool AT, bool BT, int WM, int WN, int WS>
+// XT: batch members blockIdx.y at strides sa, sb, sc, K ranges trimmed by
+// ktrim, K a multiple of GW_K; the tiles in gemm_rega_f64's order.
+template <class S, bool AT, bool BT, int WM, int WN, int WS, bool XT = false>
 __global__ void __launch_bounds__(64 * WM * WN * WS)
 gemm_wave(int M, int N, int K, S alpha, const S* A, long lda, const S* B, long ldb, S beta,
-          S* C, long ldc, int mode,
-          const int* __restrict__ skip) {
+          S* C, long ldc, int mode, const int* __restrict__ skip, long sa, long sb, long sc,
+          int ktrim) {
   typedef Mfma<S> MF;
   constexpr int TM_ = GW_T * WM, TN_ = GW_T * WN, NW = WM * WN;
   if (skip && *skip) return;
   __shared__ S part[WS > 1 ? WS * NW * 16 * 64 : 1];
   const int tilesM = (M + TM_ - 1) / TM_, tilesN = (N + TN_ - 1) / TN_;
   int tm, tn;
+  if (XT) {
+    const unsigned id = blockIdx.y * gridDim.x + blockIdx.x, member = id % gridDim.y;
+    trim_tile_of(id / gridDim.y, mode, ktrim, tilesM, tilesN, tm, tn);
+    A += (size_t)member * sa;
+    B += (size_t)member * sb;
+    C += (size_t)member * sc;
+  } else
   // (the triangle's enumeration needs square tiles; others drop what lies
   // outside it wave by wave)
   if (WM != WN || mode == 0) tile_of(blockIdx.x, gridDim.x, tilesM, tilesN, tm, tn);
@@ -120,8 +129,15 @@ gemm_wave(int M, int N, int K, S alpha, const S* A, long lda, const S* B, long l
     GwOperand<S, BT> ob;
     oa.init(A, lda, m0, M, fx, fk);
     ob.init(B, ldb, n0, N, fx, fk);
-    const int nch = (K + GW_K - 1) / GW_K, full = K / GW_K;
-    const int c0 = (int)((long)nch * sl / WS), c1 = (int)((long)nch * (sl + 1) / WS);
+    const int full = K / GW_K;
+    int nch = (K + GW_K - 1) / GW_K, cb = 0;  // chunks, and the first
+    if (XT) {
+      if (ktrim & 1) cb = n0 / GW_K;
+      if (ktrim & 2) cb = max(cb, m0 / GW_K);
+      if (ktrim & 4) nch = min(nch, (m0 + GW_T) / GW_K);
+      nch = max(0, nch - cb);
+    }
+    const int c0 = cb + (int)((long)nch * sl / WS), c1 = cb + (int)((long)nch * (sl + 1) / WS);
     const int ce = min(c1, full);  // whole chunks [c0, ce)
     S a[2][4][2], b[2][4][2];
     auto mma = [&](int d) {

@@ -1,0 +1,89 @@
+"""Triangular inverse, LAUUM and POTRI at the orders where their products
+change form: one 128-row block, the dense copy's smallest orders, ragged last
+blocks, levels of several blocks in one launch (FP64).
+
+Accepted: residuals of 4 n eps, the sums of n terms of each product, relative
+to the norms of the factors they are taken over (largest row sums)."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+EPS = 2.0 ** -53
+SIZES = [1, 33, 47, 48, 64, 127, 128, 129, 160, 255, 256, 257, 385, 511, 640, 777, 1024, 1055, 1300, 2049]
+
+
+@pytest.fixture(scope="module")
+def G():
+    import torch
+    assert torch.cuda.is_available()
+    import atlas_gpu
+    return atlas_gpu
+
+
+def norm(a):
+    return np.abs(a).sum(1).max()
+
+
+def triangle(n, uplo):
+    """A triangle with diagonal in [1, 2], a marker in the other one, padding."""
+    rng = np.random.default_rng(n)
+    a = rng.uniform(-1, 1, (n + 3, n)) / n
+    a[np.arange(n), np.arange(n)] = rng.uniform(1, 2, n)
+    other = np.triu_indices(n, 1) if uplo == O.Lower else np.tril_indices(n, -1)
+    a[:n][other] = 9.0
+    return np.asfortranarray(a), other
+
+
+def run(G, f, a, *args):
+    import torch
+    d = G.from_fortran(a)
+    info = torch.full((1,), -7, dtype=torch.int32, device="cuda")
+    f(*args, a.shape[1], d, a.shape[0], *(() if f is G.dlauum else (info,)))
+    assert f is G.dlauum or int(info.item()) == 0
+    return G.to_fortran(d)
+
+
+@pytest.mark.parametrize("uplo", [O.Lower, O.Upper])
+@pytest.mark.parametrize("n", SIZES)
+def test_inverse_and_product(G, uplo, n):
+    a, other = triangle(n, uplo)
+    part = np.tril if uplo == O.Lower else np.triu
+    t = part(a[:n])
+
+    x = run(G, G.dtrtri, a, uplo, G.NonUnit)
+    assert np.array_equal(x[:n][other], a[:n][other]) and np.array_equal(x[n:], a[n:])
+    x = part(x[:n])
+    assert norm(t @ x - np.eye(n)) <= 4 * n * EPS * norm(t) * norm(x)
+
+    p = run(G, G.dlauum, a, uplo)
+    assert np.array_equal(p[:n][other], a[:n][other]) and np.array_equal(p[n:], a[n:])
+    want = t.T @ t if uplo == O.Lower else t @ t.T
+    assert norm(part(p[:n] - want)) <= 4 * n * EPS * norm(t) * norm(t.T)
+
+    q = run(G, G.dpotri, a, uplo)
+    assert np.array_equal(q[:n][other], a[:n][other]) and np.array_equal(q[n:], a[n:])
+    q = part(q[:n])
+    q = q + q.T - np.diag(q.diagonal())
+    assert norm(want_full(t, uplo) @ q - np.eye(n)) <= 4 * n * EPS * (norm(t) * norm(t.T)
+                                                                    * norm(x) * norm(x.T))
+
+
+def want_full(t, uplo):
+    return t @ t.T if uplo == O.Lower else t.T @ t
+
+
+@pytest.mark.parametrize("n,zero", [(48, 47), (100, 0), (300, 130), (777, 776)])
+def test_zero_diagonal(G, n, zero):
+    import torch
+    a, _ = triangle(n, O.Lower)
+    a[zero, zero] = 0.0
+    for f in (lambda d, i: G.dtrtri(O.Lower, G.NonUnit, n, d, n + 3, i),
+              lambda d, i: G.dpotri(O.Lower, n, d, n + 3, i)):
+        d = G.from_fortran(a)
+        info = torch.zeros(1, dtype=torch.int32, device="cuda")
+        f(d, info)
+        assert int(info.item()) == zero + 1
+        assert np.array_equal(G.to_fortran(d), a)
