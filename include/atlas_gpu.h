@@ -150,7 +150,10 @@ int atlg_dpotri(int Uplo, long N, double *A, long lda, int *dinfo,
  *   Bbar = L^-T Xbar, and -tril(Bbar X^T) is added to Lbar (if not NULL).
  * atlg_dlogdet_chol: *out (device) = log det K = 2 sum log L_ii.
  * atlg_dlogdet_chol_adjoint: adds 2 (*dbar) / L_ii to the diagonal of Lbar
- *   (dbar in device memory). */
+ *   (dbar in device memory).
+ * atlg_dloglik_grad: W <- *g / 2 (A A^T - K inv(L L^T)), both triangles, for
+ *   A (N x K): the gradient of a Gaussian log-likelihood by its covariance;
+ *   W may be L; info as atlg_dpotri's. */
 int atlg_dpotrf_adjoint(long N, const double *L, long ldl, double *G, long ldg,
                         atlg_stream_t stream);
 int atlg_dtrsm_adjoint(long N, long NRHS, const double *L, long ldl,
@@ -161,6 +164,9 @@ int atlg_dlogdet_chol(long N, const double *L, long ldl, double *out,
 int atlg_dlogdet_chol_adjoint(long N, const double *L, long ldl,
                               const double *dbar, double *Lbar, long ldlb,
                               atlg_stream_t stream);
+int atlg_dloglik_grad(long N, long K, const double *L, long ldl,
+                      const double *A, long lda, const double *g, double *W,
+                      long ldw, int *info, atlg_stream_t stream);
 
 /* ---- Single precision and the mixed-precision solver (the FP32 path is
  * the ATL_s instance of the same ATLAS routines: ATL_sgemm, ATL_sgetrf,

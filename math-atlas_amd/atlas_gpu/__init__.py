@@ -119,6 +119,7 @@ _SIGS = {
     "atlg_dpotrf_adjoint": (_i, [_l, _v, _l, _v, _l, _v]),
     "atlg_dtrsm_adjoint": (_i, [_l, _l, _v, _l, _v, _l, _v, _l, _v, _l, _v]),
     "atlg_dlogdet_chol": (_i, [_l, _v, _l, _v, _v]),
+    "atlg_dloglik_grad": (_i, [_l, _l, _v, _l, _v, _l, _v, _v, _l, _v, _v]),
     "atlg_dlogdet_chol_adjoint": (_i, [_l, _v, _l, _v, _v, _l, _v]),
     "atlg_sgemm": (_i, [_i, _i, _l, _l, _l, ctypes.c_float, _v, _l, _v, _l, ctypes.c_float, _v,
                         _l, _v]),
@@ -530,6 +531,11 @@ def dlogdet_chol(n, L, ldl, out, stream=None):
 def dlogdet_chol_adjoint(n, L, ldl, dbar, Lbar, ldlb, stream=None):
     _check(lib().atlg_dlogdet_chol_adjoint(n, _ptr(L), ldl, _ptr(dbar), _ptr(Lbar), ldlb,
                                            _stream(stream)), "atlg_dlogdet_chol_adjoint")
+
+
+def dloglik_grad(n, k, L, ldl, A, lda, g, W, ldw, info, stream=None):
+    _check(lib().atlg_dloglik_grad(n, k, _ptr(L), ldl, _ptr(A), lda, _ptr(g), _ptr(W), ldw,
+                                   _ptr(info), _stream(stream)), "atlg_dloglik_grad")
 
 
 # ---------------------------------------------------------------- batched SPD solvers

@@ -4,7 +4,7 @@ Forward and backward both run in libatlas_gpu.so: potrf, the triangular
 solve and logdet forward, and the hand-written adjoint kernels
 (atlg_dpotrf_adjoint, atlg_dtrsm_adjoint, atlg_dlogdet_chol_adjoint)
 backward of the primitives.  The fused log-likelihood's backward uses the
-closed form of its gradient (potri, a triangular solve and a SYRK).  Matrices are torch float64 CUDA tensors in their natural
+closed form of its gradient (a triangular solve and atlg_dloglik_grad).  Matrices are torch float64 CUDA tensors in their natural
 orientation (K symmetric, L lower triangular with K = L L^T); the column-major
 buffers the library works on are built internally.
 
@@ -25,7 +25,7 @@ import math
 
 import torch
 
-from . import (Lower, NoTrans, Trans, NonUnit, Left, dpotrf, dpotri, dsyrk, dtrsm,
+from . import (Lower, NoTrans, Trans, NonUnit, Left, dpotrf, dtrsm, dloglik_grad,
                dpotrf_adjoint, dtrsm_adjoint, dlogdet_chol, dlogdet_chol_adjoint)
 
 
@@ -174,16 +174,14 @@ class GaussianLogLik(torch.autograd.Function):
         # eq. 5.9): with A = K^-1 Y = L^-T X,
         #   dloss/dK = g/2 (A A^T - k K^-1),   dloss/dY = -g A,
         # K^-1 = L^-T L^-1 by potri (trtri + lauum, 2N^3/3 flops) in place of
-        # the chain of the three adjoints (about 3N^3).  The lower triangle
-        # of K^-1 takes the rank-k term by SYRK, then is mirrored.
+        # the chain of the three adjoints (about 3N^3), and one pass that adds
+        # the rank-k term to its triangle, scales and mirrors it.
         A = X.clone()
         dtrsm(Left, Lower, Trans, NonUnit, n, k, 1.0, buf, n, A, n)
-        W = buf.clone() if ctx.store else buf
-        info = torch.zeros(1, dtype=torch.int32, device=W.device)
-        dpotri(Lower, n, W, n, info)  # cannot fail: the factor's diagonal is positive
-        dsyrk(Lower, NoTrans, n, k, 0.5, A, n, -0.5 * k, W, n)
-        # W's column-major lower triangle is the tensor's upper one
-        G = torch.triu(W).add_(torch.triu(W, 1).t()).mul_(gval)
+        G = torch.empty_like(buf) if ctx.store else buf
+        info = torch.zeros(1, dtype=torch.int32, device=G.device)
+        # (cannot fail: the factor's diagonal is positive)
+        dloglik_grad(n, k, buf, n, A, n, gval, G, n, info)
         ybar = _rhs_out(A.mul_(-gval), y)
         return G, ybar, None
 

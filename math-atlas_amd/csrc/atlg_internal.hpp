@@ -226,6 +226,8 @@ void syr2k(hipStream_t s, int uplo, int trans, long N, long K, double alpha, con
 void trtri(hipStream_t s, int uplo, int diag, long N, double* A, long lda, int* dinfo);
 void lauum(hipStream_t s, int uplo, long N, double* A, long lda, const int* skip = nullptr);
 void potri(hipStream_t s, int uplo, long N, double* A, long lda, int* dinfo);
+void loglik_grad(hipStream_t s, long N, long K, const double* L, long ldl, const double* A,
+                 long lda, const double* g, double* W, long ldw, int* dinfo);
 
 // Precision of getrf's trailing-update GEMMs: the scalar type's own MFMA,
 // or (float only) BF16 operands with FP32 accumulation, single or split

@@ -256,6 +256,40 @@ tri_copy_out_kernel(int n, int np, const double* __restrict__ X, int lower, int 
   }
 }
 
+// W's lower triangle <- g (wa A A^T + wb W), and its mirror above, by 32x32
+// tiles through LDS, block i (i + 1) / 2 + j taking tile (i, j); A is n x k.
+constexpr long kGradMaxK = 16;
+__global__ void __launch_bounds__(256)
+sym_grad_kernel(int n, int k, double wa, const double* __restrict__ A, long lda, double wb,
+                const double* __restrict__ g, double* __restrict__ W, long ldw) {
+  __shared__ double tl[kCT][kCT + 1];
+  const int id = blockIdx.x;
+  int ti = (int)((sqrtf(8.0f * (float)id + 1.0f) - 1.0f) * 0.5f);
+  while ((ti + 1) * (ti + 2) / 2 <= id) ti++;
+  while (ti * (ti + 1) / 2 > id) ti--;
+  const int i0 = ti * kCT, j0 = (id - ti * (ti + 1) / 2) * kCT;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
+  const double gs = *g;
+#pragma unroll
+  for (int r = ty; r < kCT; r += 8) {
+    const int i = i0 + tx, j = j0 + r;
+    double v = 0.0;
+    if (i < n && j <= i) {
+      double s = 0.0;
+      for (int q = 0; q < k; q++) s += A[i + (size_t)q * lda] * A[j + (size_t)q * lda];
+      v = gs * (wa * s + wb * W[i + (size_t)j * ldw]);
+      W[i + (size_t)j * ldw] = v;
+    }
+    tl[tx][r] = v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = ty; r < kCT; r += 8) {  // W(j, i) = W(i, j)
+    const int j = j0 + tx, i = i0 + r;
+    if (i < n && j < i) W[j + (size_t)i * ldw] = tl[r][tx];
+  }
+}
+
 double* tri_copy_in(hipStream_t s, bool lower, bool unit, long n, const double* A, long lda,
                     const int* skip) {
   const long np = tri_full_order(n);
@@ -519,22 +553,58 @@ void lauum(hipStream_t s, int uplo, long N, double* A, long lda, const int* skip
 }
 
 // clapack_dpotri (atlas-clp.base:316-362): trtri, then lauum only when the
-// factor had no zero on its diagonal (the device info word skips it).
-void potri(hipStream_t s, int uplo, long N, double* A, long lda, int* dinfo) {
+// factor had no zero on its diagonal (the device info word skips it).  The
+// factor is F, the result's triangle goes to A (F itself, or another matrix).
+static void potri_from(hipStream_t s, int uplo, long N, const double* F, long ldf, double* A,
+                       long lda, int* dinfo) {
   if (N > 0 && tri_full_fits(N, kLauumFullMin)) {
     // the inverse stays in the dense copy, from which the product reads
     const bool lower = uplo == kLower;
     set_int(s, dinfo, 0);
-    hipLaunchKernelGGL(diag_zero_kernel, dim3(1), dim3(256), 0, s, (int)N, A, lda, dinfo);
+    hipLaunchKernelGGL(diag_zero_kernel, dim3(1), dim3(256), 0, s, (int)N, F, ldf, dinfo);
     ATLG_LAUNCHED();
     const long np = tri_full_order(N);
-    double* X = tri_copy_in(s, lower, false, N, A, lda, dinfo);
+    double* X = tri_copy_in(s, lower, false, N, F, ldf, dinfo);
     tri_invert_full(s, kNonUnit, N, X, np, dinfo);
     lauum_from_full(s, lower, N, X, np, A, lda, dinfo);
     return;
   }
+  if (A != F)
+    ATLG_HIP(hipMemcpy2DAsync(A, sizeof(double) * lda, F, sizeof(double) * ldf, sizeof(double) * N,
+                              N, hipMemcpyDeviceToDevice, s));
   trtri(s, uplo, kNonUnit, N, A, lda, dinfo);
   lauum(s, uplo, N, A, lda, dinfo);
+}
+
+void potri(hipStream_t s, int uplo, long N, double* A, long lda, int* dinfo) {
+  potri_from(s, uplo, N, A, lda, A, lda, dinfo);
+}
+
+// dloss/dK of the Gaussian log-likelihood, g/2 (A A^T - K inv(K)) for A (N x
+// K columns), from the Cholesky factor L: inv(K)'s lower triangle by
+// potri_from, then one pass that adds the rank-K term, scales and mirrors.
+// That pass reads the triangle and writes the matrix once (order 8192: 0.2 ms;
+// a rank-K update, two triangles extracted, an addition and a scaling took
+// 1.5 ms, and a copy of the factor 0.2).
+void loglik_grad(hipStream_t s, long N, long K, const double* L, long ldl, const double* A,
+                 long lda, const double* g, double* W, long ldw, int* dinfo) {
+  if (N <= 0) {
+    set_int(s, dinfo, 0);
+    return;
+  }
+  potri_from(s, kLower, N, L, ldl, W, ldw, dinfo);
+  double wa = 0.5, wb = -0.5 * (double)K;
+  long k = K;
+  if (k > kGradMaxK) {  // the update by the matrix cores
+    gemm<double>(s, kNoTrans, kTrans, N, N, K, wa, A, lda, A, lda, wb, W, ldw, 1);
+    wa = 0.0;
+    wb = 1.0;
+    k = 0;
+  }
+  const long t = (N + kCT - 1) / kCT;
+  hipLaunchKernelGGL(sym_grad_kernel, dim3((unsigned)(t * (t + 1) / 2)), dim3(256), 0, s, (int)N,
+                     (int)k, wa, A, lda, wb, g, W, ldw);
+  ATLG_LAUNCHED();
 }
 
 }  // namespace atlg

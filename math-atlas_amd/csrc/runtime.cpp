@@ -642,6 +642,15 @@ int atlg_dlogdet_chol_adjoint(long N, const double* L, long ldl, const double* d
   return guarded([&] { logdet_chol_adjoint(resolve_stream(stream), N, L, ldl, dbar, Lbar, ldlb); });
 }
 
+int atlg_dloglik_grad(long N, long K, const double* L, long ldl, const double* A, long lda,
+                      const double* g, double* W, long ldw, int* info, atlg_stream_t stream) {
+  if (N < 0) return -1;
+  if (K < 0) return -2;
+  if (ldl < std::max(1L, N)) return -4;
+  if (lda < std::max(1L, N)) return -6;
+  if (ldw < std::max(1L, N)) return -9;
+  return guarded([&] { loglik_grad(resolve_stream(stream), N, K, L, ldl, A, lda, g, W, ldw, info); });
+}
 
 int atlg_sgemm(int TA, int TB, long M, long N, long K, float alpha, const float* A, long lda,
                const float* B, long ldb, float beta, float* C, long ldc, atlg_stream_t stream) {

@@ -1,4 +1,4 @@
-"""Triangular inverse, LAUUM and POTRI at the orders where their products
+"""Triangular inverse, LAUUM, POTRI and the likelihood gradient over it at the orders where their products
 change form: one 128-row block, the dense copy's smallest orders, ragged last
 blocks, levels of several blocks in one launch (FP64).
 
@@ -24,7 +24,7 @@ def G():
 
 
 def norm(a):
-    return np.abs(a).sum(1).max()
+    return np.abs(a).sum(1).max(initial=0.0)
 
 
 def triangle(n, uplo):
@@ -87,3 +87,29 @@ def test_zero_diagonal(G, n, zero):
         f(d, info)
         assert int(info.item()) == zero + 1
         assert np.array_equal(G.to_fortran(d), a)
+
+
+@pytest.mark.parametrize("n,k,same", [(1, 1, False), (20, 2, False), (47, 0, False), (48, 3, True), (65, 16, False),
+                                      (100, 17, True), (129, 1, False), (300, 40, False), (513, 2, True)])
+def test_loglik_grad(G, n, k, same):
+    # g/2 (A A^T - k inv(L L^T)), symmetric to the bit; the sums as above
+    import torch
+    a, _ = triangle(n, O.Lower)
+    t = np.tril(a[:n])
+    rng = np.random.default_rng(k)
+    x = np.asfortranarray(rng.standard_normal((n + 1, max(k, 1))))
+    d, dx = G.from_fortran(a), G.from_fortran(x)
+    w = d if same else G.from_fortran(np.full((n + 3, n), np.nan, order="F"))
+    g = torch.tensor(-1.7, dtype=torch.float64, device="cuda")
+    info = torch.full((1,), -7, dtype=torch.int32, device="cuda")
+    G.dloglik_grad(n, k, d, n + 3, dx, n + 1, g, w, n + 3, info)
+    assert int(info.item()) == 0
+    got = G.to_fortran(w)[:n]
+    assert np.array_equal(got, got.T)
+    if not same:
+        assert np.array_equal(G.to_fortran(d), a)
+    ti = np.linalg.inv(t)
+    aa = x[:n, :k] @ x[:n, :k].T
+    want = -0.85 * (aa - k * (ti.T @ ti))
+    scale = norm(t) * norm(t.T) * norm(ti) ** 2 * norm(ti.T) ** 2
+    assert norm(got - want) <= 4 * max(n, k, 1) * EPS * (norm(x[:n, :k]) * norm(x[:n, :k].T) + k * scale)
