@@ -50,14 +50,29 @@ __global__ void tx_reset(tx_word* x, long n, int* err) {
 template <class S>
 struct TxRows {
   S v[kTxB / 16][4];
-  // element (row n, column k) at p[k * step]; rows and columns outside are zero
-  __device__ __forceinline__ void load(const S* __restrict__ p, long step, int lk, int cols, bool in) {
+  // element (row n, column k) at p[k * step] (STEP1: step is 1, and a block
+  // known to be full takes a lane's four columns by 16-byte loads: transposed,
+  // order 2500 with 1701 right-hand sides 502 -> 453 us); rows and columns
+  // outside are zero
+  template <bool STEP1>
+  __device__ __forceinline__ void load(const S* __restrict__ p, long step, int lk, int cols, bool in,
+                                       bool full) {
+    if (STEP1 && full) {
+#pragma unroll
+      for (int c = 0; c < kTxB / 16; c++) {
+        typedef S quad __attribute__((ext_vector_type(4), aligned(sizeof(S))));
+        const quad w = *reinterpret_cast<const quad*>(p + 16 * c + 4 * lk);
+#pragma unroll
+        for (int s = 0; s < 4; s++) v[c][s] = w[s];
+      }
+      return;
+    }
 #pragma unroll
     for (int c = 0; c < kTxB / 16; c++)
 #pragma unroll
       for (int s = 0; s < 4; s++) {
         const int k = 16 * c + 4 * lk + s;
-        v[c][s] = in && k < cols ? p[(size_t)k * step] : S(0);
+        v[c][s] = in && k < cols ? p[(size_t)k * (STEP1 ? 1 : step)] : S(0);
       }
   }
 };
@@ -69,7 +84,8 @@ __device__ __forceinline__ int tx_lane_col(int ln) {
   return sizeof(S) == 8 ? 4 * (ln & 3) + (ln >> 2) : ln;
 }
 
-template <class S, bool TR>
+// FOLD: the last block's product is folded into the inverse (see above)
+template <class S, bool TR, bool FOLD>
 __global__ void __launch_bounds__(kTxThreads)
 trsv_xcd(int n, int nb, int nrhs, int gpad, int upper, S alpha, const S* __restrict__ A, long lda,
          const S* __restrict__ Dinv, int dtrans, S* __restrict__ B, long bi, long bj,
@@ -82,7 +98,7 @@ trsv_xcd(int n, int nb, int nrhs, int gpad, int upper, S alpha, const S* __restr
   if (c0 >= nrhs || (skip && *skip)) return;
   const int nc = min(kTxCols, nrhs - c0);
   __shared__ S xs[2][kTxB * kTxLd], ys[kTxB * kTxLd];
-  __shared__ S al[kTxB][kTxB + 1];
+  __shared__ S al[FOLD ? kTxB : 1][kTxB + 1];
   __shared__ int bad;
   const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int ln = lane & 15, lk = lane >> 4;
@@ -118,10 +134,11 @@ trsv_xcd(int n, int nb, int nrhs, int gpad, int upper, S alpha, const S* __restr
       for (int u = 0; u < 4; u++)
         xs[lj & 1][lane * kTxLd + v + 4 * u] =
             (S)__longlong_as_double(static_cast<long long>(x[u]));
-      if (lj + 1 == li) lds_barrier();
+      if (FOLD && lj + 1 == li) lds_barrier();
       lds_barrier();
       if (bad) return;
     }
+    if (!FOLD) lds_barrier();
     return;
   }
   const int row = 16 * w + ln;
@@ -130,25 +147,27 @@ trsv_xcd(int n, int nb, int nrhs, int gpad, int upper, S alpha, const S* __restr
   TxRows<S> a0, a1, d, f;
   auto load_a = [&](TxRows<S>& a, int lj) {
     const int q0 = (upper ? nb - 1 - lj : lj) * kTxB;
+    const bool full = rows == kTxB && n - q0 >= kTxB;
     if (TR)
-      a.load(A + (size_t)(r0 + row) * lda + q0, 1, lk, n - q0, in);
+      a.template load<true>(A + (size_t)(r0 + row) * lda + q0, 1, lk, n - q0, in, full);
     else
-      a.load(A + (r0 + row) + (size_t)q0 * lda, lda, lk, n - q0, in);
+      a.template load<false>(A + (r0 + row) + (size_t)q0 * lda, lda, lk, n - q0, in, full);
   };
-  if (li > 0) load_a(f, li - 1);
+  if (FOLD && li > 0) load_a(f, li - 1);
   const S* D = Dinv + (size_t)(r0 / NB) * NB * NB + (size_t)(r0 % NB) * (NB + 1);
   if (dtrans)
-    d.load(D + (size_t)row * NB, 1, lk, rows, in);
+    d.template load<true>(D + (size_t)row * NB, 1, lk, rows, in, rows == kTxB);
   else
-    d.load(D + row, NB, lk, rows, in);
+    d.template load<false>(D + row, NB, lk, rows, in, rows == kTxB);
   S rhs[4];
 #pragma unroll
   for (int r = 0; r < 4; r++) {
     const int c = M::row(lane, r);
     rhs[r] = in && c < nc ? alpha * B[(r0 + row) * bi + (c0 + c) * bj] : S(0);
   }
-  if (li > 1) load_a(a0, 0);
-  if (li > 2) load_a(a1, 1);
+  const int ls = FOLD ? li - 1 : li;  // blocks folded in one by one
+  if (ls > 0) load_a(a0, 0);
+  if (ls > 1) load_a(a1, 1);
   acc_t acc, acc2;
   auto mul = [&](const S* xl, const TxRows<S>& m) {
 #pragma unroll
@@ -161,14 +180,14 @@ trsv_xcd(int n, int nb, int nrhs, int gpad, int upper, S alpha, const S* __restr
   };
   // f = -inv(A_pp) A_pq, q the block solved right before this one: one product
   // only follows q on the chain
-  if (li > 0) {
+  if (FOLD && li > 0) {
 #pragma unroll
     for (int c = 0; c < kTxB / 16; c++)
 #pragma unroll
       for (int s = 0; s < 4; s++) al[row][16 * c + 4 * lk + s] = -f.v[c][s];
   }
   lds_barrier();
-  if (li > 0) {
+  if (FOLD && li > 0) {
     const int fm = tx_lane_col<S>(ln);
 #pragma unroll
     for (int c = 0; c < kTxB / 16; c++) {
@@ -189,13 +208,13 @@ trsv_xcd(int n, int nb, int nrhs, int gpad, int upper, S alpha, const S* __restr
     lds_barrier();
     if (bad) return false;
     mul(xs[lj & 1], a);
-    if (lj + 3 < li) load_a(a, lj + 2);
+    if (lj + 2 < ls) load_a(a, lj + 2);
     return true;
   };
   bool ok = true;
-  for (int lj = 0; lj + 1 < li && ok; lj += 2) {
+  for (int lj = 0; lj < ls && ok; lj += 2) {
     ok = step(a0, lj);
-    if (ok && lj + 2 < li) ok = step(a1, lj + 1);
+    if (ok && lj + 1 < ls) ok = step(a1, lj + 1);
   }
   if (ok) {
     // inv(A_pp) (alpha b - the blocks before q), then q's share
@@ -205,7 +224,7 @@ trsv_xcd(int n, int nb, int nrhs, int gpad, int upper, S alpha, const S* __restr
     lds_barrier();
     acc = acc2 = acc_t{0, 0, 0, 0};
     mul(ys, d);
-    if (li > 0) {
+    if (FOLD && li > 0) {
       lds_barrier();
       ok = !bad;
       mul(xs[(li - 1) & 1], f);
@@ -228,15 +247,15 @@ trsv_xcd(int n, int nb, int nrhs, int gpad, int upper, S alpha, const S* __restr
   }
 }
 
-// Largest order solved in one launch.  Up to 128 right-hand sides (a group per
-// XCD) 2048: longer triangles are halved first, so that the whole device
-// reads what lies off the diagonal blocks.  More groups take turns on a
-// compute unit and the products outweigh the chain: order 2500 with 200 / 500
-// / 1000 / 1701 right-hand sides takes 180 / 213 / 303 / 460 us with launches
-// up to order 1024, 220 / 251 / 334 / 492 up to 512 and 347 / 375 / 441 / 549
-// without; with 4000 they lose (914 against 836).
+// Largest order solved in one launch.  Longer triangles are halved first, so
+// that the whole device reads what lies off the diagonal blocks; the more
+// right-hand sides, the more its large products save over the 16-column
+// groups, which take turns on a compute unit.  Order 2500 by launches up to
+// order 2048 / 1024 / 512 / none: 200 right-hand sides 152 / 178 / 220 / 347
+// us, 500 181 / 208 / 251 / 375, 1701 455 / 425 / 492 / 549, 2500 - / 567 /
+// 597 / 669, 4000 - / 831 / 828 / 842; order 4096, transposed, 500 467 / 436.
 inline long tx_order(long nrhs) {
-  return nrhs <= kTxCols * kTxGroups ? 2048 : nrhs <= 2048 ? 1024 : 0;
+  return nrhs <= 384 ? 2048 : nrhs <= 3072 ? 1024 : nrhs <= 4096 ? 512 : 0;
 }
 
 // Solves op(A) X = alpha B, op(A) lower (or upper) triangular of order n <=
@@ -262,12 +281,12 @@ bool trsv_one_launch(hipStream_t s, bool lower, bool tr, long n, long nrhs, S al
   const int up = lower ? 0 : 1;
   int* status = status_word(s);
   const long limit = wait_limit(kSvSpin);
-  if (tr)
-    hipLaunchKernelGGL((trsv_xcd<S, true>), grid, block, 0, s, (int)n, nb, (int)nrhs, gpad, up, alpha, A,
-                       lda, Dinv, dtrans, B, bi, bj, xb, err, status, limit, skip);
-  else
-    hipLaunchKernelGGL((trsv_xcd<S, false>), grid, block, 0, s, (int)n, nb, (int)nrhs, gpad, up, alpha, A,
-                       lda, Dinv, dtrans, B, bi, bj, xb, err, status, limit, skip);
+  // more groups than XCDs: throughput counts, and folding adds to the products
+  const bool fold = groups <= kTxGroups;
+  const auto fn = tr ? (fold ? trsv_xcd<S, true, true> : trsv_xcd<S, true, false>)
+                     : (fold ? trsv_xcd<S, false, true> : trsv_xcd<S, false, false>);
+  hipLaunchKernelGGL(fn, grid, block, 0, s, (int)n, nb, (int)nrhs, gpad, up, alpha, A, lda, Dinv,
+                     dtrans, B, bi, bj, xb, err, status, limit, skip);
   ATLG_LAUNCHED();
   return true;
 }

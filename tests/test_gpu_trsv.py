@@ -1,5 +1,5 @@
-"""Triangular solves with few right-hand sides (one launch up to order 2048 or
-1024, halves above; one right-hand side above 4096 by the sync-free launch):
+"""Triangular solves with few right-hand sides (one launch up to order 2048,
+1024 or 512, halves above; one right-hand side above 4096 by the sync-free launch):
 orders around the 64-row blocks and the 128-row inverses, right-hand sides
 around the 16-column groups, every side, triangle, transpose and diagonal.
 
@@ -48,7 +48,7 @@ def close(n, t, x, b, alpha):
 @pytest.mark.parametrize("trans", [O.NoTrans, O.Trans])
 @pytest.mark.parametrize("n,k", [(129, 1), (191, 16), (192, 17), (193, 3), (256, 128), (257, 129),
                                  (500, 5), (1000, 33), (2047, 2), (2048, 1), (2049, 1), (4097, 1),
-                                 (1024, 250), (1025, 300), (300, 2048), (200, 2049)])
+                                 (1024, 385), (1025, 400), (2049, 384), (300, 3073), (200, 4097)])
 def test_few_rhs(G, uplo, trans, n, k):
     a, b = system(n, k, n + k)
     for diag, alpha in ((O.NonUnit, 1.0), (O.Unit, -0.7)):
