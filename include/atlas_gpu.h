@@ -87,15 +87,17 @@ int atlg_dtrsm(int Side, int Uplo, int TA, int Diag, long M, long N,
  * semantics and results as atlg_dtrsm, except that the order of op(A)
  * (M for Left, N for Right) may be at most 8192: larger orders return
  * ATLG_ESIZE (atlg_last_error() says why) and queue nothing.  Its workspace
- * (the inverses of the 128 x 128 diagonal blocks, 8 MiB) is a static device
- * array, one per GPU, held until the process ends and shared by every call
+ * (the inverses of the 128 x 128 diagonal blocks and the blocks that the
+ * one-launch solves exchange, 32 MiB) is a static device array, one per GPU,
+ * held until the process ends and shared by every call
  * on that GPU: calls that overlap on one GPU (different streams, or host
  * threads) race and must be serialized by the caller.  It never calls
  * hipMalloc or hipFree (atlg_init resolves the array's address on the
- * current device; another device's on its first call).  Few right-hand
- * sides take the blocked solve here, not atlg_dtrsm's sync-free one, so
- * results agree with atlg_dtrsm to rounding, bit for bit when NRHS > 4 or
- * the order is below 1024. */
+ * current device; another device's on its first call).  One right-hand
+ * side above order 4096 takes the blocked solve here, not atlg_dtrsm's
+ * sync-free one, so results agree with atlg_dtrsm to rounding, bit for bit
+ * when NRHS > 4 or the order is below 1024.  A wait that fails is reported
+ * as atlg_dtrsm's is. */
 #define ATLG_ESIZE (-1002)
 int atlg_dtrsm_noalloc(int Side, int Uplo, int TA, int Diag, long M, long N,
                        double alpha, const double *A, long lda, double *B,

@@ -308,12 +308,16 @@ int* status_word(hipStream_t s) {
 int take_status(hipStream_t s) {
   int* w = status_word(s);
   int v = 0;
-  ATLG_HIP(hipMemcpyAsync(&v, w, sizeof(int), hipMemcpyDeviceToHost, s));
+  int* const words[2] = {w, noalloc_status()};  // and that of the allocation-free solves
+  int got[2] = {0, 0};
+  for (int i = 0; i < 2; i++)
+    if (words[i])
+      ATLG_HIP(hipMemcpyAsync(&got[i], words[i], sizeof(int), hipMemcpyDeviceToHost, s));
   ATLG_HIP(hipStreamSynchronize(s));
-  if (v != 0) {
-    set_int(s, w, 0);
-    ATLG_HIP(hipStreamSynchronize(s));
-  }
+  for (int i = 0; i < 2; i++)
+    if (got[i] != 0) set_int(s, words[i], 0);
+  v = got[0] | got[1];
+  if (v != 0) ATLG_HIP(hipStreamSynchronize(s));
   return v;
 }
 

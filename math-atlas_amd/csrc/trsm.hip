@@ -8,15 +8,17 @@
 // diagonals and runs everything off the diagonal as amm GEMM; this version
 // goes one step further:
 //   1. one launch inverts every NB x NB diagonal block of op(A) in LDS
-//      (one workgroup per block: 8x8 register inverses, then recursive
-//      doubling), writing full NB x NB inverses;
-//   2. a recursive halving driver (the same split as trsm_recL/R) applies
-//      each inverse to its block row/column as an in-place GEMM and updates
-//      the rest with large GEMMs.
+//      (one workgroup per block, by 16x16 tiles), writing full NB x NB
+//      inverses;
+//   2. a recursive halving driver (the same split as trsm_recL/R) updates
+//      with large GEMMs down to an order that one launch solves with these
+//      inverses (trsv_xcd.hpp), or, for very many right-hand sides, to single
+//      blocks, whose inverses apply as in-place GEMMs.
 // All flops but the small inversions run on the 16x16x4 MFMA GEMM.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <type_traits>
 
@@ -51,7 +53,8 @@ __device__ inline S opa(const S* A, long lda, bool trans, long i, long j) {
 // four columns at a time, each its own, by carrying the identity to L^-T;
 // then each computes its row of L^-T tile by tile from its own results, the
 // tiles of L in LDS and the diagonal inverses, with no barrier between the
-// waves.  128-block 31 -> 11 us (8x8 register inverses and five doubling
+// waves.  The 64 blocks of an order-8192 triangle take 20 us; a solve of
+// order 128 went from 38 to 28 us (8x8 register inverses and five doubling
 // levels with four barriers each before).
 template <class R, int NT>
 __global__ void __launch_bounds__(4 * NT)
@@ -202,7 +205,7 @@ struct Ctx {
   const S* Dinv;
   int dtrans;  // kTrans when Dinv holds the transposes of inv(op(A)_bb)
   const int* skip;
-  bool alloc;  // scratch memory may be used
+  unsigned char* fixed;  // exchange memory of the one-launch solves, or nullptr: the stream's own
 };
 
 // op(A)[i0:, j0:] as a GEMM operand: pointer and transpose flag.
@@ -241,11 +244,11 @@ void solve(const Ctx<S>& c, long r0, long n, S alpha) {
   }
   // X op(A) = B is op(A)^T X^T = B^T
   const long rhs = c.left ? c.N : c.M;
-  if (c.alloc && n <= tx_order(rhs) &&
+  if (n <= tx_order(rhs) &&
       trsv_one_launch<S>(c.s, c.lower_eff == c.left, c.trans == c.left, n, rhs, alpha,
                          c.A + r0 + r0 * c.lda, c.lda, c.Dinv + (size_t)(r0 / NB) * NB * NB,
                          (c.dtrans == kTrans) == c.left, c.B + (c.left ? r0 : r0 * c.ldb),
-                         c.left ? 1 : c.ldb, c.left ? c.ldb : 1, c.skip))
+                         c.left ? 1 : c.ldb, c.left ? c.ldb : 1, c.skip, c.fixed))
     return;
   const long n1 = split(n), n2 = n - n1;
   const S* Ap;
@@ -488,7 +491,7 @@ void trsm(hipStream_t s, int side, int uplo, int ta, int diag, long M, long N, S
   c.M = M;
   c.N = N;
   c.skip = skip;
-  c.alloc = true;
+  c.fixed = nullptr;
   const long na = c.left ? M : N;
   c.dtrans = dinv ? (dinv_trans ? kTrans : kNoTrans) : kNoTrans;
   if (dinv) {
@@ -507,11 +510,12 @@ void trsm(hipStream_t s, int side, int uplo, int ta, int diag, long M, long N, S
 }
 
 void* noalloc_scratch();
+void noalloc_used();
 
 // The allocation-free form: the diagonal-block inverses go to the file-scope
-// device array (at most kNoAllocMaxOrder / kTrsmNB blocks), and the solve is
-// the blocked recursion of trsm() (no few-RHS launch, whose ready flags and
-// failure word would need memory of their own).
+// device array (at most kNoAllocMaxOrder / kTrsmNB blocks), and so does the
+// exchange area of the one-launch solves; the solve is otherwise trsm()'s
+// without its sync-free launch for one right-hand side.
 template <class S>
 void trsm_noalloc(hipStream_t s, int side, int uplo, int ta, int diag, long M, long N, S alpha,
                   const S* A, long lda, S* B, long ldb) {
@@ -536,7 +540,8 @@ void trsm_noalloc(hipStream_t s, int side, int uplo, int ta, int diag, long M, l
   c.M = M;
   c.N = N;
   c.skip = nullptr;
-  c.alloc = false;
+  c.fixed = static_cast<unsigned char*>(noalloc_scratch()) + kNoAllocInvBytes;
+  noalloc_used();
   c.Dinv = D;
   c.dtrans = kNoTrans;
   solve(c, 0, na, alpha);
@@ -557,8 +562,9 @@ template void trsm<float>(hipStream_t, int, int, int, int, long, long, float, co
 }  // namespace atlg
 
 // ---- the device array behind atlg_dtrsm_noalloc ---------------------------
-// kNoAllocMaxOrder / kTrsmNB inverses of 128 x 128 doubles (8 MiB), one copy
-// per device, held until the process ends.  Its name is only a host-side
+// kNoAllocMaxOrder / kTrsmNB inverses of 128 x 128 doubles (8 MiB), the
+// exchange area of the one-launch solves (24 MiB) and their failure word, one
+// copy per device, held until the process ends.  Its name is only a host-side
 // stand-in for the symbol: host code uses the address that
 // hipGetSymbolAddress returns for the current device, never the name itself.
 static __device__ __align__(256) unsigned char scratch[atlg::kNoAllocBytes];
@@ -568,6 +574,7 @@ namespace {
 constexpr int kMaxDevices = 64;
 std::mutex g_noalloc_mu;
 void* g_noalloc_ptr[kMaxDevices] = {};
+std::atomic<bool> g_noalloc_used[kMaxDevices];
 }  // namespace
 
 // Address of the array on the current device, resolved once per device
@@ -583,6 +590,19 @@ void* noalloc_scratch() {
     g_noalloc_ptr[dev] = p;
   }
   return g_noalloc_ptr[dev];
+}
+
+void noalloc_used() {
+  int dev = 0;
+  ATLG_HIP(hipGetDevice(&dev));
+  g_noalloc_used[dev].store(true);  // (noalloc_scratch() has checked the index)
+}
+
+int* noalloc_status() {
+  int dev = 0;
+  ATLG_HIP(hipGetDevice(&dev));
+  if (dev < 0 || dev >= kMaxDevices || !g_noalloc_used[dev].load()) return nullptr;
+  return reinterpret_cast<int*>(static_cast<unsigned char*>(noalloc_scratch()) + kNoAllocBytes - 256);
 }
 
 }  // namespace atlg

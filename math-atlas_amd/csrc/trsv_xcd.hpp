@@ -257,19 +257,29 @@ trsv_xcd(int n, int nb, int nrhs, int gpad, int upper, S alpha, const S* __restr
 inline long tx_order(long nrhs) {
   return nrhs <= 384 ? 2048 : nrhs <= 3072 ? 1024 : nrhs <= 4096 ? 512 : 0;
 }
+// The largest exchange area that this asks for (kNoAllocTxBlocks blocks), with
+// its error word.
+constexpr size_t kTxFixedBytes = 256 + sizeof(tx_word) * kTxBlock * kNoAllocTxBlocks;
+static_assert(kNoAllocTxBlocks >= 384 / kTxCols * (2048 / kTxB) &&
+              kNoAllocTxBlocks >= 3072 / kTxCols * (1024 / kTxB) &&
+              kNoAllocTxBlocks >= 4096 / kTxCols * (512 / kTxB), "fixed exchange area");
+static_assert(kTxFixedBytes + 256 == kNoAllocTxBytes, "fixed exchange area");
 
 // Solves op(A) X = alpha B, op(A) lower (or upper) triangular of order n <=
 // tx_order(nrhs), element (i, j) of X and B at i bi + j bj; Dinv holds the inverses
-// of op(A)'s NB x NB diagonal blocks, or their transposes (dtrans).  False, with nothing queued,
+// of op(A)'s NB x NB diagonal blocks, or their transposes (dtrans).  `fixed`,
+// when not null, is memory for the exchange area (kTxFixedBytes), with a
+// failure word behind it, in place of the stream's own.  False, with nothing queued,
 // where the exchange area cannot be had.
 template <class S>
 bool trsv_one_launch(hipStream_t s, bool lower, bool tr, long n, long nrhs, S alpha, const S* A,
-                     long lda, const S* Dinv, int dtrans, S* B, long bi, long bj, const int* skip) {
+                     long lda, const S* Dinv, int dtrans, S* B, long bi, long bj, const int* skip,
+                     unsigned char* fixed) {
   const int nb = (int)((n + kTxB - 1) / kTxB);
   const int groups = (int)((nrhs + kTxCols - 1) / kTxCols);
   const long words = (long)groups * nb * kTxBlock;
   tx_word* xb = static_cast<tx_word*>(
-      scratch_in_capture(s, kSlotTrsv, 256 + sizeof(tx_word) * words));
+      fixed ? fixed : scratch_in_capture(s, kSlotTrsv, 256 + sizeof(tx_word) * words));
   if (!xb) return false;
   int* err = reinterpret_cast<int*>(xb);
   xb += 256 / sizeof(tx_word);
@@ -279,7 +289,7 @@ bool trsv_one_launch(hipStream_t s, bool lower, bool tr, long n, long nrhs, S al
   const int gpad = (groups + kTxGroups - 1) / kTxGroups * kTxGroups;
   const dim3 grid(gpad * (nb - 1) + groups), block(kTxThreads);
   const int up = lower ? 0 : 1;
-  int* status = status_word(s);
+  int* status = fixed ? reinterpret_cast<int*>(fixed + kTxFixedBytes) : status_word(s);
   const long limit = wait_limit(kSvSpin);
   // more groups than XCDs: throughput counts, and folding adds to the products
   const bool fold = groups <= kTxGroups;

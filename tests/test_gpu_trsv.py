@@ -117,3 +117,27 @@ def test_captured_without_workspace(G):
             G.dtrsm(G.Left, G.Lower, G.NoTrans, G.NonUnit, n, k, 1.0, da, n + 1, db, n + 2)
         torch.cuda.synchronize()
         assert close(n, t, G.to_fortran(db)[:n], b[:n], 1.0)
+
+
+def test_noalloc_same_bits_and_failure(G):
+    # the allocation-free entry takes the same launches in its own memory, and
+    # a wait that runs over is reported the same way
+    n, k = 1500, 40
+    a, b = system(n, k, 11)
+    da, x, y = G.from_fortran(a), G.from_fortran(b), G.from_fortran(b)
+    G.dtrsm(G.Left, G.Lower, G.NoTrans, G.NonUnit, n, k, 1.0, da, n + 1, x, n + 2, check=True)
+    G.dtrsm_noalloc(G.Left, G.Lower, G.NoTrans, G.NonUnit, n, k, 1.0, da, n + 1, y, n + 2)
+    G.check_stream()
+    assert np.array_equal(G.to_fortran(x), G.to_fortran(y))
+    G.set_wait_limit(1)
+    try:
+        G.dtrsm_noalloc(G.Left, G.Lower, G.NoTrans, G.NonUnit, n, k, 1.0, da, n + 1, y, n + 2)
+        with pytest.raises(G.AtlgWaitError) as e:
+            G.check_stream()
+        assert e.value.bits & G.FAIL_TRSV
+    finally:
+        G.set_wait_limit(0)
+    y.copy_(G.from_fortran(b))
+    G.dtrsm_noalloc(G.Left, G.Lower, G.NoTrans, G.NonUnit, n, k, 1.0, da, n + 1, y, n + 2)
+    G.check_stream()
+    assert np.array_equal(G.to_fortran(x), G.to_fortran(y))
