@@ -1518,7 +1518,7 @@ void launch_xcd(LU<S>& f, int M, int w, int off, int G, int* lst) {
   // Outside the look-ahead's reserved units, panels of several callers'
   // streams could hold an XCD's units while each waits for more of its own
   // workgroups: cooperative launches do not overlap each other (they cost
-  // about 40 us each, N=1500: 7.2 against 5.0 ms, so the device's gang
+  // about 40 us each, N=1500: 5.7 against 4.4 ms, so the device's gang
   // stream goes without).
   int p = par, g = G;
   long lda = f.lda;

@@ -1,13 +1,12 @@
-// In-LDS inversion of a lower-triangular block (order 32, 64 or 128) by one
-// 256-thread workgroup, shared by the TRSM diagonal-block inverter and the
-// Cholesky leaf kernel.
+// What the kernels that work on triangles in LDS share: a barrier for LDS
+// alone, a lane broadcast, the 16x16x4 MFMA per scalar type, and the in-LDS
+// inversion of a lower-triangular block (order 32 or 64) by one 256-thread
+// workgroup, for the LU's small nodes.
 #pragma once
 #include <hip/hip_runtime.h>
 
 namespace atlg {
 
-constexpr int kTriN = 128;          // largest block order
-constexpr int kTriLD = kTriN + 1;   // LDS pitch (elements) of a kTriN block
 constexpr int kTriThreads = 256;
 
 // A workgroup barrier that orders LDS accesses only: global stores (results
@@ -143,9 +142,9 @@ __device__ inline void tri_level_mfma(R* S, int sz, int n) {
 // general: rows and columns at or beyond n are the identity padding, so
 // every off-diagonal block that starts at or beyond n stays zero and is
 // skipped.  Must be called by all kTriThreads threads; ends with a barrier.
-template <class R, int NT = kTriN>
+template <class R, int NT>
 __device__ inline void lower_inverse_inplace(R* S, int n = NT) {
-  static_assert(NT == 32 || NT == 64 || NT == 128, "block order");
+  static_assert(NT == 32 || NT == 64, "block order");
   constexpr int LD = NT + 1;
   const int t = threadIdx.x;
   if (t < NT / 8 && 8 * t < n) {
