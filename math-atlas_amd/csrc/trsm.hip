@@ -311,8 +311,12 @@ constexpr int SV_T = 256;                  // threads: 2 per block row
 // trsv_xcd.hpp's launches, one right-hand side, op(A) = A: order 4096 178
 // against 168 us, 6000 238 against 268, 16384 734 against 830; with two
 // right-hand sides or op(A) = A^T the halving is the faster at every order
-// (8192: 378 against 406 and 390 against 648 us).
-constexpr long kTrsvMin = 4097;
+// (8192: 378 against 406 and 390 against 648 us).  FP32, by whole mixed
+// solves with six such solves each (the cooperative launch costs its 40 us
+// there): order 6000 21.46 against 21.02 ms, 8192 30.0 against 29.7, 12288
+// 64.8 against 64.9, 20000 123.0 against 124.9.
+template <class S>
+constexpr long kTrsvMin = sizeof(S) == 8 ? 4097 : 10240;
 
 template <class S>
 __device__ inline S ld_co(const S* p);
@@ -502,7 +506,7 @@ void trsm(hipStream_t s, int side, int uplo, int ta, int diag, long M, long N, S
     tri_inverse_blocks<S>(s, na, A, lda, ta, uplo, diag, D, skip);
     c.Dinv = D;
   }
-  if (c.left && !c.trans && c.dtrans == kNoTrans && !skip && N == 1 && na >= kTrsvMin) {
+  if (c.left && !c.trans && c.dtrans == kNoTrans && !skip && N == 1 && na >= kTrsvMin<S>) {
     trsv_long<S>(s, c.lower_eff, na, alpha, A, lda, c.Dinv, B);
     return;
   }
