@@ -42,13 +42,14 @@ void atlg_set_xerbla_hook(void (*hook)(int p, const char *rout,
                                        const char *msg));
 
 /* ---- Failure reporting of the bounded waits (no ATLAS counterpart) ----
- * Two kernels wait on other workgroups of their own launch: the getrf
- * panel (pivot-candidate mailboxes) and the few-RHS triangular solve
- * (per-block ready flags).  Every such wait is bounded; a wait that runs
- * past its bound makes the kernel exit early and ORs one of the bits below
- * into the stream's failure word (the results of that call are then
- * unspecified; getrf also writes *dinfo = INT_MIN and identity pivots for
- * the affected panel, so later launches stay in bounds).
+ * Kernels of two kinds wait on other workgroups of their own launch: the
+ * getrf panels (pivot candidates) and the triangular solves that take one
+ * launch (solved blocks), which getrf, potrf and their solves use too.
+ * Every such wait is bounded; a wait that runs past its bound makes the
+ * kernel exit early and ORs one of the bits below into the failure word of
+ * the stream that the call was given (the results of that call are then
+ * unspecified; getrf and potrf also write *dinfo = INT_MIN, getrf identity
+ * pivots for an affected panel, so later launches stay in bounds).
  * atlg_stream_status: synchronizes `stream`, stores its failure word in
  *   *status (0: no failure) and clears it.
  * atlg_set_failure_hook: the host-pointer entry points (cblas_, clapack_,

@@ -476,8 +476,11 @@ def dgetrs(trans, n, nrhs, a, lda, ipiv, b, ldb, stream=None, check=False):
         check_stream(stream)
 
 
-def dpotrf(uplo, n, a, lda, info, stream=None):
+def dpotrf(uplo, n, a, lda, info, stream=None, check=False):
+    """check=True: as dgetrf's."""
     _check(lib().atlg_dpotrf(uplo, n, _ptr(a), lda, _ptr(info), _stream(stream)), "atlg_dpotrf")
+    if check:
+        check_stream(stream)
 
 
 def dpotrs(uplo, n, nrhs, a, lda, b, ldb, stream=None):

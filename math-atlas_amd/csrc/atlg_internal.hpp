@@ -116,9 +116,9 @@ enum Slot : int {
   kNumSlots = 24
 };
 void* scratch(hipStream_t s, Slot slot, size_t bytes);
-// The same, or nullptr where that (or the stream's failure word) would have
-// to be allocated while the stream is being captured.
-void* scratch_in_capture(hipStream_t s, Slot slot, size_t bytes);
+// The same, or nullptr where that (or, with `status`, the stream's failure
+// word) would have to be allocated while the stream is being captured.
+void* scratch_in_capture(hipStream_t s, Slot slot, size_t bytes, bool status);
 
 // The stream's failure word: a device int that kernels whose bounded waits
 // give up OR their ATLG_FAIL_* bit into (zero otherwise).  Allocated and
@@ -186,10 +186,18 @@ constexpr int kTrsmNB = 128;
 template <class S>
 void tri_inverse_blocks(hipStream_t s, long na, const S* A, long lda, int ta, int uplo, int diag,
                         S* Dinv, const int* skip = nullptr);
+// Where a solve reports a wait that gave up: the failure word of the stream
+// that the caller asks (nullptr: of the stream the solve is queued on; nobody
+// asks a factorization's own streams), and an info word (or nullptr) that
+// becomes INT_MIN.
+struct WaitReport {
+  int* status = nullptr;
+  int* info = nullptr;
+};
 template <class S>
 void trsm(hipStream_t s, int side, int uplo, int ta, int diag, long M, long N, S alpha,
           const S* A, long lda, S* B, long ldb, const int* skip = nullptr,
-          const S* dinv = nullptr, int dinv_trans = 0);
+          const S* dinv = nullptr, int dinv_trans = 0, WaitReport rep = {});
 
 // trsm() without allocation: the diagonal-block inverses, the exchange area
 // of the one-launch solves and their failure word live in a file-scope device

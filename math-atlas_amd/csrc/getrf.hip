@@ -1568,17 +1568,18 @@ void leaf(LU<S>& f, long off, long m, int w) {
 template <class S>
 void node_trsm_cols(LU<S>& f, long off, long nl, long c0, long nc) {
   if (nc <= 0) return;
+  const WaitReport rep = {f.status, f.dinfo};  // f.s may be one of the look-ahead's streams
   if (f.small_lds && nl == kTrsmNB) {
     // beside a running GEMM: two 64-column halves, whose diagonal-block
     // inverses need a quarter of the LDS of a 128-block inverse (which
     // would wait for a compute unit free of GEMM workgroups)
     const long h = nl / 2;
     trsm<S>(f.s, kLeft, kLower, kNoTrans, kUnit, h, nc, S(1), at(f, off, off), f.lda,
-            at(f, off, c0), f.lda);
+            at(f, off, c0), f.lda, nullptr, nullptr, 0, rep);
     gemm<S>(f.s, kNoTrans, kNoTrans, h, nc, h, S(-1), at(f, off + h, off), f.lda, at(f, off, c0),
             f.lda, S(1), at(f, off + h, c0), f.lda);
     trsm<S>(f.s, kLeft, kLower, kNoTrans, kUnit, h, nc, S(1), at(f, off + h, off + h), f.lda,
-            at(f, off + h, c0), f.lda);
+            at(f, off + h, c0), f.lda, nullptr, nullptr, 0, rep);
     return;
   }
   if (nl >= kTrsmNB && off % kTrsmNB == 0 && nl % kTrsmNB == 0) {
@@ -1592,10 +1593,10 @@ void node_trsm_cols(LU<S>& f, long off, long nl, long c0, long nc) {
       for (long b = first; b < b1; b++) f.inv_done[b] = 1;
     }
     trsm<S>(f.s, kLeft, kLower, kNoTrans, kUnit, nl, nc, S(1), at(f, off, off), f.lda,
-            at(f, off, c0), f.lda, nullptr, f.Winv + (size_t)b0 * kTrsmNB * kTrsmNB, 0);
+            at(f, off, c0), f.lda, nullptr, f.Winv + (size_t)b0 * kTrsmNB * kTrsmNB, 0, rep);
   } else {
     trsm<S>(f.s, kLeft, kLower, kNoTrans, kUnit, nl, nc, S(1), at(f, off, off), f.lda,
-            at(f, off, c0), f.lda);
+            at(f, off, c0), f.lda, nullptr, nullptr, 0, rep);
   }
 }
 

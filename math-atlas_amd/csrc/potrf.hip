@@ -322,7 +322,7 @@ potf2_inv_kernel(int n, double* __restrict__ A, long lda, int lower, int* __rest
 }
 
 void potrf_rec(hipStream_t s, bool lower, long N, double* A, long lda, int* dinfo, int off,
-               double* W) {
+               double* W, int* status) {
   if (N <= 0) return;
   if (N <= DB) {
     hipLaunchKernelGGL(potf2_inv_kernel, dim3(1), dim3(PW_THREADS), 0, s, (int)N, A, lda,
@@ -336,22 +336,24 @@ void potrf_rec(hipStream_t s, bool lower, long N, double* A, long lda, int* dinf
   long nl = (N > 2 * RB) ? RB : ((N / 2) / DB) * DB;
   if (nl < DB) nl = DB;
   const long nr = N - nl;
-  potrf_rec(s, lower, nl, A, lda, dinfo, off, W);
+  potrf_rec(s, lower, nl, A, lda, dinfo, off, W, status);
   double* A22 = A + nl + nl * lda;
   const double* Winv = W + (size_t)(off / DB) * DB * DB;  // inverses of this node's A11
   if (lower) {
     // A21 <- A21 L11^-T: op(A) = L11^T, whose diagonal-block inverses are
     // the transposes of the stored inv(L_bb)
     double* A21 = A + nl;
-    trsm(s, kRight, kLower, kTrans, kNonUnit, nr, nl, 1.0, A, lda, A21, lda, dinfo, Winv, 1);
+    trsm(s, kRight, kLower, kTrans, kNonUnit, nr, nl, 1.0, A, lda, A21, lda, dinfo, Winv, 1,
+         {status, dinfo});
     gemm(s, kNoTrans, kTrans, nr, nr, nl, -1.0, A21, lda, A21, lda, 1.0, A22, lda, 1, dinfo);
   } else {
     // A12 <- U11^-T A12: op(A) = U11^T = L11, inverses stored as is
     double* A12 = A + nl * lda;
-    trsm(s, kLeft, kUpper, kTrans, kNonUnit, nl, nr, 1.0, A, lda, A12, lda, dinfo, Winv, 0);
+    trsm(s, kLeft, kUpper, kTrans, kNonUnit, nl, nr, 1.0, A, lda, A12, lda, dinfo, Winv, 0,
+         {status, dinfo});
     gemm(s, kTrans, kNoTrans, nr, nr, nl, -1.0, A12, lda, A12, lda, 1.0, A22, lda, 2, dinfo);
   }
-  potrf_rec(s, lower, nr, A22, lda, dinfo, off + (int)nl, W);
+  potrf_rec(s, lower, nr, A22, lda, dinfo, off + (int)nl, W, status);
 }
 
 // Look-ahead (1) or plain right-looking steps (0).  At N = 16384 the
@@ -424,8 +426,9 @@ inline bool chol_solve_wide(long rest, long nb1) {
 // block k+1, the auxiliary stream factors block k+1 (updated first) and
 // solves its panel.  lower: A = L L^T, panel L21 = A21 L11^-T, update
 // A22 -= L21 L21^T; upper: A = U^T U, U12 = U11^-T A12, A22 -= U12^T U12.
+// `status`: the failure word of the caller's stream.
 void potrf_lookahead(hipStream_t s0, bool lower, long N, double* A, long lda, int* dinfo,
-                     double* W) {
+                     double* W, int* status) {
   const auto lock = aux_lock();
   hipStream_t s1 = aux_stream();
   hipEvent_t e_upd = aux_event(0), e_panel = aux_event(1);
@@ -449,10 +452,10 @@ void potrf_lookahead(hipStream_t s0, bool lower, long N, double* A, long lda, in
     const double* Winv = W + (size_t)(k / DB) * DB * DB;
     if (lower)
       trsm(s, kRight, kLower, kTrans, kNonUnit, r, kb, 1.0, at(k, k), lda, panel_ptr(k, kb), lda,
-           dinfo, Winv, 1);
+           dinfo, Winv, 1, {status, dinfo});
     else
       trsm(s, kLeft, kUpper, kTrans, kNonUnit, kb, r, 1.0, at(k, k), lda, panel_ptr(k, kb), lda,
-           dinfo, Winv, 0);
+           dinfo, Winv, 0, {status, dinfo});
   };
   // A(c0.., c0..c0+nc) -= P_c P_c^T restricted to the stored triangle, P the
   // panel of block k (kb wide) from its row/column c0 on; m rows/cols in all
@@ -486,7 +489,7 @@ void potrf_lookahead(hipStream_t s0, bool lower, long N, double* A, long lda, in
   hipEvent_t e_col = aux_event(4);
   auto width = [&](long k) { return std::min(chol_step(N - k), N - k); };
   const long kb0 = width(0);
-  potrf_rec(s0, lower, kb0, A, lda, dinfo, 0, W);
+  potrf_rec(s0, lower, kb0, A, lda, dinfo, 0, W, status);
   solve_panel(s0, 0, kb0, N - kb0);
   for (long k0 = 0; k0 + width(k0) < N; k0 += width(k0)) {
     const long kb = width(k0), k1 = k0 + kb, nb1 = width(k1);
@@ -507,7 +510,7 @@ void potrf_lookahead(hipStream_t s0, bool lower, long N, double* A, long lda, in
     }
     update(s0, k0, kb, k1 + nb1, rest, rest, split ? 0 : ATLG_CHOL_CAP);
     ATLG_HIP(hipStreamWaitEvent(s1, e_upd, 0));
-    potrf_rec(s1, lower, nb1, at(k1, k1), lda, dinfo, (int)k1, W);
+    potrf_rec(s1, lower, nb1, at(k1, k1), lda, dinfo, (int)k1, W, status);
     // The panel solve is a GEMM-shaped TRSM of rest x nb1: on the panel
     // units while the trailing update keeps the others busy, on the update
     // side once that update is the shorter path (its units would wait).
@@ -533,10 +536,11 @@ void potrf(hipStream_t s, int uplo, long N, double* A, long lda, int* dinfo) {
   if (N <= 0) return;
   const long nblk = (N + DB - 1) / DB;
   double* W = static_cast<double*>(scratch(s, kSlotFactInv, sizeof(double) * nblk * DB * DB));
+  int* status = status_word(s);
   if (ATLG_CHOL_LOOKAHEAD && N >= kCholLaMin)
-    potrf_lookahead(s, uplo == kLower, N, A, lda, dinfo, W);
+    potrf_lookahead(s, uplo == kLower, N, A, lda, dinfo, W, status);
   else
-    potrf_rec(s, uplo == kLower, N, A, lda, dinfo, 0, W);
+    potrf_rec(s, uplo == kLower, N, A, lda, dinfo, 0, W, status);
 }
 
 void potrs(hipStream_t s, int uplo, long N, long NRHS, const double* A, long lda, double* B,

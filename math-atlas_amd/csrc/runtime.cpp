@@ -273,12 +273,13 @@ void* scratch(hipStream_t s, Slot slot, size_t bytes) {
   return p;
 }
 
-void* scratch_in_capture(hipStream_t s, Slot slot, size_t bytes) {
+void* scratch_in_capture(hipStream_t s, Slot slot, size_t bytes, bool status) {
   {
     std::lock_guard<std::mutex> lk(g_mu);
     auto it = g_slots.find(std::make_pair(s, static_cast<int>(slot)));
     auto st = g_status.find(s);
-    if (it != g_slots.end() && it->second.bytes >= bytes && st != g_status.end() && st->second)
+    if (it != g_slots.end() && it->second.bytes >= bytes &&
+        (!status || (st != g_status.end() && st->second)))
       return it->second.p;
   }
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;

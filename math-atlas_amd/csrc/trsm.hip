@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <climits>
 #include <mutex>
 #include <type_traits>
 
@@ -205,6 +206,7 @@ struct Ctx {
   const S* Dinv;
   int dtrans;  // kTrans when Dinv holds the transposes of inv(op(A)_bb)
   const int* skip;
+  WaitReport rep;
   unsigned char* fixed;  // exchange memory of the one-launch solves, or nullptr: the stream's own
 };
 
@@ -248,7 +250,7 @@ void solve(const Ctx<S>& c, long r0, long n, S alpha) {
       trsv_one_launch<S>(c.s, c.lower_eff == c.left, c.trans == c.left, n, rhs, alpha,
                          c.A + r0 + r0 * c.lda, c.lda, c.Dinv + (size_t)(r0 / NB) * NB * NB,
                          (c.dtrans == kTrans) == c.left, c.B + (c.left ? r0 : r0 * c.ldb),
-                         c.left ? 1 : c.ldb, c.left ? c.ldb : 1, c.skip, c.fixed))
+                         c.left ? 1 : c.ldb, c.left ? c.ldb : 1, c.skip, c.rep, c.fixed))
     return;
   const long n1 = split(n), n2 = n - n1;
   const S* Ap;
@@ -362,7 +364,8 @@ template <class S>
 __global__ void __launch_bounds__(SV_T)
 trsv_sf_kernel(int n, int nb, int upper, S alpha, const S* __restrict__ A, long lda,
                const S* __restrict__ Dinv, S* __restrict__ B, int* __restrict__ flags,
-               int* __restrict__ err, int* __restrict__ status, long limit) {
+               int* __restrict__ err, int* __restrict__ status, int* __restrict__ info,
+               long limit) {
   __shared__ S part[2][NB];
   __shared__ S xs[NB];
   __shared__ int ok;
@@ -391,6 +394,7 @@ trsv_sf_kernel(int n, int nb, int upper, S alpha, const S* __restrict__ A, long 
           if (++spins >= limit || ((spins & 255) == 0 && ld_flag(err))) {
             st_flag(err, 1);
             atomicOr(status, ATLG_FAIL_TRSV);
+            if (info) *info = INT_MIN;
             good = false;
             break;
           }
@@ -435,7 +439,7 @@ trsv_sf_kernel(int n, int nb, int upper, S alpha, const S* __restrict__ A, long 
 // is lower triangular, and Dinv holding the inverses of A's diagonal blocks.
 template <class S>
 void trsv_long(hipStream_t s, bool lower, long n, S alpha, const S* A, long lda, const S* Dinv,
-               S* B) {
+               S* B, const WaitReport& rep) {
   const int nb = (int)((n + NB - 1) / NB);
   int* flags = static_cast<int*>(scratch(s, kSlotTrsv, sizeof(int) * (nb + 64)));
   int* err = flags + nb;
@@ -447,9 +451,10 @@ void trsv_long(hipStream_t s, bool lower, long n, S alpha, const S* A, long lda,
   ATLG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   int nn = (int)n, nbk = nb, up = lower ? 0 : 1;
   int G = std::max(1, std::min(nb, cus));
-  int* status = status_word(s);
+  int *status = rep.status ? rep.status : status_word(s), *info = rep.info;
   long limit = wait_limit(kSvSpin);
-  void* args[] = {&nn, &nbk, &up, &alpha, &A, &lda, &Dinv, &B, &flags, &err, &status, &limit};
+  void* args[] = {&nn, &nbk, &up,  &alpha,  &A,    &lda,  &Dinv,
+                  &B,  &flags, &err, &status, &info, &limit};
   ATLG_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&trsv_sf_kernel<S>), dim3(G),
                                       dim3(SV_T), args, 0, s));
 }
@@ -477,7 +482,8 @@ void tri_inverse_blocks(hipStream_t s, long na, const S* A, long lda, int ta, in
 
 template <class S>
 void trsm(hipStream_t s, int side, int uplo, int ta, int diag, long M, long N, S alpha,
-          const S* A, long lda, S* B, long ldb, const int* skip, const S* dinv, int dinv_trans) {
+          const S* A, long lda, S* B, long ldb, const int* skip, const S* dinv, int dinv_trans,
+          WaitReport rep) {
   if (M <= 0 || N <= 0) return;
   if (alpha == S(0)) {
     scale<S>(s, M, N, S(0), B, ldb, 0, skip);
@@ -495,6 +501,7 @@ void trsm(hipStream_t s, int side, int uplo, int ta, int diag, long M, long N, S
   c.M = M;
   c.N = N;
   c.skip = skip;
+  c.rep = rep;
   c.fixed = nullptr;
   const long na = c.left ? M : N;
   c.dtrans = dinv ? (dinv_trans ? kTrans : kNoTrans) : kNoTrans;
@@ -507,7 +514,7 @@ void trsm(hipStream_t s, int side, int uplo, int ta, int diag, long M, long N, S
     c.Dinv = D;
   }
   if (c.left && !c.trans && c.dtrans == kNoTrans && !skip && N == 1 && na >= kTrsvMin<S>) {
-    trsv_long<S>(s, c.lower_eff, na, alpha, A, lda, c.Dinv, B);
+    trsv_long<S>(s, c.lower_eff, na, alpha, A, lda, c.Dinv, B, rep);
     return;
   }
   solve(c, 0, na, alpha);
@@ -559,9 +566,9 @@ template void tri_inverse_blocks<double>(hipStream_t, long, const double*, long,
 template void tri_inverse_blocks<float>(hipStream_t, long, const float*, long, int, int, int,
                                         float*, const int*);
 template void trsm<double>(hipStream_t, int, int, int, int, long, long, double, const double*,
-                           long, double*, long, const int*, const double*, int);
+                           long, double*, long, const int*, const double*, int, WaitReport);
 template void trsm<float>(hipStream_t, int, int, int, int, long, long, float, const float*, long,
-                          float*, long, const int*, const float*, int);
+                          float*, long, const int*, const float*, int, WaitReport);
 
 }  // namespace atlg
 

@@ -89,8 +89,8 @@ template <class S, bool TR, bool FOLD>
 __global__ void __launch_bounds__(kTxThreads)
 trsv_xcd(int n, int nb, int nrhs, int gpad, int upper, S alpha, const S* __restrict__ A, long lda,
          const S* __restrict__ Dinv, int dtrans, S* __restrict__ B, long bi, long bj,
-         tx_word* __restrict__ xb, int* __restrict__ err, int* __restrict__ status, long limit,
-         const int* __restrict__ skip) {
+         tx_word* __restrict__ xb, int* __restrict__ err, int* __restrict__ status, int* info,
+         long limit, const int* skip) {  // (info may be skip)
   typedef TriMfma<S> M;
   typedef typename M::acc_t acc_t;
   const int grp = blockIdx.x % gpad, li = blockIdx.x / gpad;
@@ -231,7 +231,10 @@ trsv_xcd(int n, int nb, int nrhs, int gpad, int upper, S alpha, const S* __restr
     }
   }
   if (!ok) {
-    if (t == 0) atomicOr(status, ATLG_FAIL_TRSV);
+    if (t == 0) {
+      atomicOr(status, ATLG_FAIL_TRSV);
+      if (info) *info = INT_MIN;
+    }
     return;
   }
   tx_word* out = xb + (size_t)li * kTxBlock + row;
@@ -274,12 +277,13 @@ static_assert(kTxFixedBytes + 256 == kNoAllocTxBytes, "fixed exchange area");
 template <class S>
 bool trsv_one_launch(hipStream_t s, bool lower, bool tr, long n, long nrhs, S alpha, const S* A,
                      long lda, const S* Dinv, int dtrans, S* B, long bi, long bj, const int* skip,
-                     unsigned char* fixed) {
+                     const WaitReport& rep, unsigned char* fixed) {
   const int nb = (int)((n + kTxB - 1) / kTxB);
   const int groups = (int)((nrhs + kTxCols - 1) / kTxCols);
   const long words = (long)groups * nb * kTxBlock;
   tx_word* xb = static_cast<tx_word*>(
-      fixed ? fixed : scratch_in_capture(s, kSlotTrsv, 256 + sizeof(tx_word) * words));
+      fixed ? fixed
+            : scratch_in_capture(s, kSlotTrsv, 256 + sizeof(tx_word) * words, !rep.status));
   if (!xb) return false;
   int* err = reinterpret_cast<int*>(xb);
   xb += 256 / sizeof(tx_word);
@@ -289,14 +293,16 @@ bool trsv_one_launch(hipStream_t s, bool lower, bool tr, long n, long nrhs, S al
   const int gpad = (groups + kTxGroups - 1) / kTxGroups * kTxGroups;
   const dim3 grid(gpad * (nb - 1) + groups), block(kTxThreads);
   const int up = lower ? 0 : 1;
-  int* status = fixed ? reinterpret_cast<int*>(fixed + kTxFixedBytes) : status_word(s);
+  int* status = fixed        ? reinterpret_cast<int*>(fixed + kTxFixedBytes)
+                : rep.status ? rep.status
+                             : status_word(s);
   const long limit = wait_limit(kSvSpin);
   // more groups than XCDs: throughput counts, and folding adds to the products
   const bool fold = groups <= kTxGroups;
   const auto fn = tr ? (fold ? trsv_xcd<S, true, true> : trsv_xcd<S, true, false>)
                      : (fold ? trsv_xcd<S, false, true> : trsv_xcd<S, false, false>);
   hipLaunchKernelGGL(fn, grid, block, 0, s, (int)n, nb, (int)nrhs, gpad, up, alpha, A, lda, Dinv,
-                     dtrans, B, bi, bj, xb, err, status, limit, skip);
+                     dtrans, B, bi, bj, xb, err, status, rep.info, limit, skip);
   ATLG_LAUNCHED();
   return true;
 }
