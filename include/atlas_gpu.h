@@ -61,7 +61,13 @@ void atlg_set_xerbla_hook(void (*hook)(int p, const char *rout,
  *   synchronizes) returns ATLG_EWAIT instead.
  * atlg_set_wait_limit: polls (each one memory round trip) before a wait
  *   gives up, process-wide; polls <= 0 restores the defaults (2^20 for the
- *   panel, 2^22 for the solve, far beyond any wait of a resident grid). */
+ *   panel, 2^22 for the solve, far beyond any wait of a resident grid).
+ * atlg_set_gather_limit: a getrf panel of up to 8192 rows needs its
+ *   workgroups on one XCD at the same time; where other work keeps them from
+ *   starting, one of them factors the panel alone, slower, with the same
+ *   pivots.  polls: how long they wait for each other first, process-wide; 0
+ *   restores the default (2^13, a few ms), negative: not at all, every such
+ *   panel is factored alone. */
 #define ATLG_EWAIT (-1001)
 #define ATLG_FAIL_PANEL 1
 #define ATLG_FAIL_TRSV 2
@@ -69,6 +75,7 @@ int atlg_stream_status(atlg_stream_t stream, int *status);
 void atlg_set_failure_hook(void (*hook)(const char *rout, int bits,
                                         const char *msg));
 void atlg_set_wait_limit(long polls);
+void atlg_set_gather_limit(long polls);
 
 /* C <- alpha*op(A)*op(B) + beta*C; beta == 0 never reads C. */
 int atlg_dgemm(int TA, int TB, long M, long N, long K, double alpha,

@@ -101,6 +101,7 @@ _SIGS = {
     "atlg_stream_status": (_i, [_v, _ip]),
     "atlg_set_failure_hook": (None, [FAILURE_HOOK]),
     "atlg_set_wait_limit": (None, [_l]),
+    "atlg_set_gather_limit": (None, [_l]),
     "atlg_dgemm": (_i, [_i, _i, _l, _l, _l, _d, _v, _l, _v, _l, _d, _v, _l, _v]),
     "atlg_dsyrk": (_i, [_i, _i, _l, _l, _d, _v, _l, _d, _v, _l, _v]),
     "atlg_dtrsm": (_i, [_i, _i, _i, _i, _l, _l, _d, _v, _l, _v, _l, _v]),
@@ -202,6 +203,12 @@ def _host(fn, *args):
 def set_wait_limit(polls):
     """Polls before a bounded wait gives up (<= 0: the defaults)."""
     lib().atlg_set_wait_limit(int(polls))
+
+
+def set_gather_limit(polls):
+    """Polls before an LU panel is left to one workgroup (0: the default,
+    negative: always)."""
+    lib().atlg_set_gather_limit(int(polls))
 
 
 def stream_status(stream=None):

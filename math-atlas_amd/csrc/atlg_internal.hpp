@@ -73,12 +73,6 @@ bool split_streams(int cus, hipStream_t caller, hipStream_t* small, hipStream_t*
 // Compute units that work queued on the stream runs on: a split_streams()
 // stream's share, else the device's.
 int stream_units(hipStream_t s);
-// Whether ordinary launches on this stream may hold workgroups that wait for
-// each other on one XCD (at most 16 compute units of its 32).  Two such
-// launches at once always fit, more might each hold units the others need:
-// one stream per device gets the right, the first to ask, beside the
-// look-ahead's reserved units; others launch cooperatively or go without.
-bool gang_stream(hipStream_t s);
 // Held by a look-ahead driver while it queues work on the shared auxiliary
 // streams and events above, so that calls from several host threads do not
 // interleave their event records and waits (the device work of successive
@@ -130,6 +124,9 @@ int take_status(hipStream_t s);
 // Poll bound of the bounded waits: the process-wide value set by
 // atlg_set_wait_limit, or `dflt` when none is set.
 long wait_limit(long dflt);
+// Polls before the workgroups of an LU panel stop waiting for each other's
+// start: the value of atlg_set_gather_limit, or `dflt` when that is 0.
+long gather_limit(long dflt);
 // Reports a failure of a host entry point through the failure hook
 // (atlg_set_failure_hook); the default hook prints and aborts.
 void report_failure(const char* rout, int status, const char* msg);

@@ -39,7 +39,10 @@
 // ATL_sgetrf instance of the same ATLAS source).
 #include <hip/hip_runtime.h>
 
+#include <unistd.h>
+
 #include <algorithm>
+#include <atomic>
 #include <cfloat>
 #include <climits>
 #include <limits>
@@ -1424,7 +1427,8 @@ struct LU {
   int mb_g[2] = {0, 0};       // grid of each mailbox's last user (0: clean)
   XpBox* box = nullptr;       // exchange areas of the XCD panel
   int box_par = 0;            // the one its next multi-workgroup launch uses
-  bool gang = false;          // the stream may launch XCD panels without a cooperative launch
+  int xcd = 0;                // the XCD of its panels of several workgroups
+  long gather = kXpGather;    // polls before such a panel is left to one workgroup
   int xcd_units = 32;         // compute units of one XCD the panel may count on
 };
 
@@ -1507,25 +1511,11 @@ template <class S>
 void launch_xcd(LU<S>& f, int M, int w, int off, int G, int* lst) {
   const int per = (M + G - 1) / G, par = f.box_par;
   if (G > 1) f.box_par ^= 1;
-  const dim3 grid(8 * (G - 1) + 1), block(64 * ((per + 63) / 64));
-  S* P = at(f, off, off);
-  if (G == 1 || !f.coop || f.gang) {
-    hipLaunchKernelGGL(panel_xcd<S>, grid, block, 0, f.s, M, w, off, P, f.lda, f.ipiv, f.dinfo,
-                       f.box, par, G, lst, f.status, f.limit);
-    ATLG_LAUNCHED();
-    return;
-  }
-  // Outside the look-ahead's reserved units, panels of several callers'
-  // streams could hold an XCD's units while each waits for more of its own
-  // workgroups: cooperative launches do not overlap each other (they cost
-  // about 40 us each, N=1500: 5.7 against 4.4 ms, so the device's gang
-  // stream goes without).
-  int p = par, g = G;
-  long lda = f.lda;
-  void* args[] = {&M,     &w, &off, &P, &lda,      &f.ipiv, &f.dinfo,
-                  &f.box, &p, &g,   &lst, &f.status, &f.limit};
-  ATLG_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&panel_xcd<S>), grid, block,
-                                      args, 0, f.s));
+  const int xcd = G > 1 ? f.xcd : 0;
+  const dim3 grid(8 * (G - 1) + xcd + 1), block(64 * ((per + 63) / 64));
+  hipLaunchKernelGGL(panel_xcd<S>, grid, block, 0, f.s, M, w, off, at(f, off, off), f.lda, f.ipiv,
+                     f.dinfo, f.box, par, G, xcd, lst, f.status, f.limit, f.gather);
+  ATLG_LAUNCHED();
 }
 
 // Factors the leaf panel at (off, off): m rows, w columns, and applies its
@@ -1749,6 +1739,9 @@ void init_lu(LU<S>& f, hipStream_t s, long M, long N, S* A, long lda, int* ipiv,
   hipLaunchKernelGGL(xp_init, dim3(2), dim3(256), 0, s, f.box);
   ATLG_LAUNCHED();
   f.box_par = 0;
+  static std::atomic<unsigned> turn{(unsigned)getpid()};  // (other processes start elsewhere)
+  f.xcd = (int)(turn.fetch_add(1, std::memory_order_relaxed) & 7u);
+  f.gather = gather_limit(kXpGather);
   const long nblk = (std::min(M, N) + kTrsmNB - 1) / kTrsmNB;
   f.Winv = static_cast<S*>(
       scratch(s, kSlotFactInv, sizeof(S) * std::max<long>(nblk, 1) * kTrsmNB * kTrsmNB));
@@ -1973,7 +1966,6 @@ void getrf(hipStream_t s, long M, long N, S* A, long lda, int* ipiv, int* dinfo,
   if (M == 0 || N == 0) return;
   LU<S> f;
   init_lu(f, s, M, N, A, lda, ipiv, dinfo, gemm_prec);
-  f.gang = gang_stream(s);
   f.status = status_word(s);
   f.limit = wait_limit(kSpinLimit);
   if (ATLG_LU_LOOKAHEAD && std::min(M, N) >= kLaMin)

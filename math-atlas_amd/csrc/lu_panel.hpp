@@ -30,7 +30,17 @@
 //    stop at the XCD's L2: an exchange of eight workgroups takes 840 cycles,
 //    against 1500 with agent-scope stores and 2000 across XCDs (one line per
 //    candidate, timed by itself).  The waits are bounded as panel_coop's are,
-//    so a device that dealt the workgroups otherwise would report a failure.
+//    so a device that dealt the workgroups otherwise would report a failure;
+//  * workgroups wait for each other only once all of a panel's are resident.
+//    A full one fills a compute unit and sixteen take half an XCD's, so panels
+//    of several streams or processes, or other kernels, may each hold units
+//    that the others need.  A workgroup therefore first counts itself in and
+//    waits, some milliseconds at most, for the others (xp_gather); when they
+//    do not come all give up at once, and the first factors the panel alone,
+//    in memory (xp_alone, 1.4 ms for 8192 rows).  The panel is unchanged until
+//    the end, so nothing is lost, and no launch needs to be cooperative (N=1500
+//    4.9 ms with that, 4.3 without; counting in costs a leaf 2 of its 80 us).  Successive
+//    factorizations take the XCDs in turn, to keep out of each other's way.
 //
 // A column takes 4000-4500 cycles (about 1.8 us), most of it the issue of
 // some 450 dependent instructions by one or two waves per SIMD.  M x 32 LU,
@@ -68,8 +78,13 @@ struct XpBox {
   xp_word cand[kXpW][kXpCand][kXpMaxG];  // word-major: xp_pick reads a word per lane
   xp_word trail[kXpW][kXpW];  // pivot row of column j: its entries right of the block
   int err;
-  int pad[15];
+  int here;  // workgroups that have arrived, and kXpAlone
+  int pad[14];
 };
+constexpr int kXpAlone = 1 << 16;
+// Polls (each a round trip to the L2) before a panel's workgroups stop waiting
+// for one of them to become resident.
+constexpr long kXpGather = 1L << 13;
 
 __device__ inline xp_word xp_ld(const xp_word* p) {
   return __hip_atomic_load(const_cast<xp_word*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -82,7 +97,10 @@ __device__ inline double xp_val(xp_word u) { return __longlong_as_double(static_
 __device__ inline void xp_clear(XpBox* m, int t, int nt) {
   for (int e = t; e < kXpW * kXpCand * kXpMaxG; e += nt) xp_st(&m->cand[0][0][0] + e, kXpSent);
   for (int e = t; e < kXpW * kXpW; e += nt) xp_st(&m->trail[0][0] + e, kXpSent);
-  if (t == 0) st_agent(&m->err, 0);
+  if (t == 0) {
+    st_agent(&m->err, 0);
+    __hip_atomic_store(&m->here, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
 }
 __global__ void xp_init(XpBox* m) {
   xp_clear(m + blockIdx.x, threadIdx.x, blockDim.x);
@@ -168,27 +186,117 @@ __device__ __forceinline__ int xp_pick(const XpWords& w, int n, int lane) {
   return __builtin_amdgcn_readfirstlane(__builtin_ctz(b | 0x10000u) & 15);
 }
 
+// Whether all G workgroups are resident; when they are not within `patience`
+// polls (negative: in any case) every one of them gets the same no.  (Atomics
+// that end at the XCD's L2, as the exchange's stores do.)
+__device__ bool xp_gather(XpBox* m, int G, long patience) {
+  if (patience < 0)
+    __hip_atomic_fetch_or(&m->here, kXpAlone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  for (long spins = 0;;) {
+    int v = ld_agent(&m->here);
+    if (v & kXpAlone) return false;
+    if (v == G) return true;
+    // (fails when one arrived meanwhile: at most G times)
+    if (++spins > patience &&
+        __hip_atomic_compare_exchange_strong(&m->here, &v, v | kXpAlone, __ATOMIC_RELAXED,
+                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
+      return false;
+  }
+}
+
+// The panel by one workgroup, column by column in memory.  slot: 32 words;
+// urow: w entries; pa, pb, zcol as panel_xcd fills them.  (Not inlined: it
+// would spill the panel's scalar registers.)
+template <class S>
+__device__ __attribute__((noinline)) void xp_alone(int M, int w, int off, S* P, long lda,
+                                                   xp_word* slot, S* urow, int* pa, int* pb,
+                                                   int* zcol) {
+  const int t = threadIdx.x, nt = blockDim.x, mn = min(M, w);
+#pragma unroll 1
+  for (int j = 0; j < mn; j++) {
+    S* cj = P + (size_t)j * lda;
+    S key = S(-2);
+    int p = INT_MAX;
+    for (int i = j + t; i < M; i += nt) {  // (ascending: the first of equal keys stays)
+      const S a = xp_key(__builtin_canonicalize(cj[i]));
+      if (a > key) {
+        key = a;
+        p = i;
+      }
+    }
+    S m = key;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = xp_max(m, __shfl_xor(m, o));
+    p = xp_wave_min(key == m ? p : INT_MAX);
+    if ((t & 63) == 0) {
+      slot[t >> 6] = xp_bits((double)m);
+      slot[16 + (t >> 6)] = (xp_word)(unsigned)p;
+    }
+    __syncthreads();
+    double best = -3.0;
+    p = j;
+    for (int q = 0; q < nt / 64; q++) {
+      const double k = xp_val(slot[q]);
+      const int c = static_cast<int>(slot[16 + q]);
+      if (k > best || (k == best && c < p)) {
+        best = k;
+        p = c;
+      }
+    }
+    if (t < w) {  // rows j and p change places
+      S* c = P + (size_t)t * lda;
+      const S x = c[j], u = c[p];
+      c[j] = u;
+      c[p] = x;
+      urow[t] = u;
+    }
+    __syncthreads();
+    const S piv = urow[j];
+    if (piv != S(0)) {
+      const bool small = !(fabs(piv) >= std::numeric_limits<S>::min());
+      const S up = !small ? S(1) : std::is_same<S, double>::value ? S(0x1p600) : S(0x1p100f);
+      const S ps = piv * up, rinv = S(1) / ps;
+      for (int i = j + 1 + t; i < M; i += nt) {
+        const S x = cj[i] * up;
+        S l = x * rinv;
+        if (small) l += (x - l * ps) * rinv;
+        cj[i] = l;
+#pragma unroll 4
+        for (int c = j + 1; c < w; c++) P[i + (size_t)c * lda] -= l * urow[c];
+      }
+    }
+    if (t == 0) {
+      pa[j] = off + j;
+      pb[j] = off + p;
+      if (piv == S(0) && *zcol < 0) *zcol = j;
+    }
+    __syncthreads();
+  }
+}
+
 // Factors the M x w (w <= 32) panel P, row 0 of which is absolute row `off`
 // on the matrix's diagonal; 32 columns of P span less than 2 GiB.  Outputs
-// as panel_coop's.  G workgroups of blockDim.x / 64 waves; grid
-// 8 (G - 1) + 1 (see above).
+// as panel_coop's.  G workgroups of blockDim.x / 64 waves on XCD `xcd`; grid
+// 8 (G - 1) + xcd + 1 (see above).
 template <class S>
 __global__ void __launch_bounds__(64 * kXpWaves)
 panel_xcd(int M, int w, int off, S* __restrict__ P, long lda, int* __restrict__ ipiv,
-          int* __restrict__ dinfo, XpBox* __restrict__ box, int par, int G,
-          int* __restrict__ list, int* __restrict__ status, long limit) {
+          int* __restrict__ dinfo, XpBox* __restrict__ box, int par, int G, int xcd,
+          int* __restrict__ list, int* __restrict__ status, long limit, long gather) {
   typedef TriMfma<S> Mf;
   typedef typename Mf::acc_t acc_t;
-  if (blockIdx.x & 7) return;
+  if ((blockIdx.x & 7) != xcd) return;
   __shared__ xp_word slot[2][kXpCand][16];  // the waves' candidates, word-major
   __shared__ S ubuf[4][kXpW];  // G == 1: trailing entries of the block's pivot rows
   __shared__ S l11[kXpWaves][4][4];  // each wave's copy of the block's pivot rows
   __shared__ int pa[kXpW], pb[kXpW];
-  __shared__ int sbad, zcol;
+  __shared__ int sbad, zcol, together;
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int NW = blockDim.x >> 6, g = blockIdx.x >> 3;
   const int n = lane & 15, k = lane >> 4;
   XpBox* mb = box + par;
+  if (G > 1 && t == 0)
+    __hip_atomic_fetch_add(&mb->here, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   if (G > 1) xp_clear(box + (par ^ 1), g * blockDim.x + t, G * blockDim.x);
   for (int e = t; e < 2 * kXpCand * 16; e += blockDim.x) (&slot[0][0][0])[e] = xp_bits(-3.0);
   if (t == 0) {
@@ -237,9 +345,16 @@ panel_xcd(int M, int w, int off, S* __restrict__ P, long lda, int* __restrict__ 
   bool bad = false;  // this wave gave up waiting (no further waits or updates)
   // every row is in registers before any workgroup can finish and store
   __builtin_amdgcn_s_waitcnt(0);
+  if (G > 1 && t == 0) together = xp_gather(mb, G, gather);
   __syncthreads();
+  const bool alone = G > 1 && !together;
+  if (alone) {
+    if (g > 0) return;
+    xp_alone(M, w, off, P, lda, &slot[0][0][0], &ubuf[0][0], pa, pb, &zcol);
+  }
+  const int held = alone ? 0 : mn;  // columns factored in registers
 #pragma unroll 1
-  for (int b = 0; 4 * b < mn; b++) {
+  for (int b = 0; 4 * b < held; b++) {
     const int jb = 4 * b, nq = min(4, mn - jb);
     // the block's entries of this lane's rows, and back below: selects by the
     // uniform b (a switch makes the compiler copy whole accumulator tuples)
@@ -407,7 +522,7 @@ panel_xcd(int M, int w, int off, S* __restrict__ P, long lda, int* __restrict__ 
       }
 #pragma unroll
       for (int rt = 0; rt < RT; rt++) pos[rt] = pos[rt] == j ? p : (pos[rt] == p ? j : pos[rt]);
-      if (blockIdx.x == 0 && t == 0) {
+      if (g == 0 && t == 0) {
         pa[j] = off + j;
         pb[j] = off + p;
         if (piv == S(0) && zcol < 0) zcol = j;
@@ -521,7 +636,7 @@ panel_xcd(int M, int w, int off, S* __restrict__ P, long lda, int* __restrict__ 
   }
 #pragma unroll
   for (int rt = 0; rt < RT; rt++)
-    if (row0 + 16 * rt < M) {
+    if (!alone && row0 + 16 * rt < M) {
       const unsigned vo = static_cast<unsigned>(pos[rt] * (int)sizeof(S) + k * cstride);
       if (w == kXpW) {
 #pragma unroll
@@ -538,13 +653,13 @@ panel_xcd(int M, int w, int off, S* __restrict__ P, long lda, int* __restrict__ 
       *dinfo = INT_MIN;
       atomicOr(status, ATLG_FAIL_PANEL);
     }
-    if (blockIdx.x == 0) {
+    if (g == 0) {
       if (t < mn) ipiv[off + t] = off + t;  // identity: later users stay in bounds
       if (t == 0) list[0] = 0;              // apply no interchanges
     }
     return;
   }
-  if (blockIdx.x == 0) {
+  if (g == 0) {
     if (t < mn) ipiv[off + t] = pb[t];
     if (t == 0 && zcol >= 0 && *dinfo == 0) *dinfo = off + zcol + 1;
     if (t < 64) compose_swaps_wave(pa, pb, mn, list);

@@ -35,7 +35,7 @@ struct SlotBuf {
 };
 std::map<std::pair<hipStream_t, int>, SlotBuf> g_slots;
 std::map<hipStream_t, int*> g_status;  // stream -> failure word
-std::atomic<long> g_wait_limit{0};
+std::atomic<long> g_wait_limit{0}, g_gather_limit{0};
 void (*g_failure_hook)(const char*, int, const char*) = nullptr;
 
 // Orderly release of everything the runtime created: run once at process
@@ -80,7 +80,6 @@ struct Aux {
 };
 std::map<int, Aux> g_aux;
 std::map<hipStream_t, int> g_units;  // CU-masked stream -> its compute units
-std::map<int, hipStream_t> g_gang;   // device -> the stream of gang_stream()
 Aux& aux_for_device() {
   int dev = 0;
   ATLG_HIP(hipGetDevice(&dev));
@@ -237,13 +236,6 @@ int stream_units(hipStream_t s) {
   return n;
 }
 
-bool gang_stream(hipStream_t s) {
-  int dev = 0;
-  ATLG_HIP(hipGetDevice(&dev));
-  std::lock_guard<std::mutex> lk(g_mu);
-  return g_gang.emplace(dev, s).first->second == s;
-}
-
 void* scratch(hipStream_t s, Slot slot, size_t bytes) {
   if (bytes == 0) bytes = 256;
   std::lock_guard<std::mutex> lk(g_mu);
@@ -325,6 +317,11 @@ int take_status(hipStream_t s) {
 long wait_limit(long dflt) {
   const long v = g_wait_limit.load();
   return v > 0 ? v : dflt;
+}
+
+long gather_limit(long dflt) {
+  const long v = g_gather_limit.load();
+  return v != 0 ? v : dflt;
 }
 
 void report_failure(const char* rout, int status, const char* msg) {
@@ -415,6 +412,7 @@ void atlg_set_failure_hook(void (*hook)(const char*, int, const char*)) {
 }
 
 void atlg_set_wait_limit(long polls) { g_wait_limit.store(polls); }
+void atlg_set_gather_limit(long polls) { g_gather_limit.store(polls); }
 
 int atlg_dgemm(int TA, int TB, long M, long N, long K, double alpha,
                const double* A, long lda, const double* B, long ldb,
