@@ -1829,10 +1829,11 @@ void getrf_lookahead(LU<S>& f0) {
   const int panel_cus = la_panel_cus(f0.M);
   const bool split = panel_cus > 0 && split_streams(panel_cus, caller, &sp, &sg);
   if (split) {
-    // after the last look-ahead too, which may have run on another split:
-    // its panels and these would share compute units
-    ATLG_HIP(hipStreamWaitEvent(sg, aux_event(3), 0));
-    ATLG_HIP(hipStreamWaitEvent(sp, aux_event(3), 0));
+    // after the last look-ahead LU too, which may have run on another pair:
+    // its panels and these would share compute units (an event of its own: a
+    // Cholesky's end says nothing about the LU before it)
+    ATLG_HIP(hipStreamWaitEvent(sg, aux_event(7), 0));
+    ATLG_HIP(hipStreamWaitEvent(sp, aux_event(7), 0));
     ATLG_HIP(hipEventRecord(aux_event(2), caller));
     ATLG_HIP(hipStreamWaitEvent(sg, aux_event(2), 0));
     ATLG_HIP(hipStreamWaitEvent(sp, aux_event(2), 0));
@@ -1952,8 +1953,8 @@ void getrf_lookahead(LU<S>& f0) {
   if (chunk_pending) ATLG_HIP(hipStreamWaitEvent(s0, e_chunk, 0));
   apply_deferred_left(f0, kLaNB, mn);
   if (split) {  // every panel and panel-side update was joined into s0 above
-    ATLG_HIP(hipEventRecord(aux_event(3), s0));
-    ATLG_HIP(hipStreamWaitEvent(caller, aux_event(3), 0));
+    ATLG_HIP(hipEventRecord(aux_event(7), s0));
+    ATLG_HIP(hipStreamWaitEvent(caller, aux_event(7), 0));
     f0.s = caller;
   }
 }

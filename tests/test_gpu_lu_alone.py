@@ -164,3 +164,37 @@ def test_streams_together(G):
         for w, x in zip(want, got):
             assert np.array_equal(w, x)
         assert torch.equal(ch0, ch)
+
+
+def test_lookaheads_in_turn(G):
+    # look-ahead LUs of both widths of reserved units (order 12000: 64, order
+    # 2304: 128), whose panels would share units, run one after the other, also
+    # with a Cholesky between them
+    import torch
+    dev = "cuda"
+    g = torch.Generator(device=dev)
+    g.manual_seed(2)
+    big, small = (torch.rand((n, n), generator=g, device=dev, dtype=torch.float64) * 2 - 1
+                  for n in (12000, 2304))
+    spd = torch.eye(2304, dtype=torch.float64, device=dev) * 4.0 + 1.0 / 2304
+    piv = [torch.zeros(n, dtype=torch.int32, device=dev) for n in (12000, 2304)]
+    info = torch.zeros(3, dtype=torch.int32, device=dev)
+    s = [torch.cuda.Stream() for _ in range(3)]
+    end = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    for _ in range(2):  # the first pass makes streams and workspaces
+        a, b, c = big.clone(), small.clone(), spd.clone()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s[0]):
+            G.dgetrf(12000, 12000, a, 12000, piv[0], info)
+            end[0].record()
+        with torch.cuda.stream(s[1]):
+            G.dpotrf(O.Lower, 2304, c, 2304, info[1:])
+        with torch.cuda.stream(s[2]):
+            G.dgetrf(2304, 2304, b, 2304, piv[1], info[2:])
+            end[1].record()
+        torch.cuda.synchronize()
+    assert (info == 0).all()
+    for x in s:
+        with torch.cuda.stream(x):
+            G.check_stream()
+    assert end[0].elapsed_time(end[1]) > 0
