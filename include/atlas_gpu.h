@@ -13,7 +13,12 @@
  * Return codes: 0 on success; -i when the i-th argument is illegal (nothing
  * is queued); ATLG_EHIP when a HIP call failed (atlg_last_error() has the
  * message).  LAPACK info values are written to DEVICE memory (*dinfo), so
- * no call synchronizes.  ipiv arrays live in device memory as int32, 0-based
+ * no call synchronizes for its results.  (Two exceptions once each: a call
+ * that needs more workspace than those before it on its stream waits for the
+ * stream to replace it, and the first getrf and potrf of order >= 2048 on a
+ * stream spend some 10 ms of host time, at most 60, timing which of the
+ * library's own streams go with it; that waits at most 10 ms for queued work,
+ * and a later call tries again.)  ipiv arrays live in device memory as int32, 0-based
  * absolute row indices, as in ATLAS's C interface.
  *
  * Streams: `stream` is a hipStream_t passed as void*; NULL is HIP's null

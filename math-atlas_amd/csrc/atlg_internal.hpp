@@ -67,8 +67,10 @@ hipEvent_t aux_event(int i);  // i = 0 .. kAuxEvents-1
 // first `cus` units, *large the rest (hipExtStreamCreateWithCUMask); false
 // when cus <= 0 or the masked streams are unavailable.  `caller` is the
 // stream that will wait for them: its first call makes pairs and times which
-// one its wait does not slow down (some 10 ms, synchronizing these streams;
-// under capture nothing is timed).  Called with aux_lock() held.
+// one its wait does not slow down (some 10 ms, at most 60; nothing under
+// capture, nor where that stream stays busy).  The exchange area of the solves
+// that these streams will run is there, so that no growth of it synchronizes
+// them.  Called with aux_lock() held.
 bool split_streams(int cus, hipStream_t caller, hipStream_t* small, hipStream_t* large);
 // Compute units that work queued on the stream runs on: a split_streams()
 // stream's share, else the device's.

@@ -75,6 +75,7 @@ struct Aux {
   struct Split {
     std::vector<std::pair<hipStream_t, hipStream_t>> pairs;
     std::map<hipStream_t, int> choice;
+    std::map<hipStream_t, int> tries;  // calls that found their stream busy
   };
   std::map<int, Split> split;
 };
@@ -110,9 +111,18 @@ hipEvent_t aux_event(int i) { return aux_for_device().ev[(unsigned)i % kAuxEvent
 // asked, so it is timed, once per caller's stream: a chain of empty kernels
 // across the pair with the caller's stream waiting for it, against the same
 // chain without; a pair that slows down is passed over for a new one.
+//
+// The calls are asynchronous, and what is queued on a caller's stream may wait
+// for something that its thread does next, so nothing here waits without a
+// deadline: where the streams are not idle soon, the call goes on with the
+// first pair and a later one tries again.
 namespace {
 constexpr int kProbeChain = 24;      // kernels on each stream of the pair
 constexpr int kMaxPairs = 4;         // pairs made per unit count
+constexpr int kMaxProbed = 16;       // streams timed per unit count: each costs some 10 ms
+constexpr int kMaxTries = 3;         // calls that may wait for an idle stream
+constexpr auto kProbeIdle = std::chrono::milliseconds(10);  // that wait
+constexpr auto kProbeAll = std::chrono::milliseconds(60);   // and all of a call's timing
 constexpr double kProbeSlow = 1.35;  // waiting caller / free caller (seen: 1.07-1.14 or 1.60-1.68)
 
 __global__ void probe_empty() {}
@@ -122,11 +132,31 @@ __global__ void probe_hold() {
   for (int i = 0; i < 9000; i++) __builtin_amdgcn_s_sleep(2);
 }
 
-// Seconds from the first launch until the caller's stream is idle again.
-double probe(hipStream_t small, hipStream_t large, hipStream_t caller, const Aux& a, bool waiting) {
-  ATLG_HIP(hipStreamSynchronize(caller));
-  ATLG_HIP(hipStreamSynchronize(small));
-  ATLG_HIP(hipStreamSynchronize(large));
+typedef std::chrono::steady_clock::time_point TimePoint;
+
+// Whether the event is done before `until`.
+bool done_by(TimePoint until, hipEvent_t ev) {
+  for (;;) {
+    const hipError_t e = hipEventQuery(ev);
+    if (e == hipSuccess) return true;
+    (void)hipGetLastError();
+    if (e != hipErrorNotReady || std::chrono::steady_clock::now() > until) return false;
+  }
+}
+// Whether what is queued on the streams is done before `until`.  (By events: a
+// query of the null stream queues work on it.)
+bool idle_by(TimePoint until, const Aux& a, hipStream_t small, hipStream_t large,
+             hipStream_t caller) {
+  const hipStream_t s[3] = {caller, small, large};
+  for (int i = 0; i < 3; i++) ATLG_HIP(hipEventRecord(a.ev[4 + i], s[i]));
+  return done_by(until, a.ev[4]) && done_by(until, a.ev[5]) && done_by(until, a.ev[6]);
+}
+
+// Seconds from the first launch on idle streams until the caller's stream is
+// idle again; negative when that takes too long.
+double probe(hipStream_t small, hipStream_t large, hipStream_t caller, const Aux& a, bool waiting,
+             TimePoint until) {
+  if (!idle_by(until, a, small, large, caller)) return -1.0;
   const auto t0 = std::chrono::steady_clock::now();
   hipLaunchKernelGGL(probe_hold, dim3(1), dim3(64), 0, small);
   for (int i = 0; i < kProbeChain; i++)
@@ -139,10 +169,9 @@ double probe(hipStream_t small, hipStream_t large, hipStream_t caller, const Aux
   ATLG_HIP(hipEventRecord(a.ev[1], large));
   if (waiting) {
     ATLG_HIP(hipStreamWaitEvent(caller, a.ev[1], 0));
-    ATLG_HIP(hipStreamSynchronize(caller));
-  } else {
-    ATLG_HIP(hipStreamSynchronize(large));
+    ATLG_HIP(hipEventRecord(a.ev[2], caller));
   }
+  if (!done_by(until, a.ev[waiting ? 2 : 1])) return -1.0;
   return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
 
@@ -168,6 +197,18 @@ bool make_pair(int cus, std::pair<hipStream_t, hipStream_t>* out) {
   *out = {p[0], p[1]};
   return true;
 }
+
+// The pair as split_streams() returns it.
+bool give_pair(const std::pair<hipStream_t, hipStream_t>& p, bool capturing, hipStream_t* small,
+               hipStream_t* large) {
+  if (!capturing) {
+    (void)scratch(p.first, kSlotTrsv, kNoAllocTxBytes);
+    (void)scratch(p.second, kSlotTrsv, kNoAllocTxBytes);
+  }
+  *small = p.first;
+  *large = p.second;
+  return true;
+}
 }  // namespace
 
 bool split_streams(int cus, hipStream_t caller, hipStream_t* small, hipStream_t* large) {
@@ -181,12 +222,23 @@ bool split_streams(int cus, hipStream_t caller, hipStream_t* small, hipStream_t*
   int pick = 0;
   auto it = sp.choice.find(caller);
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  // (an error: some other capture is open)
+  const bool capturing =
+      hipStreamIsCapturing(caller, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+  if (capturing) (void)hipGetLastError();
   if (it != sp.choice.end()) {
     pick = it->second;
-  } else if (hipStreamIsCapturing(caller, &cap) == hipSuccess &&
-             cap == hipStreamCaptureStatusNone) {  // (an error: some other capture is open)
+  } else if (!capturing) {
+    const auto now = std::chrono::steady_clock::now();
+    bool timed = (int)sp.choice.size() < kMaxProbed;
+    if (timed) {
+      const auto& p = sp.pairs[0];
+      timed = idle_by(now + kProbeIdle, a, p.first, p.second, caller);
+      if (!timed && ++sp.tries[caller] < kMaxTries)  // a later call tries again
+        return give_pair(p, false, small, large);
+    }
     double best = 0.0;
-    for (int i = 0; i < kMaxPairs; i++) {
+    for (int i = 0; i < kMaxPairs && timed; i++) {
       if (i == (int)sp.pairs.size()) {
         std::pair<hipStream_t, hipStream_t> p;
         if (!make_pair(cus, &p)) break;
@@ -195,12 +247,14 @@ bool split_streams(int cus, hipStream_t caller, hipStream_t* small, hipStream_t*
       const auto& p = sp.pairs[i];
       // the first round also warms the streams up; the faster of two counts
       double wait = 0.0, free = 0.0;
-      for (int r = 0; r < 3; r++) {
-        const double f = probe(p.first, p.second, caller, a, false);
-        const double w = probe(p.first, p.second, caller, a, true);
+      for (int r = 0; r < 3 && timed; r++) {
+        const double f = probe(p.first, p.second, caller, a, false, now + kProbeAll);
+        const double w = f < 0.0 ? f : probe(p.first, p.second, caller, a, true, now + kProbeAll);
+        timed = w >= 0.0;
         if (r == 1 || (r > 1 && f < free)) free = f;
         if (r == 1 || (r > 1 && w < wait)) wait = w;
       }
+      if (!timed) break;
       const double slow = wait / free;
       if (i == 0 || slow < best) {
         best = slow;
@@ -208,14 +262,12 @@ bool split_streams(int cus, hipStream_t caller, hipStream_t* small, hipStream_t*
       }
       if (slow < kProbeSlow) break;
     }
-    if (sp.choice.size() > 64) sp.choice.clear();  // streams come and go
+    sp.tries.erase(caller);
+    if (sp.tries.size() >= 1024) sp.tries.clear();
+    if (sp.choice.size() >= 1024) sp.choice.clear();  // streams come and go
     sp.choice[caller] = pick;
-  } else {
-    (void)hipGetLastError();
   }
-  *small = sp.pairs[pick].first;
-  *large = sp.pairs[pick].second;
-  return true;
+  return give_pair(sp.pairs[pick], capturing, small, large);
 }
 
 int stream_units(hipStream_t s) {
@@ -284,16 +336,15 @@ int* status_word(hipStream_t s) {
   int*& w = g_status[s];
   if (!w) {
     int* p = nullptr;
-    hipError_t e = hipMalloc(&p, 256);
-    if (e == hipSuccess) e = hipMemset(p, 0, 256);
+    const hipError_t e = hipMalloc(&p, 256);
     if (e != hipSuccess) {
       (void)hipGetLastError();
-      if (p) (void)hipFree(p);
       g_status.erase(s);
       throw HipFailure{std::string("failure word: ") + hipGetErrorString(e)};
     }
     w = p;
     arm_teardown();
+    set_int(s, p, 0);  // (a hipMemset would wait for other streams' work)
   }
   return w;
 }
