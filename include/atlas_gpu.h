@@ -110,7 +110,8 @@ int atlg_dtrsm(int Side, int Uplo, int TA, int Diag, long M, long N,
  * side above order 4096 takes the blocked solve here, not atlg_dtrsm's
  * sync-free one, so results agree with atlg_dtrsm to rounding, bit for bit
  * when NRHS > 4 or the order is below 1024.  A wait that fails is reported
- * as atlg_dtrsm's is. */
+ * as atlg_dtrsm's is, to its own stream alone (a process's streams past the
+ * first 1023 that call this entry share one report). */
 #define ATLG_ESIZE (-1002)
 int atlg_dtrsm_noalloc(int Side, int Uplo, int TA, int Diag, long M, long N,
                        double alpha, const double *A, long lda, double *B,

@@ -199,23 +199,26 @@ void trsm(hipStream_t s, int side, int uplo, int ta, int diag, long M, long N, S
           const S* dinv = nullptr, int dinv_trans = 0, WaitReport rep = {});
 
 // trsm() without allocation: the diagonal-block inverses, the exchange area
-// of the one-launch solves and their failure word live in a file-scope device
+// of the one-launch solves and their failure words live in a file-scope device
 // array sized for op(A) of order <= kNoAllocMaxOrder (one copy per device,
 // shared by every call on it, so calls that overlap on one device race).
 // noalloc_scratch() resolves the array's address on the current device (once
-// per device), noalloc_status() that of the failure word, or nullptr where no
-// solve has used it.
+// per device).  noalloc_word(): the stream's failure word there, so that
+// nobody takes another stream's; nullptr for a stream that has no such solve,
+// unless `make`.  (The streams past the first kNoAllocWords - 1 share the last
+// word.)
 constexpr long kNoAllocMaxOrder = 8192;
 constexpr size_t kNoAllocInvBytes =
     (size_t)(kNoAllocMaxOrder / kTrsmNB) * kTrsmNB * kTrsmNB * sizeof(double);
 constexpr size_t kNoAllocTxBlocks = 3072;  // 64 x 16 words each
-constexpr size_t kNoAllocTxBytes = 512 + kNoAllocTxBlocks * 64 * 16 * 8;
+constexpr size_t kNoAllocWords = 1024;     // failure words
+constexpr size_t kNoAllocTxBytes = 256 + kNoAllocTxBlocks * 64 * 16 * 8 + 4 * kNoAllocWords;
 constexpr size_t kNoAllocBytes = kNoAllocInvBytes + kNoAllocTxBytes;
 template <class S>
 void trsm_noalloc(hipStream_t s, int side, int uplo, int ta, int diag, long M, long N, S alpha,
                   const S* A, long lda, S* B, long ldb);
 void* noalloc_scratch();
-int* noalloc_status();
+int* noalloc_word(hipStream_t s, bool make);
 
 template <class S>
 void laswp(hipStream_t s, long N, S* A, long lda, int K1, int K2, const int* ipiv, int inci);

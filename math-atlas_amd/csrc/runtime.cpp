@@ -352,7 +352,7 @@ int* status_word(hipStream_t s) {
 int take_status(hipStream_t s) {
   int* w = status_word(s);
   int v = 0;
-  int* const words[2] = {w, noalloc_status()};  // and that of the allocation-free solves
+  int* const words[2] = {w, noalloc_word(s, false)};  // and of its allocation-free solves
   int got[2] = {0, 0};
   for (int i = 0; i < 2; i++)
     if (words[i])

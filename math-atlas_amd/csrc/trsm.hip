@@ -18,8 +18,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <climits>
+#include <map>
 #include <mutex>
 #include <type_traits>
 
@@ -520,13 +520,10 @@ void trsm(hipStream_t s, int side, int uplo, int ta, int diag, long M, long N, S
   solve(c, 0, na, alpha);
 }
 
-void* noalloc_scratch();
-void noalloc_used();
-
 // The allocation-free form: the diagonal-block inverses go to the file-scope
 // device array (at most kNoAllocMaxOrder / kTrsmNB blocks), and so does the
-// exchange area of the one-launch solves; the solve is otherwise trsm()'s
-// without its sync-free launch for one right-hand side.
+// exchange area of the one-launch solves and their failure words; the solve is
+// otherwise trsm()'s without its sync-free launch for one right-hand side.
 template <class S>
 void trsm_noalloc(hipStream_t s, int side, int uplo, int ta, int diag, long M, long N, S alpha,
                   const S* A, long lda, S* B, long ldb) {
@@ -552,7 +549,7 @@ void trsm_noalloc(hipStream_t s, int side, int uplo, int ta, int diag, long M, l
   c.N = N;
   c.skip = nullptr;
   c.fixed = static_cast<unsigned char*>(noalloc_scratch()) + kNoAllocInvBytes;
-  noalloc_used();
+  c.rep.status = noalloc_word(s, true);
   c.Dinv = D;
   c.dtrans = kNoTrans;
   solve(c, 0, na, alpha);
@@ -574,8 +571,8 @@ template void trsm<float>(hipStream_t, int, int, int, int, long, long, float, co
 
 // ---- the device array behind atlg_dtrsm_noalloc ---------------------------
 // kNoAllocMaxOrder / kTrsmNB inverses of 128 x 128 doubles (8 MiB), the
-// exchange area of the one-launch solves (24 MiB) and their failure word, one
-// copy per device, held until the process ends.  Its name is only a host-side
+// exchange area of the one-launch solves (24 MiB) and their failure words, one
+// copy per device, zero at first, held until the process ends.  Its name is only a host-side
 // stand-in for the symbol: host code uses the address that
 // hipGetSymbolAddress returns for the current device, never the name itself.
 static __device__ __align__(256) unsigned char scratch[atlg::kNoAllocBytes];
@@ -585,7 +582,7 @@ namespace {
 constexpr int kMaxDevices = 64;
 std::mutex g_noalloc_mu;
 void* g_noalloc_ptr[kMaxDevices] = {};
-std::atomic<bool> g_noalloc_used[kMaxDevices];
+std::map<hipStream_t, int> g_noalloc_words[kMaxDevices];  // stream -> its word's index
 }  // namespace
 
 // Address of the array on the current device, resolved once per device
@@ -603,17 +600,25 @@ void* noalloc_scratch() {
   return g_noalloc_ptr[dev];
 }
 
-void noalloc_used() {
+int* noalloc_word(hipStream_t s, bool make) {
   int dev = 0;
   ATLG_HIP(hipGetDevice(&dev));
-  g_noalloc_used[dev].store(true);  // (noalloc_scratch() has checked the index)
-}
-
-int* noalloc_status() {
-  int dev = 0;
-  ATLG_HIP(hipGetDevice(&dev));
-  if (dev < 0 || dev >= kMaxDevices || !g_noalloc_used[dev].load()) return nullptr;
-  return reinterpret_cast<int*>(static_cast<unsigned char*>(noalloc_scratch()) + kNoAllocBytes - 256);
+  if (dev < 0 || dev >= kMaxDevices) return nullptr;  // (noalloc_scratch() refuses the solve)
+  int index = 0;
+  {
+    std::lock_guard<std::mutex> lk(g_noalloc_mu);
+    auto& words = g_noalloc_words[dev];
+    const auto it = words.find(s);
+    if (it != words.end()) {
+      index = it->second;
+    } else {
+      if (!make) return nullptr;
+      index = (int)std::min(words.size(), kNoAllocWords - 1);
+      words[s] = index;
+    }
+  }
+  unsigned char* end = static_cast<unsigned char*>(noalloc_scratch()) + kNoAllocBytes;
+  return reinterpret_cast<int*>(end) - kNoAllocWords + index;
 }
 
 }  // namespace atlg

@@ -266,13 +266,13 @@ constexpr size_t kTxFixedBytes = 256 + sizeof(tx_word) * kTxBlock * kNoAllocTxBl
 static_assert(kNoAllocTxBlocks >= 384 / kTxCols * (2048 / kTxB) &&
               kNoAllocTxBlocks >= 3072 / kTxCols * (1024 / kTxB) &&
               kNoAllocTxBlocks >= 4096 / kTxCols * (512 / kTxB), "fixed exchange area");
-static_assert(kTxFixedBytes + 256 == kNoAllocTxBytes, "fixed exchange area");
+static_assert(kTxFixedBytes + 4 * kNoAllocWords == kNoAllocTxBytes, "fixed exchange area");
 
 // Solves op(A) X = alpha B, op(A) lower (or upper) triangular of order n <=
 // tx_order(nrhs), element (i, j) of X and B at i bi + j bj; Dinv holds the inverses
 // of op(A)'s NB x NB diagonal blocks, or their transposes (dtrans).  `fixed`,
-// when not null, is memory for the exchange area (kTxFixedBytes), with a
-// failure word behind it, in place of the stream's own.  False, with nothing queued,
+// when not null, is memory for the exchange area (kTxFixedBytes) in place of
+// the stream's own.  False, with nothing queued,
 // where the exchange area cannot be had.
 template <class S>
 bool trsv_one_launch(hipStream_t s, bool lower, bool tr, long n, long nrhs, S alpha, const S* A,
@@ -293,9 +293,7 @@ bool trsv_one_launch(hipStream_t s, bool lower, bool tr, long n, long nrhs, S al
   const int gpad = (groups + kTxGroups - 1) / kTxGroups * kTxGroups;
   const dim3 grid(gpad * (nb - 1) + groups), block(kTxThreads);
   const int up = lower ? 0 : 1;
-  int* status = fixed        ? reinterpret_cast<int*>(fixed + kTxFixedBytes)
-                : rep.status ? rep.status
-                             : status_word(s);
+  int* status = rep.status ? rep.status : status_word(s);
   const long limit = wait_limit(kSvSpin);
   // more groups than XCDs: throughput counts, and folding adds to the products
   const bool fold = groups <= kTxGroups;

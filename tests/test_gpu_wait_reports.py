@@ -77,3 +77,37 @@ def test_getrf_failed_solve_reported(G):
     G.dgetrf(n, n, da, n, ipiv, info, check=True)
     assert int(info.item()) == 0
     assert O.lu_resid(n, n, a0, G.to_fortran(da), ipiv.cpu().numpy()) <= 100
+
+
+def test_noalloc_failure_stays_with_its_stream(G):
+    import torch
+    n, k = 1500, 40
+    rng = np.random.default_rng(4)
+    a = G.from_fortran(np.asfortranarray(np.tril(rng.uniform(-1, 1, (n, n))) / n + 2 * np.eye(n)))
+    b = G.from_fortran(np.asfortranarray(rng.uniform(-1, 1, (n, k))))
+    s = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+
+    def solve(stream):
+        with torch.cuda.stream(stream):
+            x = b.clone()
+            G.dtrsm_noalloc(G.Left, G.Lower, G.NoTrans, G.NonUnit, n, k, 1.0, a, n, x, n)
+        torch.cuda.synchronize()  # (such solves on different streams may not overlap)
+        return x
+
+    def status(stream):
+        with torch.cuda.stream(stream):
+            return G.stream_status()
+
+    want = solve(s[1])
+    G.set_wait_limit(1)
+    try:
+        solve(s[0])
+    finally:
+        G.set_wait_limit(0)
+    assert status(s[1]) == 0  # a stream with such solves of its own
+    assert status(s[2]) == 0  # and one without
+    assert torch.equal(solve(s[1]), want) and status(s[1]) == 0
+    assert status(s[0]) == G.FAIL_TRSV
+    assert status(s[0]) == 0
+    assert torch.equal(solve(s[0]), want) and status(s[0]) == 0
