@@ -177,7 +177,19 @@ potf2_inv_kernel(int n, double* __restrict__ A, long lda, int lower, int* __rest
             for (int i = c; i < 4; i++) a[i][c] -= a[i][j] * a[c][j];
         }
         bad = __builtin_amdgcn_readfirstlane(bad);
-        if (bad >= 0) break;
+        if (bad >= 0) {  // the block's columns before it are part of the leading factor
+          if (lane == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+              for (int c = 0; c < i; c++)
+                if (4 * b + c < bad) S[(c0 + 4 * b + i) * PLD + c0 + 4 * b + c] = a[i][c];
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+              if (4 * b + c < bad) S[(c0 + 4 * b + c) * PLD + c0 + 4 * b + c] = a[c][c];
+          }
+          break;
+        }
         // inv(L11): every lane solves for the column lk, and keeps row ln of it
         double wc[4];
 #pragma unroll
@@ -258,13 +270,13 @@ potf2_inv_kernel(int n, double* __restrict__ A, long lda, int lower, int* __rest
     lds_barrier();
     const int fail = fail_sh;
     if (fail >= 0) {
-      // as ATLAS leaves a failing block: columns left of the failing one
-      // done (as far as they got), the rest as it was
+      // the factor of the leading minor (all rows and columns before the
+      // failing one) is complete in memory; of the rows from there on, this
+      // tile's earlier columns as far as they got, the rest as it was
       if (w == 0) {
-        const int bf = 4 * ((fail - c0) >> 2);
 #pragma unroll
         for (int b = 0; b < 4; b++)
-          if (4 * b < bf) store(c0 + ln, c0 + 4 * b + lk, row_d[c0 + 4 * b]);
+          if (c0 + 4 * b + lk < fail) store(c0 + ln, c0 + 4 * b + lk, row_d[c0 + 4 * b]);
         if (t == 0) *dinfo = info_off + fail + 1;
       }
       return;

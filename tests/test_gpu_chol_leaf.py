@@ -78,3 +78,17 @@ def test_leaf_failing_minor(G, uplo, n, bad, value):
     f, info = potrf(G, uplo, s)
     assert info == bad + 1
     assert np.array_equal(f[other(uplo, n)], s[other(uplo, n)])
+
+
+@pytest.mark.parametrize("uplo", UPLO)
+@pytest.mark.parametrize("n, q", [(5, 1), (20, 2), (20, 7), (64, 17), (64, 63), (128, 98),
+                                  (150, 131), (400, 390), (2304, 1301)])
+def test_leading_factor_of_a_failing_matrix(G, uplo, n, q):
+    # the leading minor of order info - 1 has its factor in place
+    s = O.lltgen(uplo, n, n * 7 + q)
+    s[q, q] = -1.0
+    f, info = potrf(G, uplo, s)
+    assert info == q + 1
+    lead = np.asfortranarray(s[:q, :q])
+    assert O.llt_resid(uplo, q, lead, np.asfortranarray(f[:q, :q])) <= 16
+    assert np.array_equal(f[other(uplo, n)], s[other(uplo, n)])
