@@ -399,12 +399,6 @@ constexpr long kCholLaMin = 2048;
 #ifndef ATLG_CHOL_STEP
 #define ATLG_CHOL_STEP 0
 #endif
-// Widest block (columns) whose look-ahead update goes in two parts, the
-// diagonal block's triangle and then the rest of the block column: the leaf
-// starts after the first part (N=4096 2.26 -> 2.18 ms, 8192 the same).
-#ifndef ATLG_CHOL_SPLIT_MAX
-#define ATLG_CHOL_SPLIT_MAX 512
-#endif
 inline long chol_step(long rem) {
   if (ATLG_CHOL_STEP > 0) return ATLG_CHOL_STEP;
   return rem < 4608 ? 256 : (rem < 12288 ? 384 : 512);
@@ -494,10 +488,6 @@ void potrf_lookahead(hipStream_t s0, bool lower, long N, double* A, long lda, in
       gemm(s, kTrans, kNoTrans, nc, r, kb, -1.0, at(k, c0), lda, at(k, c0 + nc), lda, 1.0,
            at(c0, c0 + nc), lda, 0, dinfo);
   };
-  // the stored triangle of diagonal block c0 (nc wide) likewise
-  auto update_diag = [&](hipStream_t s, long k, long kb, long c0, long nc) {
-    update(s, k, kb, c0, nc, nc, 0);
-  };
   hipEvent_t e_col = aux_event(4);
   auto width = [&](long k) { return std::min(chol_step(N - k), N - k); };
   const long kb0 = width(0);
@@ -507,19 +497,13 @@ void potrf_lookahead(hipStream_t s0, bool lower, long N, double* A, long lda, in
     const long kb = width(k0), k1 = k0 + kb, nb1 = width(k1);
     const long rest = N - k1 - nb1;
     // block k+1 first, then the rest of step k's update, beside which the
-    // auxiliary stream factors block k+1 and solves its panel; for narrow
-    // blocks its diagonal block alone goes first (all the leaf needs), then
-    // the rest of its block column (what the panel solve needs)
-    const bool diag_first = nb1 <= ATLG_CHOL_SPLIT_MAX;
-    if (diag_first) {
-      update_diag(s0, k0, kb, k1, nb1);
-      ATLG_HIP(hipEventRecord(e_upd, s0));
-      update_col(s0, k0, kb, k1, nb1, rest);
-      ATLG_HIP(hipEventRecord(e_col, s0));
-    } else {
-      update(s0, k0, kb, k1, N - k1, nb1, 0);
-      ATLG_HIP(hipEventRecord(e_upd, s0));
-    }
+    // auxiliary stream factors block k+1 and solves its panel: its diagonal
+    // block alone (all the leaf needs; N=4096 2.26 -> 2.18 ms, 8192 the same),
+    // then the rest of its block column (what the panel solve needs)
+    update(s0, k0, kb, k1, nb1, nb1, 0);
+    ATLG_HIP(hipEventRecord(e_upd, s0));
+    update_col(s0, k0, kb, k1, nb1, rest);
+    ATLG_HIP(hipEventRecord(e_col, s0));
     update(s0, k0, kb, k1 + nb1, rest, rest, split ? 0 : ATLG_CHOL_CAP);
     ATLG_HIP(hipStreamWaitEvent(s1, e_upd, 0));
     potrf_rec(s1, lower, nb1, at(k1, k1), lda, dinfo, (int)k1, W, status);
@@ -528,7 +512,7 @@ void potrf_lookahead(hipStream_t s0, bool lower, long N, double* A, long lda, in
     // side once that update is the shorter path (its units would wait).
     const bool solve_wide = split && chol_solve_wide(rest, nb1);
     if (!solve_wide) {
-      if (diag_first) ATLG_HIP(hipStreamWaitEvent(s1, e_col, 0));
+      ATLG_HIP(hipStreamWaitEvent(s1, e_col, 0));
       solve_panel(s1, k1, nb1, rest);
     }
     ATLG_HIP(hipEventRecord(e_panel, s1));
