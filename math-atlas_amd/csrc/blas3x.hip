@@ -290,14 +290,6 @@ sym_grad_kernel(int n, int k, double wa, const double* __restrict__ A, long lda,
   }
 }
 
-double* tri_copy_in(hipStream_t s, bool lower, bool unit, long n, const double* A, long lda,
-                    const int* skip) {
-  const long np = tri_full_order(n);
-  double* X = static_cast<double*>(scratch(s, kSlotTriFull, sizeof(double) * np * np));
-  tri_copy_to(s, lower, unit, n, A, lda, X, skip);
-  return X;
-}
-
 // A's triangle <- X^T X (lower: L^T L; upper, X = U^T: U U^T), one product
 // masked to the triangle, each tile's K range starting at its row and column.
 void lauum_from_full(hipStream_t s, bool lower, long n, const double* X, long np, double* A,
@@ -394,9 +386,28 @@ void trtri_rec(hipStream_t s, bool lower, int diag, long off, long N, double* A0
 
 long tri_full_order(long n) { return (n + kCT - 1) / kCT * kCT; }
 
-static bool tri_full_fits(long n, long least) {
-  const long np = tri_full_order(n);
-  return n >= least && (size_t)np * np * sizeof(double) <= kTriFullCap;
+// Elements of tri_invert_full's products.
+static long tri_temp_size(long n) {
+  long t = 0;
+  for (long sz = 2 * NB; sz / 2 < n; sz *= 2)
+    t = std::max(t, std::max(n / sz, 1L) * (sz / 2) * (sz / 2));
+  return t;
+}
+
+// Space for the dense copy of a triangle of order n, or nullptr where the
+// recursions take it: below order `least`, above kTriFullCap, and where the
+// workspace (with that of tri_invert_full when `invert`) would have to be
+// allocated under capture, which they need less of.
+static double* tri_full(hipStream_t s, long n, long least, bool invert) {
+  const size_t np = tri_full_order(n), nblk = (n + NB - 1) / NB;
+  if (n < least || np * np * sizeof(double) > kTriFullCap) return nullptr;
+  const size_t temp = sizeof(double) * tri_temp_size(n);
+  if (invert &&
+      (!scratch_in_capture(s, kSlotTrsmInv, sizeof(double) * nblk * NB * NB, false) ||
+       (temp > 0 && !scratch_in_capture(s, kSlotTriTemp, temp, false))))
+    return nullptr;
+  return static_cast<double*>(
+      scratch_in_capture(s, kSlotTriFull, sizeof(double) * np * np, false));
 }
 
 void tri_copy_to(hipStream_t s, bool lower, bool unit, long n, const double* A, long lda,
@@ -421,8 +432,7 @@ void tri_invert_full(hipStream_t s, int diag, long n, double* X, long np, const 
   hipLaunchKernelGGL(put_tri_blocks_kernel, dim3((unsigned)nblk), dim3(256), 0, s, (int)n, X, np,
                      1, 0, D, skip);
   ATLG_LAUNCHED();
-  long tneed = 0;
-  for (long sz = 2 * NB; sz / 2 < n; sz *= 2) tneed = std::max(tneed, std::max(n / sz, 1L) * (sz / 2) * (sz / 2));
+  const long tneed = tri_temp_size(n);
   if (tneed == 0) return;
   double* T = static_cast<double*>(scratch(s, kSlotTriTemp, sizeof(double) * tneed));
   for (long sz = 2 * NB; sz / 2 < n; sz *= 2) {
@@ -522,9 +532,9 @@ void trtri(hipStream_t s, int uplo, int diag, long N, double* A, long lda, int* 
     hipLaunchKernelGGL(diag_zero_kernel, dim3(1), dim3(256), 0, s, (int)N, A, lda, dinfo);
     ATLG_LAUNCHED();
   }
-  if (tri_full_fits(N, kTriFullMin)) {
+  if (double* X = tri_full(s, N, kTriFullMin, true)) {
     const long np = tri_full_order(N);
-    double* X = tri_copy_in(s, lower, diag == kUnit, N, A, lda, dinfo);
+    tri_copy_to(s, lower, diag == kUnit, N, A, lda, X, dinfo);
     tri_invert_full(s, diag, N, X, np, dinfo);
     const long tiles = np / kCT;
     hipLaunchKernelGGL(tri_copy_out_kernel, dim3((unsigned)(tiles * tiles)), dim3(256), 0, s,
@@ -544,8 +554,8 @@ void trtri(hipStream_t s, int uplo, int diag, long N, double* A, long lda, int* 
 void lauum(hipStream_t s, int uplo, long N, double* A, long lda, const int* skip) {
   if (N <= 0) return;
   const bool lower = uplo == kLower;
-  if (tri_full_fits(N, kLauumFullMin)) {
-    const double* X = tri_copy_in(s, lower, false, N, A, lda, skip);
+  if (double* X = tri_full(s, N, kLauumFullMin, false)) {
+    tri_copy_to(s, lower, false, N, A, lda, X, skip);
     lauum_from_full(s, lower, N, X, tri_full_order(N), A, lda, skip);
     return;
   }
@@ -557,14 +567,14 @@ void lauum(hipStream_t s, int uplo, long N, double* A, long lda, const int* skip
 // factor is F, the result's triangle goes to A (F itself, or another matrix).
 static void potri_from(hipStream_t s, int uplo, long N, const double* F, long ldf, double* A,
                        long lda, int* dinfo) {
-  if (N > 0 && tri_full_fits(N, kLauumFullMin)) {
+  if (double* X = tri_full(s, N, kLauumFullMin, true)) {
     // the inverse stays in the dense copy, from which the product reads
     const bool lower = uplo == kLower;
     set_int(s, dinfo, 0);
     hipLaunchKernelGGL(diag_zero_kernel, dim3(1), dim3(256), 0, s, (int)N, F, ldf, dinfo);
     ATLG_LAUNCHED();
     const long np = tri_full_order(N);
-    double* X = tri_copy_in(s, lower, false, N, F, ldf, dinfo);
+    tri_copy_to(s, lower, false, N, F, ldf, X, dinfo);
     tri_invert_full(s, kNonUnit, N, X, np, dinfo);
     lauum_from_full(s, lower, N, X, np, A, lda, dinfo);
     return;

@@ -113,3 +113,48 @@ def test_loglik_grad(G, n, k, same):
     want = -0.85 * (aa - k * (ti.T @ ti))
     scale = norm(t) * norm(t.T) * norm(ti) ** 2 * norm(ti.T) ** 2
     assert norm(got - want) <= 4 * max(n, k, 1) * EPS * (norm(x[:n, :k]) * norm(x[:n, :k].T) + k * scale)
+
+
+@pytest.mark.parametrize("routine, n", [("dlauum", 48), ("dlauum", 100), ("dtrtri", 200),
+                                        ("dpotri", 100), ("dpotri", 128)])
+def test_captured_without_workspace(G, routine, n):
+    # a stream that has only seen a triangular solve holds no space for the
+    # dense copy: a captured call does without it, an eager one may make it
+    import torch
+    rng = np.random.default_rng(n)
+    t = np.asfortranarray(np.tril(rng.uniform(-1, 1, (n, n))) / n + 2 * np.eye(n))
+    inv = np.linalg.inv(t)
+    want = {"dlauum": t.T @ t, "dtrtri": inv, "dpotri": inv.T @ inv}[routine]
+    low = np.tril_indices(n)
+    # each entry: sums of at most n products in each of the (at most two)
+    # products and the inversion, entries of |L^-1||L||L^-1| of order one
+    tol = 8 * n * np.finfo(float).eps * np.abs(want).max()
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        a0 = G.from_fortran(t)
+        a = a0.clone()
+        info = torch.zeros(1, dtype=torch.int32, device="cuda")
+        G.dtrsm(G.Left, G.Lower, G.NoTrans, G.NonUnit, n, n, 1.0, a0, n, a.clone(), n)
+
+        def call():
+            a.copy_(a0)
+            if routine == "dlauum":
+                G.dlauum(G.Lower, n, a, n)
+            elif routine == "dtrtri":
+                G.dtrtri(G.Lower, G.NonUnit, n, a, n, info)
+            else:
+                G.dpotri(G.Lower, n, a, n, info)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        call()
+    for _ in range(3):
+        a.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert int(info.item()) == 0
+        assert np.abs(G.to_fortran(a)[low] - want[low]).max() <= tol
+        with torch.cuda.stream(s):
+            call()
+        torch.cuda.synchronize()
+        assert np.abs(G.to_fortran(a)[low] - want[low]).max() <= tol
