@@ -24,7 +24,8 @@
  * Streams: `stream` is a hipStream_t passed as void*; NULL is HIP's null
  * (default) stream, as in other HIP libraries.  Workspace is owned by the
  * library per stream and reused across calls; calls on different streams
- * may run concurrently.  The host-pointer entry points use a stream of the
+ * may run concurrently.  A captured getrf or potrf of order >= 2048 is refused
+ * (ATLG_EHIP).  The host-pointer entry points use a stream of the
  * library's own.
  */
 #ifndef ATLAS_GPU_H

@@ -75,6 +75,11 @@ bool split_streams(int cus, hipStream_t caller, hipStream_t* small, hipStream_t*
 // Compute units that work queued on the stream runs on: a split_streams()
 // stream's share, else the device's.
 int stream_units(hipStream_t s);
+// Throws where the stream is being captured: the look-aheads' two streams wait
+// for each other in both directions, and the runtime, which ends a capture by
+// going from stream to stream along such waits, never gets to its end there (a
+// segmentation fault).
+void refuse_capture(hipStream_t s, const char* rout);
 // Held by a look-ahead driver while it queues work on the shared auxiliary
 // streams and events above, so that calls from several host threads do not
 // interleave their event records and waits (the device work of successive

@@ -1963,13 +1963,15 @@ void getrf_lookahead(LU<S>& f0) {
 
 template <class S>
 void getrf(hipStream_t s, long M, long N, S* A, long lda, int* ipiv, int* dinfo, int gemm_prec) {
+  const bool lookahead = ATLG_LU_LOOKAHEAD && std::min(M, N) >= kLaMin;
+  if (lookahead) refuse_capture(s, "getrf");
   set_int(s, dinfo, 0);
   if (M == 0 || N == 0) return;
   LU<S> f;
   init_lu(f, s, M, N, A, lda, ipiv, dinfo, gemm_prec);
   f.status = status_word(s);
   f.limit = wait_limit(kSpinLimit);
-  if (ATLG_LU_LOOKAHEAD && std::min(M, N) >= kLaMin)
+  if (lookahead)
     getrf_lookahead(f);
   else
     getrf_rec(f, 0, N);

@@ -528,12 +528,14 @@ void potrf_lookahead(hipStream_t s0, bool lower, long N, double* A, long lda, in
 }  // namespace
 
 void potrf(hipStream_t s, int uplo, long N, double* A, long lda, int* dinfo) {
+  const bool lookahead = ATLG_CHOL_LOOKAHEAD && N >= kCholLaMin;
+  if (lookahead) refuse_capture(s, "potrf");
   set_int(s, dinfo, 0);
   if (N <= 0) return;
   const long nblk = (N + DB - 1) / DB;
   double* W = static_cast<double*>(scratch(s, kSlotFactInv, sizeof(double) * nblk * DB * DB));
   int* status = status_word(s);
-  if (ATLG_CHOL_LOOKAHEAD && N >= kCholLaMin)
+  if (lookahead)
     potrf_lookahead(s, uplo == kLower, N, A, lda, dinfo, W, status);
   else
     potrf_rec(s, uplo == kLower, N, A, lda, dinfo, 0, W, status);

@@ -270,6 +270,13 @@ bool split_streams(int cus, hipStream_t caller, hipStream_t* small, hipStream_t*
   return give_pair(sp.pairs[pick], capturing, small, large);
 }
 
+void refuse_capture(hipStream_t s, const char* rout) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+  else if (cap != hipStreamCaptureStatusNone)
+    throw HipFailure{std::string(rout) + ": orders from 2048 on cannot be captured"};
+}
+
 int stream_units(hipStream_t s) {
   constexpr int kDevices = 64;
   static std::atomic<int> total[kDevices];  // by device, 0: not asked yet
