@@ -1513,7 +1513,8 @@ void launch_xcd(LU<S>& f, int M, int w, int off, int G, int* lst) {
   if (G > 1) f.box_par ^= 1;
   const int xcd = G > 1 ? f.xcd : 0;
   const dim3 grid(8 * (G - 1) + xcd + 1), block(64 * ((per + 63) / 64));
-  hipLaunchKernelGGL(panel_xcd<S>, grid, block, 0, f.s, M, w, off, at(f, off, off), f.lda, f.ipiv,
+  const auto fn = G == 1 ? panel_xcd<S, true> : panel_xcd<S, false>;
+  hipLaunchKernelGGL(fn, grid, block, 0, f.s, M, w, off, at(f, off, off), f.lda, f.ipiv,
                      f.dinfo, f.box, par, G, xcd, lst, f.status, f.limit, f.gather);
   ATLG_LAUNCHED();
 }

@@ -278,21 +278,24 @@ __device__ __attribute__((noinline)) void xp_alone(int M, int w, int off, S* P, 
 // on the matrix's diagonal; 32 columns of P span less than 2 GiB.  Outputs
 // as panel_coop's.  G workgroups of blockDim.x / 64 waves on XCD `xcd`; grid
 // 8 (G - 1) + xcd + 1 (see above).
-template <class S>
+// ONE: G is 1, and what several workgroups need is not compiled in (M = 256
+// 59 us, 65 in the general form; N = 1500 4.24 ms, 4.31).
+template <class S, bool ONE>
 __global__ void __launch_bounds__(64 * kXpWaves)
 panel_xcd(int M, int w, int off, S* __restrict__ P, long lda, int* __restrict__ ipiv,
-          int* __restrict__ dinfo, XpBox* __restrict__ box, int par, int G, int xcd,
+          int* __restrict__ dinfo, XpBox* __restrict__ box, int par, int groups, int xcd,
           int* __restrict__ list, int* __restrict__ status, long limit, long gather) {
   typedef TriMfma<S> Mf;
   typedef typename Mf::acc_t acc_t;
-  if ((blockIdx.x & 7) != xcd) return;
+  const int G = ONE ? 1 : groups;
+  if (!ONE && (blockIdx.x & 7) != xcd) return;
   __shared__ xp_word slot[2][kXpCand][16];  // the waves' candidates, word-major
   __shared__ S ubuf[4][kXpW];  // G == 1: trailing entries of the block's pivot rows
   __shared__ S l11[kXpWaves][4][4];  // each wave's copy of the block's pivot rows
   __shared__ int pa[kXpW], pb[kXpW];
   __shared__ int sbad, zcol, together;
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int NW = blockDim.x >> 6, g = blockIdx.x >> 3;
+  const int NW = blockDim.x >> 6, g = ONE ? 0 : blockIdx.x >> 3;
   const int n = lane & 15, k = lane >> 4;
   XpBox* mb = box + par;
   if (G > 1 && t == 0)
