@@ -39,13 +39,15 @@
 //    do not come all give up at once, and the first factors the panel alone,
 //    in memory (xp_alone, 1.4 ms for 8192 rows).  The panel is unchanged until
 //    the end, so nothing is lost, and no launch needs to be cooperative (N=1500
-//    4.9 ms with that, 4.3 without; counting in costs a leaf 2 of its 80 us).  Successive
-//    factorizations take the XCDs in turn, to keep out of each other's way.
+//    4.9 ms with that, 4.3 without; counting in costs a leaf 2 of its 80 us).
+//    Successive factorizations take the XCDs in turn, to keep out of each
+//    other's way.
 //
 // A column takes 4000-4500 cycles (about 1.8 us), most of it the issue of
 // some 450 dependent instructions by one or two waves per SIMD.  M x 32 LU,
-// set-up launches included (panel_coop -> here): M = 256 136 -> 74 us, 1000
-// 168 -> 88, 4096 178 -> 88, 8192 186 -> 96.  128 rows per wave (half the
+// set-up launches included (panel_coop -> here, by one measurement): M = 256
+// 136 -> 74 us, 1000 168 -> 88, 4096 178 -> 88, 8192 186 -> 96; without the
+// copies in it 59, 78, 80 and 94 us.  128 rows per wave (half the
 // workgroups) did not fit the registers: 160 us at M = 1000.
 #pragma once
 

@@ -371,7 +371,7 @@ void potrf_rec(hipStream_t s, bool lower, long N, double* A, long lda, int* dinf
 // Look-ahead (1) or plain right-looking steps (0).  At N = 16384 the
 // look-ahead with the panels on 32 compute units and the SYRKs on the rest
 // takes 55 ms against 65 ms for plain steps; on a shared device (no masked
-// streams) both took 65 ms: the 128-block leaves, which need 132 KB of LDS,
+// streams) both took 65 ms: the 128-block leaves, which need 156 KB of LDS,
 // wait for a compute unit free of SYRK workgroups.
 // Without masked streams: grid cap of the look-ahead's trailing SYRK
 // (workgroups).
@@ -438,7 +438,7 @@ void potrf_lookahead(hipStream_t s0, bool lower, long N, double* A, long lda, in
   const auto lock = aux_lock();
   hipStream_t s1 = aux_stream();
   hipEvent_t e_upd = aux_event(0), e_panel = aux_event(1);
-  // with a CU-masked pair the 128-block leaves (132 KB of LDS) never wait
+  // with a CU-masked pair the 128-block leaves (156 KB of LDS) never wait
   // for a compute unit free of SYRK workgroups
   hipStream_t caller = s0, sp = nullptr, sg = nullptr;
   const bool split =

@@ -10,8 +10,11 @@
 // fetch the solved blocks: with both in one wave the in-order load counter
 // makes every poll wait for the next block of op(A) as well (order 2048,
 // transposed: 112 us against 88).  The block solved right before this one is
-// multiplied by -inv(A_pp) A_pq, formed ahead, so a step of the chain is one
-// exchange, two LDS passes and one product of 1024 cycles: 1.8 us measured.
+// multiplied by -inv(A_pp) A_pq, formed ahead, so that its product does not
+// wait for a pass through the inverse.  A step of the chain is one exchange,
+// two LDS passes and two products of 1024 cycles (inv(A_pp) times what the
+// earlier blocks left starts at the barrier that the last one's arrival opens):
+// 1.8 us measured.
 // 128-row blocks double the product and spill.  Orders 500 / 1000 / 2048
 // with 3 right-hand sides take 40 / 55 / 85 us (27 of each: the inverses),
 // by blocked launches 148 / 341 and, four right-hand sides at most, 141 us.
